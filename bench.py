@@ -99,7 +99,7 @@ def variant_rate(name: str, flux: int, precision: int, batch: int, steps: int, w
     """Mcell-iter/s of `batch` copies of the workload stepped together (one launch per kernel over
     all their blocks), in the given precision mode; inputs resident before the timed region.  With
     `plain`, one copy in the per-block launch mode instead: every kernel launched once per block,
-    eagerly (no graphs), the LU-SGS sweeps on 8x8 tiles (no autotuning)."""
+    eagerly (no graphs), the LU-SGS sweeps on 8x2 tiles (no autotuning)."""
     members = [A.solver_from_case(batch_member(name, flux, q), precision=precision) for q in range(batch)]
     cells = sum(ncells(batch_member(name, flux, 0)) for _ in range(batch))
     if batch == 1:
@@ -124,7 +124,7 @@ def variant_rate(name: str, flux: int, precision: int, batch: int, steps: int, w
         run.close()
     for m in members:
         m.close()
-    return dict(precision="fp64" if precision == 0 else "mixed", batch=batch, cells=cells, lu_tile=f"{tj}x{64 // tj}",
+    return dict(precision="fp64" if precision == 0 else "mixed", batch=batch, cells=cells, lu_tile=f"{tj}x{16 // tj}",
                 launches="per block, eager" if plain else "batched" + (", graphs" if graph else ""),
                 value=round(cells * steps / wall / 1e6, 3), ms_per_step=round(wall * 1e3 / steps, 4),
                 res_rms1_max=max(rms))
@@ -194,7 +194,7 @@ def cpu_baseline(case, what: str, iters: int):
 
 
 def _plain_solver(case):
-    """The plain GPU solver of one request: per-block eager launches, 8x8 LU-SGS tiles."""
+    """The plain GPU solver of one request: per-block eager launches, 8x2 LU-SGS tiles."""
     s = A.solver_from_case(case)
     s.set_per_block(True)
     return s
@@ -391,7 +391,7 @@ def main() -> int:
         s.set_lu_tile(args.lu_tile)
     elif args.lu == "pipelined" and args.autotune > 0:
         tj, tms = s.autotune_lu(args.autotune)          # ordinary iterations, untimed
-        tune = dict(kept=f"{tj}x{64 // tj}", ms_per_sweep_pair={f"{t}x{64 // t}": round(v, 4) for t, v in tms.items()})
+        tune = dict(kept=f"{tj}x{16 // tj}", ms_per_sweep_pair={f"{t}x{16 // t}": round(v, 4) for t, v in tms.items()})
         print(f"# LU tile autotune: {tune}", file=sys.stderr, flush=True)
     for _ in range(args.warmup):
         s.step(1)
@@ -457,7 +457,7 @@ def main() -> int:
             "flux": FLUX_NAMES[int(case.params["Iflag_Flux"])],
             "graph": bool(args.graph),
             "lu_schedule": args.lu,
-            "lu_tile": (tune["kept"] if tune else f"{s_tile}x{64 // s_tile}") if args.lu != "hyperplane" else None,
+            "lu_tile": (tune["kept"] if tune else f"{s_tile}x{16 // s_tile}") if args.lu != "hyperplane" else None,
             "precision": args.precision,
         },
         "lu_autotune": tune,

@@ -176,9 +176,9 @@ int ocfd_step_timed(ocfd_ctx *ctx, int32_t niter, double *stage_ms);
 int ocfd_set_graph(ocfd_ctx *ctx, int32_t enable);
 
 /* Schedule of the LU-SGS sweeps; all give the reference's DU bit for bit.
- *   OCFD_LU_PIPELINED        (default) one persistent launch per sweep: (j,k) tiles of 64
- *                            columns (8x8 unless set otherwise) march along i, three waves per
- *                            tile (one per neighbour direction); tile-edge DU exchanged through
+ *   OCFD_LU_PIPELINED        (default) one persistent launch per sweep: (j,k) tiles of 16
+ *                            columns (8x2 unless set otherwise) march along i, four waves per
+ *                            tile (one per neighbour direction, one that loads); tile-edge DU exchanged through
  *                            sentinel-marked, device-coherent stores and loads
  *   OCFD_LU_HYPERPLANE       one launch per i+j+k hyperplane, the reference's own order
  *                            (sub_LU_SGS.f90:20-126)
@@ -190,7 +190,7 @@ int ocfd_set_graph(ocfd_ctx *ctx, int32_t enable);
 #define OCFD_LU_PIPELINED_FENCED 2
 int ocfd_set_lu_schedule(ocfd_ctx *ctx, int32_t schedule);
 
-/* Tile shape of OCFD_LU_PIPELINED: tj x (64/tj) (j,k) columns per tile, tj = 4, 8 (default) or
+/* Tile shape of OCFD_LU_PIPELINED: tj x (16/tj) (j,k) columns per tile, tj = 4, 8 (default) or
  * 16.  Results do not depend on it (bit for bit); the sweep time does.  No counterpart in the
  * reference. */
 int ocfd_set_lu_tile(ocfd_ctx *ctx, int32_t tj);
@@ -204,7 +204,7 @@ int ocfd_set_lu_tile(ocfd_ctx *ctx, int32_t tj);
 int ocfd_set_lu_fail_waits(ocfd_ctx *ctx, int32_t on);
 
 /* Launch mode.  on = 1: every kernel of the iteration is launched once per block, eagerly (no
- * graphs), and the LU-SGS sweeps keep 8x8 tiles (the autotuner refuses); on = 0 (the default):
+ * graphs), and the LU-SGS sweeps keep 8x2 tiles (the autotuner refuses); on = 0 (the default):
  * one launch per kernel over all blocks, graphs per ocfd_set_graph, any tile shape.  The results
  * are the same bit for bit.  No counterpart in the reference (the per-block form is its block
  * loop, for comparison with the batched launches). */

@@ -185,11 +185,11 @@ struct LuTask {
     int blk, j0, k0, tj, tk;
     int dep_j, off_j, last_j;    // upstream tile along j: task index (-1: none), step offset, its last step
     int dep_k, off_k, last_k;    // upstream tile along k
-    long long pofs;              // sweep-ordered storage of this tile: element (step q, field f, lane) at
-                                 // pofs + (q NF + f) 64 + lane
+    long long pofs;              // sweep-ordered storage of this tile: the run of step q at pofs + q RUN
     long long pofs_j;            // the j-upstream tile's storage offset
     long long pofs_k;            // the k-upstream tile's storage offset
     int tj_up, tk_up;            // the upstream tiles' j and k extents
+    int start;                   // steps (and tile hops) between the sweep's start and the tile's
 };
 
 // device tables of the pipelined sweeps of one context
@@ -206,53 +206,49 @@ struct LuPlan {
     long long P = 0;
     const int2* win = nullptr;   // (forward tile, first i) of every i-window of PK_W cells of the tiles
     int nwins = 0;
-    int tj = 8;                  // tile width in j (tiles are tj x 64/tj (j,k) columns)
+    int tj = 8;                  // tile width in j (tiles are tj x 16/tj (j,k) columns)
 };
 
-// lanes of a pipelined LU-SGS tile (one 64-wide wave per tile and sweep direction)
-constexpr int LU_NT = 64;
+// A wave of the pipelined LU-SGS sweep holds LU_COLS (j,k) columns of a tile, LU_PARTS lanes (a DPP
+// quad) each: lane 4 c + m works on components m + 1 (momentum for m = 0, 1, 2, energy for m = 3)
+// and on one of (density, the turbulence variables) of column c.
+constexpr int LU_NT = 64, LU_PARTS = 4, LU_COLS = LU_NT / LU_PARTS;
 
-// The sweep-ordered storage.  For a tile, step q (the cells its lanes visit at forward step q; the
-// backward sweep visits them at step nsteps-1-q) holds NF fields of 64 consecutive doubles, one
-// per lane: element (q, f, lane) at pofs + (q NF + f) 64 + lane_pos(lane).  A step's inputs therefore sit in
-// one contiguous run that a lane addresses from one pointer with constant offsets.  AL holds the
-// LU-SGS diagonal: alfa of components 1..5 (and of 6, 7 for SST) and, for SA only, the SA
-// component's alfa of the forward (AL+1) and of the backward sweep (AL+2), which sum the viscous
-// radii in different orders.  The buffer
-// has LU_PAD_STEPS steps of padding at both ends, so loads a few steps past either end of a tile
-// (prefetches of steps that do not exist, at most the larger tile side + 2 steps before an
-// upstream tile's first step) stay inside it.
+// The sweep-ordered storage.  For a tile, step q (the cells its columns visit at forward step q; the
+// backward sweep visits them at step nsteps-1-q) is one contiguous run of RUN doubles at
+// pofs + q RUN, made of groups:
+//   R, DUF, DUB   Res and the two DU arrays, NV components: components 2..5 of a column side by side
+//                 (4 c + m), so a wave's 64 lanes take 512 consecutive bytes, then density and the
+//                 turbulence variables (64 + NB c + m)
+//   NBR           what a neighbour needs of a cell, CS doubles per column: U (components 2..5, then
+//                 density and the turbulence variables with limit_vt's clamp applied), the pressure
+//                 of U and the reciprocal of its density (recip_nr), Lc and Lv of the three directions
+//   SG            the three face areas, four doubles per column
+//   AL            the LU-SGS diagonal and its reciprocal, pairs, CA doubles per column: alfa of
+//                 components 1..5 (and of 6, 7 for SST) and, for SA only, the SA component's alfa of
+//                 the forward and of the backward sweep, which sum the viscous radii in different orders
+//   N             the face normals, three directions of three components per column
+// The forward sweep reads one contiguous piece of a run, R to N, the backward sweep NBR to DUF.  A
+// column's NBR chunk is a multiple of 16 bytes, and CS and CA spread the columns over the LDS banks.
+// The buffer has LU_PAD_STEPS steps of padding at both ends, so loads a few steps past either end
+// of a tile (prefetches of steps that do not exist) stay inside it.
 template <int NV> struct Pk {
-    static constexpr int U = 0, R = NV, DUF = 2 * NV, DUB = 3 * NV, LC = 4 * NV, LV = 4 * NV + 3, AL = 4 * NV + 6,
-                         S = 4 * NV + 9, N = 4 * NV + 12, NF = 4 * NV + 21;
+    static constexpr int NB = NV - 4, NAL = NV == 6 ? 3 : 1;
+    static constexpr int CS = NV == 7 ? 18 : 14, CA = 2 * NAL;
+    static constexpr int P = 4 + NB, RD = P + 1, LC = RD + 1, LV = LC + 3;        // in an NBR chunk
+    static constexpr int R = 0, NBR = NV * LU_COLS, SG = NBR + CS * LU_COLS, AL = SG + 4 * LU_COLS, N = AL + CA * LU_COLS,
+                         DUF = N + 9 * LU_COLS, DUB = DUF + NV * LU_COLS, RUN = DUB + NV * LU_COLS;
+    static constexpr int SWEEP = DUF - R;                                          // doubles of a run a sweep reads
+    static_assert(LV + 3 <= CS && CS % 2 == 0, "an NBR chunk holds its fields in 16-byte pieces");
+    // component (0..NV-1) and column of element w of a vector group, and the inverse
+    static __device__ __host__ __forceinline__ void vec_at(int w, int& v, int& c) {
+        if (w < 4 * LU_COLS) { c = w >> 2; v = (w & 3) + 1; }
+        else { const int r = w - 4 * LU_COLS, m = r % NB; c = r / NB; v = m == 0 ? 0 : m + 4; }
+    }
+    static __device__ __host__ __forceinline__ int vec_off(int v, int c) {
+        return v >= 1 && v <= 4 ? 4 * c + v - 1 : 4 * LU_COLS + NB * c + (v == 0 ? 0 : v - 4);
+    }
 };
-// Position of lane (jl, kl) = lane % TJ, lane / TJ of a TJ x (64/TJ) tile inside a step's run of 64
-// elements: first the tile's j-edge columns (jl = TJ-1, then jl = 0), then the rest of its k-edge
-// rows (kl = TK-1, then kl = 0), then the interior row by row.  The lanes a downstream tile reads
-// across an edge therefore share few 128-byte lines (8x8 tiles: one line per field for the
-// j-edge and two for the k-edge, against four and one in row order).
-template <int TJ>
-__device__ __host__ __forceinline__ int lane_pos(int lane) {
-    constexpr int TK = 64 / TJ;
-    const int jl = lane % TJ, kl = lane / TJ;
-    if (jl == TJ - 1) return kl;
-    if (jl == 0) return TK + kl;
-    if (kl == TK - 1) return 2 * TK + (jl - 1);
-    if (kl == 0) return 2 * TK + (TJ - 2) + (jl - 1);
-    return 2 * TK + 2 * (TJ - 2) + (kl - 1) * (TJ - 2) + (jl - 1);
-}
-// the lane at position pos of a step's run (the inverse of lane_pos)
-template <int TJ>
-__device__ __host__ __forceinline__ int pos_lane(int pos) {
-    constexpr int TK = 64 / TJ;
-    int jl, kl;
-    if (pos < TK) { jl = TJ - 1; kl = pos; }
-    else if (pos < 2 * TK) { jl = 0; kl = pos - TK; }
-    else if (pos < 2 * TK + (TJ - 2)) { kl = TK - 1; jl = pos - 2 * TK + 1; }
-    else if (pos < 2 * TK + 2 * (TJ - 2)) { kl = 0; jl = pos - 2 * TK - (TJ - 2) + 1; }
-    else { const int r = pos - 2 * TK - 2 * (TJ - 2); kl = r / (TJ - 2) + 1; jl = r % (TJ - 2) + 1; }
-    return jl + TJ * kl;
-}
 constexpr int LU_PAD_STEPS = 24;
 constexpr int PK_W = 32;      // i-window of one workgroup of the sweep-order transposes and cell pass
 

@@ -806,55 +806,41 @@ __global__ void __launch_bounds__(64) k_update_detect(BSet S) {
 
 // The update of an iteration with the pipelined sweeps: the backward sweep's DU comes from the
 // sweep-ordered storage.  A workgroup takes one sweep tile's cells of an i-window (the tiles and
-// windows of that storage), the lanes of UP_ROWS consecutive positions of a step's run per pass
-// (one 128-byte line of each step).  A pass reads its lanes' DU along the steps and parks it in
-// LDS; then its threads update the pass's cells, i fastest.  DU stays in the storage until the
-// next iteration's pack; the block arrays get it only when the host asks for it.  Lane (jl, kl)
-// holds cell i at step i - 1 + jl + kl.  After a sweep gave up, the update leaves U and the
-// storage as they are; the host puts the sentinel back into the whole storage.
-constexpr int UP_ROWS = 16, UP_T = UP_ROWS * PK_W;
+// windows of that storage): it reads their DU along the steps, parks it in LDS and then updates the
+// cells, i fastest.  DU stays in the storage until the next iteration's pack; the block arrays get
+// it only when the host asks for it.  Column (jl, kl) holds cell i at step i - 1 + jl + kl.  After
+// a sweep gave up, the update leaves U and the storage as they are; the host puts the sentinel
+// back into the whole storage.
+constexpr int UP_T = LU_COLS * PK_W;
 
 template <int NV, int TJ>
 __global__ void __launch_bounds__(UP_T) k_update_pk(BSet S, const LuTask* __restrict__ tiles, const double* __restrict__ pk,
                                                     const int2* __restrict__ wins) {
     using F = Pk<NV>;
-    constexpr int DMAX = TJ + LU_NT / TJ - 2;                 // largest jl + kl of a tile
-    constexpr int SLOTS = (PK_W + DMAX) * UP_ROWS;            // (step, position) slots a pass can touch
-    __shared__ double buf[NV][UP_ROWS][PK_W + 1];
+    constexpr int M = NV * LU_COLS;
+    __shared__ double buf[NV][LU_COLS][PK_W + 2];
     if (halted(S)) return;
     const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];     // (tile, i-window), windows fastest
     const LuTask T_ = tiles[wn.x];
     const Blk& b = S.blk[T_.blk];
     const Par& p = S.par[T_.blk];
-    const int nxm = b.nx - 1;
-    const int i0 = wn.y;
-    const int W = min(PK_W, nxm - i0 + 1);
-    const int t = (int)threadIdx.x, rr = t / PK_W, c = t % PK_W;
-#pragma unroll 1
-    for (int pos0 = 0; pos0 < LU_NT; pos0 += UP_ROWS) {
-        // step i0 - 1 + qo: the lane at position pos0 + l holds cell i0 + qo - (jl + kl) there
-        for (int slot = t; slot < SLOTS; slot += UP_T) {
-            const int l = slot % UP_ROWS, qo = slot / UP_ROWS;
-            const int lane = pos_lane<TJ>(pos0 + l);
-            const int jl = lane % TJ, kl = lane / TJ, ci = qo - (jl + kl);
-            if (jl < T_.tj && kl < T_.tk && ci >= 0 && ci < W) {
-                const double* el = pk + T_.pofs + ((long long)(i0 - 1 + qo) * F::NF + F::DUB) * LU_NT + pos0 + l;
+    const int i0 = wn.y, W = min(PK_W, b.nx - 1 - i0 + 1), t = (int)threadIdx.x;
+    const double* run = pk + T_.pofs + (long long)(i0 - 1) * F::RUN + F::DUB;
+    for (int e = t; e < (W + TJ + LU_COLS / TJ - 2) * M; e += UP_T) {
+        const int qo = e / M, w = e % M;
+        int v, c;
+        F::vec_at(w, v, c);
+        const int jl = c % TJ, kl = c / TJ, x = qo - jl - kl;
+        if (jl < T_.tj && kl < T_.tk && x >= 0 && x < W) buf[v][c][x] = run[(long long)qo * F::RUN + w];
+    }
+    __syncthreads();
+    const int c = t / PK_W, x = t % PK_W, jl = c % TJ, kl = c / TJ;
+    if (jl < T_.tj && kl < T_.tk && x < W) {
+        const int i = i0 + x, j = T_.j0 + jl, k = T_.k0 + kl;
+        double DU[MAXV];
 #pragma unroll
-                for (int m = 0; m < NV; m++) buf[m][l][ci] = el[m * LU_NT];
-            }
-        }
-        __syncthreads();
-        const int lane = pos_lane<TJ>(pos0 + rr);
-        const int jl = lane % TJ, kl = lane / TJ;
-        if (jl < T_.tj && kl < T_.tk && c < W) {
-            const int i = i0 + c, j = T_.j0 + jl, k = T_.k0 + kl;
-            const size_t s = IX(b, i, j, k);
-            double DU[MAXV];
-#pragma unroll
-            for (int m = 0; m < NV; m++) DU[m] = buf[m][rr][c];
-            update_cell(b, p, i, j, k, s, DU);
-        }
-        __syncthreads();
+        for (int m = 0; m < NV; m++) DU[m] = buf[m][c][x];
+        update_cell(b, p, i, j, k, IX(b, i, j, k), DU);
     }
 }
 

@@ -62,10 +62,13 @@ void launch_lusgs_sweep(const Blk& b, const Par& p, bool forward, hipStream_t st
 // comput_force over the set's wall faces: parts (ntiles x 9 doubles), then out9 (Ft(1:9))
 void launch_forces(const SetPlan& P, const double cen[3], double* part, double* out9, hipStream_t st);
 int check_division(long long n, unsigned long long seed, int emax, long long* mismatches);
-std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int nfields, int tj, long long* total_elements);
+// tiles of tj x tk columns; run: doubles of one step of a tile in the sweep-ordered storage
+std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int run, int tj, int tk, long long* total_elements);
+// a launch's tiles (of one or several solves) in the order in which they can start
+void lusgs_start_order(std::vector<LuTask>& tasks);
 bool lusgs_tile_ok(int tj);
-int lusgs_fields(int NV);
-// (forward tile, first i) of every i-window of the tiles, tile after tile
+int lusgs_run(int NV);
+// (forward tile, first i) of every i-window of the tiles, tile after tile in storage order
 std::vector<int2> lusgs_window_list(const std::vector<Blk>& blks, const std::vector<LuTask>& fwd);
 void launch_lusgs_pack_geometry(const LuPlan& L, const Par& p, hipStream_t st);
 // the sweeps' per-iteration inputs (U, Res, Lc, Lv, the diagonal) into sweep order

@@ -5,7 +5,7 @@
 // honours those three dependencies gives the reference's hyperplane result bit for bit, because
 // every cell evaluates the same expression in the same order once its neighbours are final.
 //
-// Schedule: the (j,k) cross-section of a block is cut into 8x8 tiles; one 64-lane wave owns a
+// Fenced schedule: the (j,k) cross-section of a block is cut into 8x8 tiles; one 64-lane wave owns a
 // tile and marches along i, lane (jl,kl) handling cell i = q - jl - kl + 1 at local step q (a
 // hyperplane inside the tile).  Within the tile the j/k neighbours come through LDS (the lane
 // that computed them one step earlier) and the i neighbour stays in registers.  Across tiles the
@@ -16,6 +16,7 @@
 // and every wait is also bounded by a poll limit that raises an error flag instead of hanging.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "ocfd_dev.h"
@@ -27,6 +28,7 @@ namespace ocfd {
 constexpr int LU_TJ = 8, LU_TK = 8;
 static_assert(LU_TJ * LU_TK == LU_NT, "the fenced sweep's tiles are 8 x 8");
 constexpr long LU_POLL_LIMIT = 1L << 26;
+constexpr int LU_HOP = 5;             // steps a tile trails its upstream tile by beyond that tile's width
 
 // err[0]: the error flag a wait sets when it gives up.  err[2]: nonzero makes every wait that
 // finds its producer behind give up at its first poll (the host's failure-path test).  The poll
@@ -204,15 +206,30 @@ __global__ void __launch_bounds__(LU_NT) k_lusgs_sweep(const Blk* __restrict__ b
 }
 
 // ---------------------------------------------------------------------------------------------
-// Team sweep: the same tiles and the same in-tile hyperplanes, three waves per tile.  Wave d
-// (d = 0, 1, 2 for i, j, k) owns the contribution of the upstream neighbour in direction d.  At
-// step q each wave first completes the DU of the cell it reads, the one its lane's neighbour
-// computed at step q - 1 (its own previous cell for d = 0, the lane across the j or k step for
-// d = 1, 2): DU = (((Res + du_i) + du_j) + du_k) / alfa in the reference's order (backward sweep:
+// Team sweep: the same in-tile hyperplanes on tiles of 16 (j,k) columns, four lanes (a DPP quad) per
+// column, three direction waves and a loader wave per tile.  Wave d (d = 0, 1, 2 for i, j, k) owns
+// the contribution of the upstream neighbour in direction d.  At step q each wave first completes
+// the DU of the cell it reads, the one its lane's neighbour computed at step q - 1 (its own previous
+// cell for d = 0, the column across the j or k step for d = 1, 2): DU = (((Res + du_i) + du_j) + du_k) / alfa in the reference's order (backward sweep:
 // DU + ((du_i + du_j) + du_k) / alfa) from the three waves' terms of step q - 1 in LDS.  It then
 // evaluates the neighbour term of its direction for its own cell and writes it to LDS.  One
 // workgroup barrier per step separates the terms of a step from their use in the next; the LDS
 // terms are double-buffered by step parity.  Wave 0 stores each completed DU of its own cell.
+//
+// What bounds it: a lone tile's step is one wave's instruction stream (every instruction of a wave
+// alone on its SIMD takes 4 to 5 clocks, dependent or not) plus the exchange (two LDS writes, the
+// barrier and six LDS reads, about 210 clocks).  Hence the split: a quad holds a column's components
+// (momentum and energy in the first slot, density and the turbulence variables in the second), so a
+// wave issues about 70 FP64 and 24 DPP instructions per step where a lane with all components issued
+// 170 FP64; the loader brings a step's inputs to the LDS by 16-byte loads (45 8-byte loads by the
+// direction waves cost more than the arithmetic: 0.69 us per step with them, 0.36 without); and the
+// pressure and the reciprocals that do not depend on DU are formed once per cell by the pack.  A
+// step takes 0.42 us against 1.05 to 1.35 us with 64 columns per wave and all components per lane:
+// forward sweep of the 257x97x33 C-grid (SA) 528 -> 262 us, of the 97x33x9 channel 137 -> 85, of the
+// 24-block wing with 6.3 M cells 1085 -> 746.  A tile trails its upstream tile by about 3 us beyond
+// its own width, so long chains of narrow tiles lose (16x1 tiles), and a launch starts its tiles in
+// the order in which they can run (lusgs_start_order): block after block, the wing's sweep took
+// 1560 us instead of 1120 with the same kernel, most resident tiles waiting.
 //
 // Cross-tile values travel through the sweep-ordered DU arrays themselves.  Before a sweep every
 // element of the array it writes holds a sentinel NaN (a payload no arithmetic produces); the
@@ -224,7 +241,6 @@ __global__ void __launch_bounds__(LU_NT) k_lusgs_sweep(const Blk* __restrict__ b
 // tile that is running or done; every wait is also bounded by a poll limit that raises the error
 // flag.
 
-constexpr int LT_NT = 3 * LU_NT;
 __device__ __forceinline__ void st_coherent(double* p, double v) {
     __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(v),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -235,98 +251,139 @@ __device__ __forceinline__ double ld_coherent(const double* p) {
 }
 
 
-// value of field f of the sweep-ordered storage at box index s (not for DUF/DUB, whose packing
-// puts the sentinel into them)
-template <int NV>
-__device__ __forceinline__ double pack_value(const Blk& b, int f, size_t s) {
-    using F = Pk<NV>;
-    if (f < F::R) return b.U[f][s];
-    if (f < F::DUF) return b.Res[f - F::R][s];
-    if (f < F::LV) return b.Lc[f - F::LC][s];
-    if (f < F::AL) return b.Lv[f - F::LV][s];
-    if (f < F::S) return b.al[f - F::AL][s];
-    if (f < F::N) return b.S[f - F::S][s];
-    return b.nv[f - F::N][s];
-}
-
 constexpr int PK_T = 256;
 
-// box -> sweep order for fields [f0,f1) and then from f2 on (one per grid z); one tile, one
-// i-window and one field per workgroup, through LDS so both sides move in contiguous runs.  Neighbouring i-windows of a tile
-// share the step rows at their boundary (each writes some lanes of them), so a tile's windows run
-// back to back on one XCD, where the L2 merges those partial lines before they go to memory.
-// A DU field's workgroup reads nothing and puts the sentinel into the elements of its window's
-// cells that a downstream tile may wait on, in whole lines: a line written in part costs a
-// read-modify-write of the memory beneath it (storing only the edge lanes of each step, before
-// they led the run, made the pack of the 60.8 M-cell swept wing 3.0 ms slower, against 1.4 ms
-// for whole steps; the U workgroups storing the sentinel beside each U, instead of workgroups of
-// their own, 1.7 ms).
+// what a workgroup of the pack takes along: the neighbour data, Res, the diagonal, the sentinel
+// into DUF and DUB, and (once per plan) the areas and normals
+enum PackGroup { PG_NBR = 0, PG_R, PG_AL, PG_SENT_F, PG_SENT_B, PG_S, PG_N, PG_END };
+
+// box -> sweep order for one tile, one i-window of PK_W cells and one group of fields, through LDS
+// so both sides move in contiguous runs: NS fields are read (value src(v, s) at box index s), fin
+// completes a cell's column of the buffer, and the N fields are written: element w (of N LU_COLS)
+// of a step, field v of column c after at(w, v, c), goes to the run's element base + pos(w, v, c).  The LDS pitch of
+// PK_W + 2 keeps the skewed reads of a step's elements on different banks.
+template <int NV, int TJ, int NS, int N, typename Src, typename Fin, typename At, typename Pos>
+__device__ __forceinline__ void pack_group(double (*buf)[LU_COLS][PK_W + 2], const LuTask& T, const Blk& b, double* pk, int i0, int W,
+                                           int base, Src&& src, Fin&& fin, At&& at, Pos&& pos) {
+    constexpr int TK = LU_COLS / TJ;
+    const int t = (int)threadIdx.x, nsteps = b.nx - 1 + T.tj + T.tk - 2;
+    for (int e = t; e < NS * LU_COLS * PK_W; e += PK_T) {
+        const int x = e % PK_W, c = (e / PK_W) % LU_COLS, v = e / (PK_W * LU_COLS), jl = c % TJ, kl = c / TJ;
+        if (jl < T.tj && kl < T.tk && x < W) buf[v][c][x] = src(v, IX(b, i0 + x, T.j0 + jl, T.k0 + kl));
+    }
+    __syncthreads();
+    if constexpr (NS < N) {
+        for (int e = t; e < LU_COLS * PK_W; e += PK_T) fin(e / PK_W, e % PK_W);
+        __syncthreads();
+    }
+    for (int e = t; e < (W + TJ + TK - 2) * (N * LU_COLS); e += PK_T) {
+        const int q = i0 - 1 + e / (N * LU_COLS), w = e % (N * LU_COLS);
+        int v, c;
+        at(w, v, c);
+        const int jl = c % TJ, kl = c / TJ, x = q - jl - kl + 1 - i0;
+        if (jl < T.tj && kl < T.tk && x >= 0 && x < W && q < nsteps) pk[(size_t)T.pofs + (size_t)q * Pk<NV>::RUN + base + pos(w, v, c)] = buf[v][c][x];
+    }
+}
+
+// The pack of one group (grid z, from group g0 on).  Neighbouring i-windows of a tile share the
+// step runs at their boundary (each writes some columns of them), so a tile's windows run back to
+// back on one XCD, where the L2 merges those partial lines before they go to memory.  A DU group's
+// workgroup reads nothing and puts the sentinel into every element of its window's cells.
 template <int NV, int TJ>
 __global__ void __launch_bounds__(PK_T) k_lu_transpose(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
-                                                       double* __restrict__ pk, const int2* __restrict__ wins, int f0, int f1, int f2) {
-    __shared__ double buf[LU_NT][PK_W + 1];
+                                                       double* __restrict__ pk, const int2* __restrict__ wins, int g0, double gamma) {
+    using F = Pk<NV>;
+    __shared__ double buf[NV + 2][LU_COLS][PK_W + 2];
     const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];     // (tile, i-window), windows fastest
     const LuTask T = tiles[wn.x];
     const Blk& b = blks[T.blk];
-    const int nxm = b.nx - 1;
-    const int i0 = wn.y;
-    const int W = min(PK_W, nxm - i0 + 1);
-    const int nsteps = nxm + T.tj + T.tk - 2;
-    const int t = threadIdx.x;
-    constexpr int NF = Pk<NV>::NF;
-    const int z = (int)blockIdx.z;
-    const int f = z < f1 - f0 ? f0 + z : f2 + (z - (f1 - f0));
-    double* pf = pk + (size_t)T.pofs + (size_t)f * LU_NT;     // element (q, f, lane) at pf[q NF 64 + lane]
-    if (f >= Pk<NV>::DUF && f < Pk<NV>::DUB + NV) {
-        // a full tile's edge lanes lead the run (lane_pos): whole lines up to the last of them;
-        // a ragged tile's edges lie elsewhere, so all of its positions
-        constexpr int NSENT = (2 * (LU_NT / TJ) + 2 * (TJ - 2) + 15) / 16 * 16;
-        const int npos = T.tj == TJ && T.tk == LU_NT / TJ ? NSENT : LU_NT;
-        for (int e = t; e < (W + TJ + LU_NT / TJ - 2) * npos; e += PK_T) {
-            int q = i0 - 1 + e / npos, pos = e % npos, lane = pos_lane<TJ>(pos), jl = lane % TJ, kl = lane / TJ;
-            int i = q - jl - kl + 1;
-            if (i >= i0 && i < i0 + W && q < nsteps) pf[(size_t)q * NF * LU_NT + pos] = sentinel_value();
+    const int i0 = wn.y, W = min(PK_W, b.nx - 1 - i0 + 1);
+    const int g = g0 + (int)blockIdx.z;
+    auto none = [](int, int) {};
+    auto vec = [](int w, int& v, int& c) { F::vec_at(w, v, c); };
+    auto lin = [](int w, int, int) { return w; };
+    switch (g) {
+    case PG_NBR:
+        pack_group<NV, TJ, NV, NV + 2>(
+            buf, T, b, pk, i0, W, F::NBR, [&](int v, size_t s) { const double u = b.U[v][s]; return v > 4 && u < 0.0 ? 0.0 : u; },
+            [&](int c, int x) {
+                // comput_DFn's pressure of the undisturbed state
+                const double d = buf[0][c][x], m1 = buf[1][c][x], m2 = buf[2][c][x], m3 = buf[3][c][x], r = recip_nr(d);
+                buf[NV][c][x] = (gamma - 1.0) * (buf[4][c][x] - div_nr(0.5 * ((m1 * m1 + m2 * m2) + m3 * m3), d, r));
+                buf[NV + 1][c][x] = r;
+            },
+            [](int w, int& v, int& c) {
+                const int m = w % (NV + 2);
+                c = w / (NV + 2);
+                v = m < 4 ? m + 1 : m == 4 ? 0 : m;
+            },
+            [](int w, int, int c) { return c * F::CS + w % (NV + 2); });
+        __syncthreads();
+        pack_group<NV, TJ, 6, 6>(
+            buf, T, b, pk, i0, W, F::NBR, [&](int v, size_t s) { return v < 3 ? b.Lc[v][s] : b.Lv[v - 3][s]; }, none,
+            [](int w, int& v, int& c) { c = w / 6; v = w % 6; }, [](int, int v, int c) { return c * F::CS + F::LC + v; });
+        break;
+    case PG_R:
+        pack_group<NV, TJ, NV, NV>(buf, T, b, pk, i0, W, F::R, [&](int v, size_t s) { return b.Res[v][s]; }, none, vec, lin);
+        break;
+    case PG_AL:
+        pack_group<NV, TJ, F::NAL, 2 * F::NAL>(
+            buf, T, b, pk, i0, W, F::AL, [&](int v, size_t s) { return b.al[v][s]; },
+            [&](int c, int x) {
+#pragma unroll
+                for (int v = 0; v < F::NAL; v++) buf[F::NAL + v][c][x] = recip_nr(buf[v][c][x]);
+            },
+            [](int w, int& v, int& c) { const int m = w % F::CA; c = w / F::CA; v = (m & 1) * F::NAL + m / 2; }, lin);
+        break;
+    case PG_S:
+        pack_group<NV, TJ, 3, 3>(buf, T, b, pk, i0, W, F::SG, [&](int v, size_t s) { return b.S[v][s]; }, none,
+                                 [](int w, int& v, int& c) { c = w / 3; v = w % 3; }, [](int, int v, int c) { return 4 * c + v; });
+        break;
+    case PG_SENT_F:
+    case PG_SENT_B: {
+        constexpr int M = NV * LU_COLS;
+        const int nsteps = b.nx - 1 + T.tj + T.tk - 2, base = g == PG_SENT_F ? F::DUF : F::DUB;
+        for (int e = (int)threadIdx.x; e < (W + TJ + LU_COLS / TJ - 2) * M; e += PK_T) {
+            const int q = i0 - 1 + e / M, w = e % M;
+            int v, c;
+            F::vec_at(w, v, c);
+            const int x = q - c % TJ - c / TJ + 1 - i0;
+            if (x >= 0 && x < W && q < nsteps) pk[(size_t)T.pofs + (size_t)q * F::RUN + base + w] = sentinel_value();
         }
-        return;
+        break;
     }
-    for (int e = t; e < LU_NT * PK_W; e += PK_T) {
-        int r = e / PK_W, c = e % PK_W, jl = r % TJ, kl = r / TJ;
-        if (jl < T.tj && kl < T.tk && c < W) buf[r][c] = pack_value<NV>(b, f, IX(b, i0 + c, T.j0 + jl, T.k0 + kl));
-    }
-    __syncthreads();
-    for (int e = t; e < (W + TJ + LU_NT / TJ - 2) * LU_NT; e += PK_T) {
-        int q = i0 - 1 + e / LU_NT, lane = e % LU_NT, jl = lane % TJ, kl = lane / TJ;
-        int i = q - jl - kl + 1;
-        if (jl < T.tj && kl < T.tk && i >= i0 && i < i0 + W && q < nsteps) pf[(size_t)q * NF * LU_NT + lane_pos<TJ>(lane)] = buf[lane][i - i0];
+    default:          // the normals, a direction at a time
+        for (int d = 0; d < 3; d++) {
+            if (d > 0) __syncthreads();
+            pack_group<NV, TJ, 3, 3>(buf, T, b, pk, i0, W, F::N, [&](int v, size_t s) { return b.nv[3 * d + v][s]; }, none,
+                                     [](int w, int& v, int& c) { c = w / 3; v = w % 3; }, [&](int, int v, int c) { return 9 * c + 3 * d + v; });
+        }
     }
 }
 
-// sweep order -> block arrays for the backward sweep's DU (component m per grid z), for a host that
-// reads DU: the storage holds it from the end of the backward sweep until the next pack
+// sweep order -> block arrays for the backward sweep's DU, for a host that reads DU: the storage
+// holds it from the end of the backward sweep until the next pack
 template <int NV, int TJ>
 __global__ void __launch_bounds__(PK_T) k_lu_du_to_box(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
                                                        const double* __restrict__ pk, const int2* __restrict__ wins) {
-    __shared__ double buf[LU_NT][PK_W + 1];
+    using F = Pk<NV>;
+    constexpr int M = NV * LU_COLS;
+    __shared__ double buf[NV][LU_COLS][PK_W + 2];
     const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
     const LuTask T = tiles[wn.x];
     const Blk& b = blks[T.blk];
-    const int nxm = b.nx - 1;
-    const int i0 = wn.y;
-    const int W = min(PK_W, nxm - i0 + 1);
-    const int nsteps = nxm + T.tj + T.tk - 2;
-    const int t = threadIdx.x, m = (int)blockIdx.z;
-    constexpr int NF = Pk<NV>::NF;
-    const double* pf = pk + (size_t)T.pofs + (size_t)(Pk<NV>::DUB + m) * LU_NT;
-    for (int e = t; e < (W + TJ + LU_NT / TJ - 2) * LU_NT; e += PK_T) {
-        int q = i0 - 1 + e / LU_NT, lane = e % LU_NT, jl = lane % TJ, kl = lane / TJ;
-        int i = q - jl - kl + 1;
-        if (jl < T.tj && kl < T.tk && i >= i0 && i < i0 + W && q < nsteps) buf[lane][i - i0] = pf[(size_t)q * NF * LU_NT + lane_pos<TJ>(lane)];
+    const int i0 = wn.y, W = min(PK_W, b.nx - 1 - i0 + 1), t = (int)threadIdx.x;
+    for (int e = t; e < (W + TJ + LU_COLS / TJ - 2) * M; e += PK_T) {
+        const int q = i0 - 1 + e / M, w = e % M;
+        int v, c;
+        F::vec_at(w, v, c);
+        const int jl = c % TJ, kl = c / TJ, x = q - jl - kl + 1 - i0;
+        if (jl < T.tj && kl < T.tk && x >= 0 && x < W) buf[v][c][x] = pk[(size_t)T.pofs + (size_t)q * F::RUN + F::DUB + w];
     }
     __syncthreads();
-    double* box = b.DU[m];
-    for (int e = t; e < LU_NT * PK_W; e += PK_T) {
-        int r = e / PK_W, c = e % PK_W, jl = r % TJ, kl = r / TJ;
-        if (jl < T.tj && kl < T.tk && c < W) box[IX(b, i0 + c, T.j0 + jl, T.k0 + kl)] = buf[r][c];
+    for (int e = t; e < M * PK_W; e += PK_T) {
+        const int x = e % PK_W, c = (e / PK_W) % LU_COLS, v = e / (PK_W * LU_COLS), jl = c % TJ, kl = c / TJ;
+        if (jl < T.tj && kl < T.tk && x < W) b.DU[v][IX(b, i0 + x, T.j0 + jl, T.k0 + kl)] = buf[v][c][x];
     }
 }
 
@@ -334,101 +391,38 @@ __global__ void __launch_bounds__(PK_T) k_lu_du_to_box(const Blk* __restrict__ b
 template <int NV>
 __global__ void k_fill_sentinel(double* p, long long n) {
     using F = Pk<NV>;
-    const long long pad = (long long)LU_PAD_STEPS * F::NF * LU_NT;
+    const long long pad = (long long)LU_PAD_STEPS * F::RUN;
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-        const int f = (int)(((e - pad) / LU_NT) % F::NF);
-        if (e < pad || e >= n - pad || (f >= F::DUF && f < F::DUB + NV)) p[e] = sentinel_value();
+        if (e < pad || e >= n - pad || (int)((e - pad) % F::RUN) >= F::DUF) p[e] = sentinel_value();
     }
 }
 
 
-// inputs of one step of wave D: its own cell's face normal and (forward) area in direction D;
-// the neighbour's U, Lc, Lv and (backward) S; and the Res (forward) or forward DU (backward) with
-// the diagonal of the cell whose DU the wave completes at this step
-template <int NV, bool FWD, int D>
-struct TeamIn {
-    double n[3], S;
-    double U[NV], Lc, Lv, Sn;
-    double R[NV], al[2];
-};
+// value x of part M of the lane's quad
+template <int M>
+__device__ __forceinline__ double quad_get(double x) {
+    const long long v = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)v, M * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), M * 0x55, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double quad_sum3(double x) { return (quad_get<0>(x) + quad_get<1>(x)) + quad_get<2>(x); }
 
-// eo: own element of the step, en: the neighbour's, es: the element of the cell whose DU is
-// completed; field f of an element at e[f * 64]
-template <int NV, bool FWD, int D>
-__device__ __forceinline__ void team_load(const double* __restrict__ eo, const double* __restrict__ en,
-                                          const double* __restrict__ es, TeamIn<NV, FWD, D>& t) {
-    using F = Pk<NV>;
-#pragma unroll
-    for (int c = 0; c < 3; c++) t.n[c] = eo[(F::N + 3 * D + c) * LU_NT];
-    t.S = FWD ? eo[(F::S + D) * LU_NT] : 0.0;
-#pragma unroll
-    for (int m = 0; m < NV; m++) t.U[m] = en[(F::U + m) * LU_NT];
-    t.Lc = en[(F::LC + D) * LU_NT];
-    t.Lv = en[(F::LV + D) * LU_NT];
-    t.Sn = FWD ? 0.0 : en[(F::S + D) * LU_NT];
-#pragma unroll
-    for (int m = 0; m < NV; m++) t.R[m] = es[((FWD ? F::R : F::DUF) + m) * LU_NT];
-    t.al[0] = es[F::AL * LU_NT];
-    t.al[1] = NV == 6 ? es[(F::AL + (FWD ? 1 : 2)) * LU_NT] : 0.0;
+// the convective flux F(U) n of comput_DFn (sub_LU_SGS.f90:135-158) in the quad's components, from
+// the density d, its reciprocal and the pressure; the normal velocity is formed by all four lanes
+__device__ __forceinline__ void quad_flux(double Ua, double Ub, double d, double rd, double p, double n, bool energy, double& fa, double& fb) {
+    const double un = div_nr(quad_sum3(Ua * n), d, rd);
+    const double fm = Ua * un + p * n, fe = (Ua + p) * un;
+    fa = energy ? fe : fm;
+    fb = Ub * un;
 }
 
-// the upstream tile's DU of a cell (may still be the sentinel).  An ordinary load, which the
-// L2 of this XCD may serve: within a sweep an element only ever holds the sentinel or its final
-// value, and every kernel starts with the L2 invalidated, so a cached copy is either current or a
-// sentinel, and a sentinel sends the lane to the device-coherent reloads of team_wait_remote.
-// Against device-coherent loads here, the sweeps of a 257x97x33 C-grid take 8 % less time.
-template <int NV, bool FWD>
-__device__ __forceinline__ void team_load_du(const double* __restrict__ e, double* DU) {
-    using F = Pk<NV>;
-#pragma unroll
-    for (int m = 0; m < NV; m++) DU[m] = e[((FWD ? F::DUF : F::DUB) + m) * LU_NT];
-}
-
-// du of one upstream neighbour (sub_LU_SGS.f90:42-60 forward, :94-119 backward)
-template <int NV, bool FWD>
-__device__ __forceinline__ void team_neighbour(double* du, const double* Un_in, const double* DUn, double Lcn, double Lvn,
-                                               double Sn, const double* n, double Sd, double wlu, double gamma, bool visc) {
-    double Un[NV], DF[NV];
-#pragma unroll
-    for (int m = 0; m < NV; m++) Un[m] = Un_in[m];
-#pragma unroll
-    for (int m = 5; m < NV; m++) if (Un[m] < 0.0) Un[m] = 0.0;     // limit_vt
-    comput_dfn_nr<NV>(DF, Un, DUn, n[0], n[1], n[2], gamma);
-    const double wLc = wlu * Lcn;
-    if (FWD) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) du[m] = 0.5 * (DF[m] * Sd + wLc * DUn[m]);
-    } else {
-#pragma unroll
-        for (int m = 0; m < NV; m++) du[m] = -0.5 * (DF[m] * Sn - wLc * DUn[m]);
-    }
-    if (visc) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) du[m] = du[m] + Lvn * DUn[m];
-    }
-}
-
-// reload an upstream DU until the producer has replaced the sentinel; true when the wait gives up
-template <int NV, bool FWD>
-__device__ __forceinline__ bool team_wait_remote(const double* __restrict__ er, double* DU, int* __restrict__ err) {
-    using F = Pk<NV>;
-    long polls = 0;
-    while (true) {
-        bool ready = true;
-#pragma unroll
-        for (int m = 0; m < NV; m++) ready = ready && !is_sentinel(DU[m]);
-        if (ready) return false;
-        if (++polls > LU_POLL_LIMIT ||
-            ((polls & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) ||
-            (polls == 1 && lu_fail_waits(err))) {
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return true;
-        }
-        __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-        for (int m = 0; m < NV; m++)
-            if (is_sentinel(DU[m])) DU[m] = ld_coherent(er + ((FWD ? F::DUF : F::DUB) + m) * LU_NT);
-    }
+// du of one upstream neighbour component (sub_LU_SGS.f90:42-60 forward, :94-119 backward); without
+// viscosity Lv is zero
+template <bool FWD>
+__device__ __forceinline__ double team_term(double DF, double DU, double wLc, double Lv, double S) {
+    const double t = FWD ? 0.5 * (DF * S + wLc * DU) : -0.5 * (DF * S - wLc * DU);
+    return t + Lv * DU;
 }
 
 // a for the lanes whose bit of mk is set, else b: one v_cndmask per half, so the choice cannot
@@ -441,189 +435,373 @@ __device__ __forceinline__ double pick(unsigned long long mk, double a, double b
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// the high half of the sentinel is enough to know it by: no arithmetic produces a signalling NaN
+__device__ __forceinline__ bool maybe_sentinel(double v) {
+    return (unsigned)(__double_as_longlong(v) >> 32) == (unsigned)(LU_SENTINEL >> 32);
+}
+
+// reload an upstream DU (elements ea, eb) on the waiting lanes until the producer has replaced the
+// sentinel; true when the wait gives up
+__device__ __forceinline__ bool team_wait_remote(const double* ea, const double* eb, bool waiting, double& a, double& b, int* __restrict__ err) {
+    long polls = 0;
+    while (true) {
+        const bool pend = waiting && (is_sentinel(a) || is_sentinel(b));
+        if (__builtin_amdgcn_ballot_w64(pend) == 0) return false;
+        if (++polls > LU_POLL_LIMIT ||
+            ((polls & 255) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) ||
+            (polls == 1 && lu_fail_waits(err))) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return true;
+        }
+        if (pend) { a = ld_coherent(ea); b = ld_coherent(eb); }
+    }
+}
+
 __device__ __forceinline__ void team_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// LDS of a tile team: the records of the previous step (double-buffered by step parity) that
-// the downstream lanes read, one array per value so a wave's 64 lanes touch 64 consecutive
-// doubles, and the three waves' neighbour terms of the current step
-template <int NV>
-struct TeamShared {
-    double dus[2][3][NV][LU_NT];      // [step parity][direction][component][lane]
+// LDS of a tile team.  ring: LU_RING slots of step inputs, filled by the loader wave; slot q holds
+// step q's piece of the tile's run (R to N forward, NBR to DUF backward) and, for the lanes at the
+// tile's upstream edges, the NBR (and backward SG) chunks that step q + 1 reads of the upstream
+// tiles.  du: the three direction waves' neighbour terms, double-buffered by step parity.
+constexpr int LU_RING = 6, LU_FAR = LU_RING - 1;      // slots, and how many steps ahead the loader writes
+template <int NV, bool FWD, int TJ> struct TeamLds {
+    using F = Pk<NV>;
+    static constexpr int BASE = FWD ? F::R : F::NBR;                 // first double of a run's piece
+    static constexpr int EDGE = TJ + LU_COLS / TJ;                   // upstream columns: along j, then along k
+    static constexpr int PIECE = F::SWEEP * 8, NBRS = PIECE, SGS = NBRS + EDGE * F::CS * 8,
+                         SLOT = (SGS + (FWD ? 0 : EDGE * 32) + 15) / 16 * 16;      // byte offsets in a slot
+    static constexpr int CHUNKS = EDGE * F::CS / 2;                  // 16-byte pieces of the upstream NBR chunks
+    static constexpr int LOADS = (PIECE + 1023) / 1024 + (CHUNKS + 63) / 64 + (FWD ? 0 : 1);     // per step
+    static_assert(PIECE % 16 == 0 && EDGE * 2 <= LU_NT && LOADS * (LU_FAR - 2) < 64, "loads of a step");
+    alignas(16) char ring[LU_RING * SLOT];
+    double du[2][3][2][LU_NT];        // [step parity][direction][component a, b][lane]
     int bail;
 };
 
-// One wave's part of a tile's sweep.  The loop is unrolled by three with three register sets for
-// the prefetched inputs, so a step's loads are issued two full steps before their use; an upstream
-// tile's DU is loaded one step before its use.  Every global load and store is issued by all
-// lanes (lanes without a cell address elements nobody reads, inside the tile's storage or the
-// buffer's padding), which keeps the wait counts the compiler derives independent of the lane
-// masks.  Each lane walks its streams of elements with one pointer each, advanced by one step of
-// NF x 64 elements per step.
+// inputs of one step of wave D for this lane's components (a: momentum or energy, b: density or a
+// turbulence variable): its own cell's face normal and (forward) area in direction D; the
+// neighbour's U, pressure, 1/density, Lc, Lv and (backward) S; and the Res (forward) or forward DU
+// (backward), the diagonal and its reciprocal of the cell whose DU the wave completes at this step
+struct TeamIn {
+    double n, S;
+    double Ua, Ub, P, RD, Lc, Lv;
+    double Ra, Rb, ala, rala, alb, ralb;
+};
+
+// 16 bytes per lane from global memory to the LDS: lane l's go to dst + 16 l
+__device__ __forceinline__ void to_lds(const char* src, char* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// wait until at most n of this wave's loads are outstanding (the other counters are left alone)
+template <int n>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+    asm volatile("" ::: "memory");
+}
+
+// The loader wave of a tile: at step q it starts the loads of step q + LU_FAR into the ring and
+// waits for those of step q + 2, which the direction waves read from the next barrier on.  The
+// direction waves finished reading slot q - 1, the one written now, before the last barrier.  A
+// step's piece of the run is contiguous, so its 5 KB take five loads of 16 bytes per lane; the
+// direction waves would need 45 loads of 8 bytes for them, at 16 clocks of the CU's address path
+// each, twice what the step's arithmetic takes.
+template <int NV, bool FWD, int TJ>
+__device__ void team_load(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask& T, const double* __restrict__ pk, int lane) {
+    using F = Pk<NV>;
+    using L = TeamLds<NV, FWD, TJ>;
+    constexpr int TK = LU_COLS / TJ, PPC = F::CS / 2;         // pieces per NBR chunk
+    const int nxm = b.nx - 1, nsteps = nxm + T.tj + T.tk - 2;
+    const long dstep = (FWD ? (long)F::RUN : -(long)F::RUN) * 8;
+    const double* first = pk + T.pofs + (FWD ? 0L : (long)(nsteps - 1) * F::RUN);       // the tile's run at step 0
+    const char* run0 = (const char*)(first + L::BASE) + 16 * lane;
+    // the upstream column `e` of the edge list and its run at this tile's step 0; a tile without
+    // that upstream tile takes its own, which nobody reads
+    auto edge = [&](int e) -> const double* {
+        const bool along_j = e < TK;
+        const int jlu = FWD ? T.tj_up - 1 : 0, klu = FWD ? T.tk_up - 1 : 0;
+        if ((along_j ? T.dep_j : T.dep_k) < 0) return first;
+        const int c = along_j ? jlu + TJ * e : (e - TK) + TJ * klu;
+        const int s0 = FWD ? (along_j ? jlu : klu) : nxm + (along_j ? T.tk : T.tj) - 2;
+        return pk + (along_j ? T.pofs_j : T.pofs_k) + (long)s0 * F::RUN + (long)c * F::CS;
+    };
+    // element offsets within a run: the chunk's column is folded into edge(); the areas' chunks
+    // lie 4 doubles apart instead of CS
+    constexpr int NE = (L::CHUNKS + 63) / 64;
+    const char* ep[NE];
+#pragma unroll
+    for (int u = 0; u < NE; u++) {
+        const int r = min(u * 64 + lane, L::CHUNKS - 1);
+        ep[u] = (const char*)(edge(r / PPC) + F::NBR) + 16 * (r % PPC);
+    }
+    const char* sp = nullptr;
+    if constexpr (!FWD) {
+        const int r = min(lane, 2 * L::EDGE - 1), e = r / 2;
+        const bool along_j = e < TK;
+        const int c = (along_j ? T.dep_j : T.dep_k) < 0 ? 0 : along_j ? TJ * e : e - TK;
+        sp = (const char*)(edge(e) - (long)c * F::CS + F::SG + 4 * c) + 16 * (r % 2);
+    }
+    auto issue = [&](int q, int slot) {
+        char* d = sh.ring + slot * L::SLOT;
+        const char* s = run0 + (long)q * dstep;
+#pragma unroll
+        for (int o = 0; o + 1024 <= L::PIECE; o += 1024) to_lds(s + o, d + o);
+        constexpr int REST = L::PIECE % 1024;
+        if constexpr (REST > 0) {
+            if (lane < REST / 16) to_lds(s + (L::PIECE - REST), d + (L::PIECE - REST));
+        }
+        // the upstream columns of the next step
+#pragma unroll
+        for (int u = 0; u < NE; u++)
+            if (u * 64 + lane < L::CHUNKS) to_lds(ep[u] + (long)(q + 1) * dstep, d + L::NBRS + u * 1024);
+        if constexpr (!FWD) {
+            if (lane < 2 * L::EDGE) to_lds(sp + (long)(q + 1) * dstep, d + L::SGS);
+        }
+    };
+    int slot = 0;
+    issue(-1, LU_RING - 1);
+#pragma unroll 1
+    for (int q = 0; q < LU_FAR; q++) issue(q, q);
+    slot = LU_FAR;
+    wait_loads<L::LOADS * (LU_FAR - 2)>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_s_barrier();      // the direction waves have read slot -1, which step 0 overwrites
+#pragma unroll 1
+    for (int q = 0; q < nsteps; q++) {
+        issue(q + LU_FAR, slot);
+        slot = slot + 1 == LU_RING ? 0 : slot + 1;
+        wait_loads<L::LOADS * (LU_FAR - 2)>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (q % LU_RING == LU_RING - 1 && *(volatile int*)&sh.bail != 0) break;
+    }
+    wait_loads<0>();      // no load may reach the LDS after the workgroup has given it back
+}
+
+// One direction wave's part of a tile's sweep.  No arithmetic is masked: what a lane without a cell
+// computes is read by no lane that has one, and it is stored to elements nobody reads, inside the
+// tile's storage.
 template <int NV, bool FWD, int D, int TJ>
-__device__ void team_sweep(TeamShared<NV>& sh, const Blk& b, const LuTask& T, double* __restrict__ pk,
+__device__ void team_sweep(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask& T, double* __restrict__ pk,
                            int* __restrict__ err, const Par& p, int lane) {
     using F = Pk<NV>;
-    constexpr long STEP = (long)F::NF * LU_NT;                 // elements per step of a tile
-    const int jl = lane % TJ, kl = lane / TJ;
+    using L = TeamLds<NV, FWD, TJ>;
+    constexpr int C = LU_COLS, NB = F::NB, TK = C / TJ;
+    const int part = lane % LU_PARTS, col = lane / LU_PARTS;
+    const int pb_ = part < NB ? part : NB - 1;              // this lane's slot of the (density, turbulence) group
+    const int jl = col % TJ, kl = col / TJ;
     const bool live = jl < T.tj && kl < T.tk;
     const int jo = FWD ? jl : T.tj - 1 - jl, ko = FWD ? kl : T.tk - 1 - kl;
     const int j = T.j0 + jl, k = T.k0 + kl;
     const int nxm = b.nx - 1;
     const double wlu = p.w_LU, gamma = p.gamma;
-    const bool visc = p.visc == 1;
     const int nsteps = nxm + T.tj + T.tk - 2;
-    // the neighbour of direction D: another lane of the tile, or the upstream tile
+    // the neighbour of direction D: another column of the tile, or the upstream tile
     const bool has_d = D == 0 ? true : D == 1 ? (FWD ? j != 1 : j != b.ny - 1) : (FWD ? k != 1 : k != b.nz - 1);
     const bool inside = D == 0 ? true : D == 1 ? jo > 0 : ko > 0;
     const bool remote = D > 0 && live && has_d && !inside;
     const unsigned long long rmask = __builtin_amdgcn_ballot_w64(remote);
-    // the lane whose cell of the previous step this lane reads (lanes without one read their own)
-    const int src = D == 0 || !inside ? lane : D == 1 ? (FWD ? lane - 1 : lane + 1) : (FWD ? lane - TJ : lane + TJ);
+    // the column whose cell of the previous step this lane reads (columns without one read their own)
+    const int scol = D == 0 || !inside ? col : D == 1 ? (FWD ? col - 1 : col + 1) : (FWD ? col - TJ : col + TJ);
+    const int src = scol * LU_PARTS + part;
+    const bool energy = part == 3;
 
     // cell i of this lane at step q is i0 + dir q
     const int i0 = FWD ? 1 - jo - ko : nxm + jo + ko;
     const int dir = FWD ? 1 : -1;
-    // this lane's element at step 0 and per step
-    const long base0 = (long)T.pofs + (FWD ? 0L : (long)(nsteps - 1) * STEP);
-    const long own0 = base0 + lane_pos<TJ>(lane);
-    const long dstep = FWD ? STEP : -STEP;
-    // the element of lane src one step back
-    const long src0 = base0 - dstep + lane_pos<TJ>(src);
-    // the upstream element: the upstream tile stores by forward step, the lane across the edge is
-    // jlu + 8 kl (j) or jl + 8 klu (k); lanes without one follow their own stream
-    long rem0 = own0;
-    if (remote) {
-        const int jlu = FWD ? T.tj_up - 1 : 0, klu = FWD ? T.tk_up - 1 : 0;
-        const long long pofs_r = D == 1 ? T.pofs_j : T.pofs_k;
-        const int lane_r = D == 1 ? jlu + TJ * kl : jl + TJ * klu;
-        // forward step of the upstream cell at this lane's step 0 (forward: i - 1 + jl_r + kl_r)
-        const int s0 = FWD ? (D == 1 ? jlu : klu) : nxm + (D == 1 ? T.tk : T.tj) - 2;
-        rem0 = (long)pofs_r + (long)s0 * STEP + lane_pos<TJ>(lane_r);
-    }
-    const long nb0 = remote ? rem0 : src0;
-    auto own_p = [&](int q) { return pk + own0 + (long)q * dstep; };
-    auto src_p = [&](int q) { return pk + src0 + (long)q * dstep; };
-    auto nb_p = [&](int q) { return pk + nb0 + (long)q * dstep; };
-    auto rem_p = [&](int q) { return pk + rem0 + (long)q * dstep; };
-    auto load = [&](int q, TeamIn<NV, FWD, D>& t) { team_load<NV, FWD, D>(own_p(q), nb_p(q), src_p(q), t); };
-    auto active = [&](int q) { const int i = i0 + dir * q; return live && q < nsteps && i >= 1 && i <= nxm; };
+    // the lane's elements of a ring slot: its own cell's, of column scol one step back, and of the
+    // neighbour, which is column scol or a column of the upstream edge
+    const int edge = D == 1 ? kl : TK + jl;
+    const char* ring = sh.ring;
+    const char* on = ring + 8 * (F::N - L::BASE + 9 * col + 3 * D + (part < 3 ? part : 2));
+    const char* os = ring + 8 * (F::SG - L::BASE + 4 * col + D);
+    const char* ra = ring + 8 * ((FWD ? F::R : F::DUF) - L::BASE + 4 * scol + part);
+    const char* rb = ring + 8 * ((FWD ? F::R : F::DUF) - L::BASE + 4 * C + NB * scol + pb_);
+    const char* al = ring + 8 * (F::AL - L::BASE + F::CA * scol);
+    const char* alb = al + (NV == 6 && pb_ == 1 ? (FWD ? 16 : 32) : 0);
+    const char* nb = ring + (remote ? L::NBRS + 8 * F::CS * edge : 8 * (F::NBR - L::BASE + F::CS * scol));
+    const char* ns = ring + (remote ? L::SGS + 32 * edge : 8 * (F::SG - L::BASE + 4 * scol)) + 8 * D;
+    const char *na = nb + 8 * part, *nbb = nb + 8 * (4 + pb_);
+    auto ld = [](const char* a) { return *(const double*)a; };
+    // step q's inputs: the own cell from slot q, the rest from slot q - 1
+    auto read = [&](int own, int prev, TeamIn& t) {
+        const int o = own * L::SLOT, s = prev * L::SLOT;
+        t.Ua = ld(na + s);
+        t.Ub = ld(nbb + s);
+        t.P = ld(nb + s + 8 * F::P);
+        t.RD = ld(nb + s + 8 * F::RD);
+        t.n = ld(on + o);
+        t.Ra = ld(ra + s);
+        t.Rb = ld(rb + s);
+        t.ala = ld(al + s);
+        t.rala = ld(al + s + 8);
+        if constexpr (NV == 6) { t.alb = ld(alb + s); t.ralb = ld(alb + s + 8); }
+        t.Lc = ld(nb + s + 8 * (F::LC + D));
+        t.Lv = ld(nb + s + 8 * (F::LV + D));
+        t.S = FWD ? ld(os + o) : ld(ns + s);
+    };
 
-    // DU of the cell of lane src at step q - 1, from the terms of that step
-    auto complete = [&](int q, const TeamIn<NV, FWD, D>& in, double* DUs) {
-        const int pb = (q & 1) ^ 1;
-        // components 1-5 (and 7) share one diagonal, the SA component has its own
-        const double r0 = recip_nr(in.al[0]), r1 = NV == 6 ? recip_nr(in.al[1]) : 0.0;
-#pragma unroll
-        for (int m = 0; m < NV; m++) {
-            const bool own = NV == 6 && m == 5;
-            const double al = in.al[own ? 1 : 0], ra = own ? r1 : r0;
-            double acc = FWD ? in.R[m] : 0.0;
-            acc = ((acc + sh.dus[pb][0][m][src]) + sh.dus[pb][1][m][src]) + sh.dus[pb][2][m][src];
-            DUs[m] = FWD ? div_nr(acc, al, ra) : in.R[m] + div_nr(acc, al, ra);
+    // The upstream tile's DU (may still be the sentinel).  An ordinary load, which the L2 of this
+    // XCD may serve: within a sweep an element only ever holds the sentinel or its final value, and
+    // every kernel starts with the L2 invalidated, so a cached copy is either current or a
+    // sentinel, and a sentinel sends the lane to the device-coherent reloads of team_wait_remote.
+    // The columns of a row (D = 1) or line (D = 2) of the tile read the same upstream column.
+    const long dstep = (FWD ? (long)F::RUN : -(long)F::RUN) * 8;
+    char* run0 = (char*)(pk + T.pofs + (FWD ? 0L : (long)(nsteps - 1) * F::RUN));
+    constexpr int DU = (FWD ? F::DUF : F::DUB) * 8;
+    const int oa = 8 * (4 * col + part), ob = 8 * (4 * C + NB * col + pb_);
+    const char *ea = run0 + DU + oa, *eb = run0 + DU + ob;
+    if (D > 0 && (D == 1 ? T.dep_j : T.dep_k) >= 0) {
+        const int jlu = FWD ? T.tj_up - 1 : 0, klu = FWD ? T.tk_up - 1 : 0;
+        const int c = D == 1 ? jlu + TJ * kl : jl + TJ * klu;
+        const int s0 = FWD ? (D == 1 ? jlu : klu) : nxm + (D == 1 ? T.tk : T.tj) - 2;
+        const char* e = (const char*)(pk + (D == 1 ? T.pofs_j : T.pofs_k) + (long)s0 * F::RUN) + DU;
+        ea = e + 8 * (4 * c + part);
+        eb = e + 8 * (4 * C + NB * c + pb_);
+    }
+    auto load_du = [&](int q, double& a, double& c) { a = ld(ea + (long)q * dstep); c = ld(eb + (long)q * dstep); };
+
+    // DU of the cell of column scol at the step before, from the terms of that step
+    auto complete = [&](int par, const TeamIn& in, double& a, double& c) {
+        const auto& d = sh.du[par ^ 1];
+        const double ta = d[0][0][src], tb = d[0][1][src], ua = d[1][0][src], ub = d[1][1][src], va = d[2][0][src], vb = d[2][1][src];
+        const double ab = NV == 6 ? in.alb : in.ala, rab = NV == 6 ? in.ralb : in.rala;
+        if (FWD) {
+            a = div_nr(((in.Ra + ta) + ua) + va, in.ala, in.rala);
+            c = div_nr(((in.Rb + tb) + ub) + vb, ab, rab);
+        } else {
+            a = in.Ra + div_nr((ta + ua) + va, in.ala, in.rala);
+            c = in.Rb + div_nr((tb + ub) + vb, ab, rab);
         }
     };
     // wave 0 stores the DU of its own cell of step q - 1 (device-coherent: the elements a
     // neighbour tile reads need it, and one kind of store for all lanes)
-    auto store = [&](int q, const double* DUs) {
+    auto store = [&](int q, double a, double c) {
         if (D == 0 && q >= 1) {
-            double* e = own_p(q - 1);
-#pragma unroll
-            for (int m = 0; m < NV; m++) st_coherent(e + ((FWD ? F::DUF : F::DUB) + m) * LU_NT, DUs[m]);
+            char* e = run0 + (long)(q - 1) * dstep + DU;
+            st_coherent((double*)(e + (unsigned)oa), a);
+            st_coherent((double*)(e + (unsigned)ob), c);
         }
     };
 
-    // one step: complete the read cell's DU, then this direction's term of the own cell, a
-    // barrier; with check, true when the workgroup gives up.  Every third step checks (an LDS
-    // read after the barrier that the other steps skip): a wave that gave up has set the error
-    // flag, so the waits of the steps in between give up within 256 polls and their values are
-    // discarded
-    auto step = [&](int q, const TeamIn<NV, FWD, D>& in, double* rdu, bool check) -> bool {
-        double DUs[NV];
-        complete(q, in, DUs);
-        store(q, DUs);
+    // one step (of parity par): the flux of the neighbour's undisturbed state, the DU of the read
+    // cell, the flux of the disturbed state, this direction's term of the own cell
+    auto step = [&](int q, int par, const TeamIn& in, double Da, double Db) {
+        double DUa, DUb, f1a, f1b;
+        const double d1 = NB == 1 ? in.Ub : quad_get<0>(in.Ub);
+        quad_flux(in.Ua, in.Ub, d1, in.RD, in.P, in.n, energy, f1a, f1b);
+        complete(par, in, DUa, DUb);
+        store(q, DUa, DUb);
         const int i = i0 + dir * q;
-        if (active(q)) {
-            const bool has = D == 0 ? (FWD ? i != 1 : i != nxm) : has_d;
-            if (D > 0 && remote) {
-                // wait off the common path, so the wait counts in front of it do not cover the
-                // loads issued for later steps
-                bool ready = true;
-#pragma unroll
-                for (int m = 0; m < NV; m++) ready = ready && !is_sentinel(rdu[m]);
-                if (!ready && team_wait_remote<NV, FWD>(rem_p(q), rdu, err)) sh.bail = 1;
+        if constexpr (D > 0) {
+            if ((__builtin_amdgcn_ballot_w64(maybe_sentinel(Da) || maybe_sentinel(Db)) & rmask) != 0) {
+                const bool waiting = remote && i >= 1 && i <= nxm;
+                if (team_wait_remote((const double*)(ea + (long)q * dstep), (const double*)(eb + (long)q * dstep), waiting, Da, Db, err)) sh.bail = 1;
             }
-            double DUn[NV];
-#pragma unroll
-            for (int m = 0; m < NV; m++) DUn[m] = D > 0 ? pick(rmask, rdu[m], DUs[m]) : DUs[m];
-            double du[NV];
-            team_neighbour<NV, FWD>(du, in.U, DUn, in.Lc, in.Lv, in.Sn, in.n, in.S, wlu, gamma, visc);
-#pragma unroll
-            for (int m = 0; m < NV; m++) sh.dus[q & 1][D][m][lane] = has ? du[m] : 0.0;
+            DUa = pick(rmask, Da, DUa);
+            DUb = pick(rmask, Db, DUb);
         }
-        team_barrier();
-        return check && sh.bail != 0;
+        const double Ua = in.Ua + DUa, Ub = in.Ub + DUb;
+        const double d2 = NB == 1 ? Ub : quad_get<0>(Ub), r2 = recip_nr(d2);
+        const double ke = div_nr(0.5 * quad_sum3(Ua * Ua), d2, r2);
+        double f2a, f2b;
+        quad_flux(Ua, Ub, d2, r2, (gamma - 1.0) * (quad_get<3>(Ua) - ke), in.n, energy, f2a, f2b);
+        const double wLc = wlu * in.Lc;
+        const double da = team_term<FWD>(f2a - f1a, DUa, wLc, in.Lv, in.S), db = team_term<FWD>(f2b - f1b, DUb, wLc, in.Lv, in.S);
+        // a lane's terms before its first cell and those of a direction without a neighbour stay zero
+        if (D == 0 ? (FWD ? i > 1 : i < nxm) : has_d) {
+            sh.du[par][D][0][lane] = da;
+            sh.du[par][D][1][lane] = db;
+        }
     };
 
-    TeamIn<NV, FWD, D> iA, iB, iC;
-    double rA[NV], rB[NV], rC[NV];
-    load(0, iA);
-    load(1, iB);
-    load(2, iC);
-    if constexpr (D > 0) team_load_du<NV, FWD>(rem_p(0), rA);
-    for (int q = 0; q < nsteps; q += 3) {
-        if constexpr (D > 0) team_load_du<NV, FWD>(rem_p(q + 1), rB);
-        if (step(q, iA, rA, false)) return;
-        load(q + 3, iA);
-        if (q + 1 >= nsteps) break;
-        if constexpr (D > 0) team_load_du<NV, FWD>(rem_p(q + 2), rC);
-        if (step(q + 1, iB, rB, false)) return;
-        load(q + 4, iB);
-        if (q + 2 >= nsteps) break;
-        if constexpr (D > 0) team_load_du<NV, FWD>(rem_p(q + 3), rA);
-        if (step(q + 2, iC, rC, true)) return;
-        load(q + 5, iC);
+    // The loop is unrolled over the ring's slots.  The inputs of step q + 1 are read during step q,
+    // an upstream tile's DU is loaded LU_AHEAD steps before its use.  The last step of a round
+    // checks whether a wave gave up (an LDS read after the barrier that the others skip): that wave
+    // has set the error flag, so the waits of the steps in between give up within 256 polls and
+    // their values are discarded, and all waves leave at the same barrier.
+    constexpr int LU_AHEAD = 2;
+    static_assert(LU_RING % 2 == 0, "the step parity is fixed per unrolled step");
+    TeamIn in[2];
+    double Da[LU_RING], Db[LU_RING];
+    if constexpr (D > 0) {
+#pragma unroll
+        for (int u = 0; u < LU_AHEAD; u++) load_du(u, Da[u], Db[u]);
+    }
+    team_barrier();
+    read(0, LU_RING - 1, in[0]);
+    team_barrier();
+    for (int q0 = 0; q0 < nsteps; q0 += LU_RING) {
+#pragma unroll
+        for (int u = 0; u < LU_RING; u++) {
+            const int q = q0 + u;
+            if (q >= nsteps) break;
+            constexpr int W = LU_RING;
+            if constexpr (D > 0) load_du(q + LU_AHEAD, Da[(u + LU_AHEAD) % W], Db[(u + LU_AHEAD) % W]);
+            read((u + 1) % W, u, in[(u + 1) & 1]);
+            step(q, u & 1, in[u & 1], Da[u], Db[u]);
+            team_barrier();
+            if (u == W - 1 && sh.bail != 0) return;
+        }
     }
     // the DU of the last step
     if constexpr (D == 0) {
-        TeamIn<NV, FWD, D> last;
-        load(nsteps, last);
-        double DUs[NV];
-        complete(nsteps, last, DUs);
-        store(nsteps, DUs);
+        double a, c;
+        if (nsteps & 1) complete(1, in[1], a, c);
+        else complete(0, in[0], a, c);
+        store(nsteps, a, c);
     }
 }
 
+constexpr int LT_NT = 4 * LU_NT;      // the three direction waves and the loader
 template <int NV, bool FWD, int TJ>
 __global__ void __launch_bounds__(LT_NT) k_lusgs_team(const Blk* __restrict__ blks, const LuTask* __restrict__ tasks,
                                                       double* __restrict__ pk, int* __restrict__ err, Par p) {
-    __shared__ TeamShared<NV> sh;
+    __shared__ TeamLds<NV, FWD, TJ> sh;
     const int wave = threadIdx.x / LU_NT, lane = threadIdx.x % LU_NT;
     // a sweep earlier in the launch sequence gave up waiting: this one does nothing either (its
     // DU stays unused, the update kernels leave U as it is)
     if (threadIdx.x == 0) sh.bail = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the terms of the steps before a lane's first cell, and of a direction without a neighbour
+    for (int e = (int)threadIdx.x; e < 2 * 3 * 2 * LU_NT; e += LT_NT) (&sh.du[0][0][0][0])[e] = 0.0;
     __syncthreads();
     if (sh.bail != 0) return;
     const LuTask T = tasks[blockIdx.x];
     const Blk& b = blks[T.blk];
     if (wave == 0) team_sweep<NV, FWD, 0, TJ>(sh, b, T, pk, err, p, lane);
     else if (wave == 1) team_sweep<NV, FWD, 1, TJ>(sh, b, T, pk, err, p, lane);
-    else team_sweep<NV, FWD, 2, TJ>(sh, b, T, pk, err, p, lane);
+    else if (wave == 2) team_sweep<NV, FWD, 2, TJ>(sh, b, T, pk, err, p, lane);
+    else team_load<NV, FWD, TJ>(sh, b, T, pk, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
 // host side
 
+// The tiles of a launch in the order in which they can start: the first tiles of all blocks, then
+// the next ones.  An upstream tile starts earlier, so it keeps a lower number.
+void lusgs_start_order(std::vector<LuTask>& tasks) {
+    std::vector<int> at(tasks.size()), num(tasks.size());
+    for (size_t q = 0; q < at.size(); q++) at[q] = (int)q;
+    std::stable_sort(at.begin(), at.end(), [&](int a, int b) { return tasks[a].start < tasks[b].start; });
+    std::vector<LuTask> out;
+    for (size_t q = 0; q < at.size(); q++) { num[at[q]] = (int)q; out.push_back(tasks[at[q]]); }
+    for (LuTask& t : out) {
+        if (t.dep_j >= 0) t.dep_j = num[t.dep_j];
+        if (t.dep_k >= 0) t.dep_k = num[t.dep_k];
+    }
+    tasks.swap(out);
+}
+
 // Tiles of every block for one sweep direction, numbered so that upstream tiles come first.
 // The sweep-ordered storage of a tile does not depend on the direction: tiles are laid out block
-// after block in forward order, each taking (nsteps x 64) elements.
-std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int NF, int TJ, long long* total) {
-    const int TK = LU_NT / TJ;
+// after block in forward order, each taking nsteps runs of `run` doubles.
+std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int run, int TJ, int TK, long long* total) {
     std::vector<LuTask> out;
-    const long long pad = (long long)LU_PAD_STEPS * NF * LU_NT;
+    const long long pad = (long long)LU_PAD_STEPS * run;
     long long pbase = pad;
     for (size_t bi = 0; bi < blks.size(); bi++) {
         const Blk& b = blks[bi];
@@ -636,7 +814,7 @@ std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int 
         std::vector<long long> pofs((size_t)NJt * NKt);
         for (int K = 0; K < NKt; K++) for (int J = 0; J < NJt; J++) {
             pofs[J + NJt * K] = pbase;
-            pbase += (long long)((b.nx - 1) + size_j(J) + size_k(K) - 2) * NF * LU_NT;
+            pbase += (long long)((b.nx - 1) + size_j(J) + size_k(K) - 2) * run;
         }
         auto P = [&](int J, int K) { return pofs[J + NJt * K]; };
         // position of tile (J,K) in this block's list
@@ -648,6 +826,7 @@ std::vector<LuTask> lusgs_tasks(const std::vector<Blk>& blks, bool forward, int 
             t.pofs = P(J, K);
             int Ju = forward ? J - 1 : J + 1, Ku = forward ? K - 1 : K + 1;
             t.dep_j = t.dep_k = -1;
+            t.start = (forward ? J : NJt - 1 - J) * (TJ + LU_HOP) + (forward ? K : NKt - 1 - K) * (TK + LU_HOP);
             if (Ju >= 0 && Ju < NJt) {
                 t.dep_j = base + idx(Ju, K);
                 t.off_j = size_j(Ju) - 1;
@@ -692,23 +871,19 @@ static void sweep_nv(const LuPlan& L, const Par& p, bool forward, bool fenced, h
                            L.blks, L.bwd, L.prog_bwd, L.prog_fwd, L.n_fwd, L.err, p);
 }
 
-// this iteration's sweep inputs into sweep order: U, Res, Lc, Lv and the diagonal (one field, or
-// three for SA), and the sentinel into the DU elements the sweeps wait on
+// this iteration's sweep inputs into sweep order: U, Res, Lc, Lv and the diagonal, and the sentinel
+// into the DU elements the sweeps wait on
 template <int NV, int TJ>
 static void pack_nv(const LuPlan& L, const Par& p, hipStream_t st) {
-    using F = Pk<NV>;
-    constexpr int NAL = NV == 6 ? 3 : 1;
-    constexpr int FEND = F::AL + NAL;
-    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(FEND - F::U)),
-                       dim3(PK_T), 0, st, L.blks, L.fwd, L.pk, L.win, F::U, FEND, FEND);
+    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(PG_S - PG_NBR)), dim3(PK_T), 0, st, L.blks, L.fwd,
+                       L.pk, L.win, PG_NBR, p.gamma);
 }
 
 // the geometry the sweeps read (S, n), into sweep order once per plan
 template <int NV, int TJ>
 static void pack_geometry_nv(const LuPlan& L, const Par& p, hipStream_t st) {
-    using F = Pk<NV>;
-    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(F::NF - F::S)),
-                       dim3(PK_T), 0, st, L.blks, L.fwd, L.pk, L.win, F::S, F::NF, F::NF);
+    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(PG_END - PG_S)), dim3(PK_T), 0, st, L.blks, L.fwd,
+                       L.pk, L.win, PG_S, p.gamma);
 }
 
 // NVAR and the plan's tile width as template arguments
@@ -731,8 +906,7 @@ template <int NV, int TJ> struct PackK { static void run(const LuPlan& L, const 
 template <int NV, int TJ> struct GeoK { static void run(const LuPlan& L, const Par& p, hipStream_t st) { pack_geometry_nv<NV, TJ>(L, p, st); } };
 template <int NV, int TJ> struct DuBoxK {
     static void run(const LuPlan& L, hipStream_t st) {
-        hipLaunchKernelGGL((k_lu_du_to_box<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)NV), dim3(PK_T), 0, st,
-                           L.blks, L.fwd, L.pk, L.win);
+        hipLaunchKernelGGL((k_lu_du_to_box<NV, TJ>), dim3((unsigned)L.nwins), dim3(PK_T), 0, st, L.blks, L.fwd, L.pk, L.win);
     }
 };
 
@@ -742,12 +916,15 @@ void launch_lusgs_pipelined(const LuPlan& L, const Par& p, bool forward, bool fe
 
 bool lusgs_tile_ok(int tj) { return tj == 4 || tj == 8 || tj == 16; }
 
-int lusgs_fields(int NV) { return 4 * NV + 21; }
+int lusgs_run(int NV) { return NV == 5 ? Pk<5>::RUN : NV == 6 ? Pk<6>::RUN : Pk<7>::RUN; }
 std::vector<int2> lusgs_window_list(const std::vector<Blk>& blks, const std::vector<LuTask>& fwd) {
     std::vector<int2> out;
-    for (size_t t = 0; t < fwd.size(); t++) {
+    std::vector<int> at(fwd.size());
+    for (size_t q = 0; q < at.size(); q++) at[q] = (int)q;
+    std::sort(at.begin(), at.end(), [&](int a, int b) { return fwd[a].pofs < fwd[b].pofs; });
+    for (int t : at) {
         const int nxm = blks[fwd[t].blk].nx - 1;
-        for (int i0 = 1; i0 <= nxm; i0 += PK_W) out.push_back(make_int2((int)t, i0));
+        for (int i0 = 1; i0 <= nxm; i0 += PK_W) out.push_back(make_int2(t, i0));
     }
     return out;
 }

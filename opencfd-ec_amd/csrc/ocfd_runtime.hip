@@ -63,7 +63,7 @@ struct Engine {
     SetPlan set{};                            // batched-launch tables (built on first use)
     std::vector<void*> set_allocs;
     // plain mode: every kernel launched once per block, eagerly (no graphs), the LU-SGS sweeps on
-    // 8x8 tiles; parts[b] holds block b's own tables and shares this engine's stream
+    // 8x2 tiles; parts[b] holds block b's own tables and shares this engine's stream
     bool per_block = false;
     std::vector<Engine> parts;
     ocfd_batch* owner = nullptr;              // set for a batch's engine: its sweep storage is the batch's pool
@@ -457,8 +457,12 @@ int build_lu_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) {
     std::vector<Blk> blks;
     for (const BlockRef& r : refs) blks.push_back(r.hb->d);
     long long P = 0;
-    const int tj = e.lu_schedule == OCFD_LU_PIPELINED_FENCED ? 8 : e.lu_tj;
-    std::vector<LuTask> f = lusgs_tasks(blks, true, lusgs_fields(NV), tj, &P), b = lusgs_tasks(blks, false, lusgs_fields(NV), tj, nullptr);
+    // the fenced sweep works on 8x8 tiles of the block arrays and needs no sweep-ordered storage
+    const bool fenced = e.lu_schedule == OCFD_LU_PIPELINED_FENCED;
+    const int tj = fenced ? 8 : e.lu_tj, tk = fenced ? 8 : LU_COLS / tj, run = fenced ? 0 : lusgs_run(NV);
+    std::vector<LuTask> f = lusgs_tasks(blks, true, run, tj, tk, &P), b = lusgs_tasks(blks, false, run, tj, tk, nullptr);
+    lusgs_start_order(f);
+    lusgs_start_order(b);
     std::vector<int> minus(std::max(f.size(), b.size()), -1), zero{0, 0, e.lu_fail, 0};
     std::vector<int> mf(minus.begin(), minus.begin() + f.size()), mb(minus.begin(), minus.begin() + b.size());
     Blk* pb; LuTask *pf, *pw; int *qf, *qb, *pe;
@@ -470,6 +474,9 @@ int build_lu_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) {
     e.lu.blks = pb; e.lu.fwd = pf; e.lu.bwd = pw;
     e.lu.n_fwd = (int)f.size(); e.lu.n_bwd = (int)b.size();
     e.lu.prog_fwd = qf; e.lu.prog_bwd = qb; e.lu.err = pe;
+    e.lu.tj = tj;
+    e.lu_nv = NV;
+    if (fenced) return OCFD_OK;
     void* pk = nullptr;
     size_t bytes = (size_t)P * sizeof(double);
     HIPCHK(hipMalloc(&pk, bytes));
@@ -484,17 +491,15 @@ int build_lu_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) {
     if ((r = upload_table(e.lu_allocs, wins, &pwin))) return r;
     e.lu.win = pwin;
     e.lu.nwins = (int)wins.size();
-    e.lu.tj = tj;
     launch_lusgs_pack_geometry(e.lu, p0, e.st);
     launch_lusgs_reset(e.lu, NV, e.st);
-    e.lu_nv = NV;
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e.st));
     return OCFD_OK;
 }
 
 // ---- a batch's sweep storage pool ----
-// Regions are multiples of one step of a tile (NF x 64 elements), so a member's storage keeps the
+// Regions are multiples of one step of a tile (its run of doubles), so a member's storage keeps the
 // alignment of a context's own (the fields of an element follow from its offset).
 void pool_release(ocfd_batch* b, ocfd_ctx* c) {
     if (c->lu_tj == 0) return;
@@ -551,8 +556,8 @@ int pool_fill_member(ocfd_batch* b, ocfd_ctx* c, int tj, const Par& p0) {
     std::vector<Blk> blks;
     for (HostBlock& hb : c->blocks) blks.push_back(hb.d);
     long long P = 0;
-    std::vector<LuTask> f = lusgs_tasks(blks, true, lusgs_fields(NV), tj, &P);
-    const long long step = (long long)lusgs_fields(NV) * 64;
+    std::vector<LuTask> f = lusgs_tasks(blks, true, lusgs_run(NV), tj, LU_COLS / tj, &P);
+    const long long step = lusgs_run(NV);
     P = (P + step - 1) / step * step;
     long long off = 0;
     int r = pool_take(b, P, step, &off);
@@ -584,7 +589,7 @@ int pool_fill_member(ocfd_batch* b, ocfd_ctx* c, int tj, const Par& p0) {
 int build_lu_plan_batch(ocfd_batch* b, const Par& p0) {
     Engine& e = b->e;
     const int NV = p0.NV;
-    const int tj = e.lu_schedule == OCFD_LU_PIPELINED_FENCED ? 8 : e.lu_tj;
+    const int tj = e.lu_tj;
     int r;
     for (ocfd_ctx* c : b->members)
         if (c->lu_tj != 0 && c->lu_tj != tj) pool_release(b, c);
@@ -596,8 +601,8 @@ int build_lu_plan_batch(ocfd_batch* b, const Par& p0) {
         std::vector<Blk> mb;
         for (HostBlock& hb : c->blocks) mb.push_back(hb.d);
         const int bb = (int)blks.size(), tf = (int)f.size(), tw = (int)w.size();
-        std::vector<LuTask> mf = lusgs_tasks(mb, true, lusgs_fields(NV), tj, nullptr);
-        std::vector<LuTask> mw = lusgs_tasks(mb, false, lusgs_fields(NV), tj, nullptr);
+        std::vector<LuTask> mf = lusgs_tasks(mb, true, lusgs_run(NV), tj, LU_COLS / tj, nullptr);
+        std::vector<LuTask> mw = lusgs_tasks(mb, false, lusgs_run(NV), tj, LU_COLS / tj, nullptr);
         auto shift = [&](std::vector<LuTask>& v, int tb, std::vector<LuTask>& out) {
             for (LuTask t : v) {
                 t.blk += bb;
@@ -611,6 +616,8 @@ int build_lu_plan_batch(ocfd_batch* b, const Par& p0) {
         shift(mw, tw, w);
         for (const Blk& q : mb) blks.push_back(q);
     }
+    lusgs_start_order(f);
+    lusgs_start_order(w);
     std::vector<int> mf(f.size(), -1), mb(w.size(), -1), zero{0, 0, e.lu_fail, 0};
     Blk* pb; LuTask *pf, *pw; int *qf, *qb, *pe;
     if ((r = upload_table(e.lu_allocs, blks, &pb)) || (r = upload_table(e.lu_allocs, f, &pf)) ||
@@ -854,7 +861,7 @@ void drop_parts(Engine& e) {
 
 int engine_set_lu_tile(Engine& e, int tj) {
     if (!lusgs_tile_ok(tj)) return fail(OCFD_EARG, "LU-SGS tile width must be 4, 8 or 16");
-    if (e.per_block && tj != 8) return fail(OCFD_EARG, "the per-block launch mode keeps 8x8 tiles");
+    if (e.per_block && tj != 8) return fail(OCFD_EARG, "the per-block launch mode keeps 8x2 tiles");
     if (tj != e.lu_tj) { drop_graphs(e); drop_lu_plan(e); drop_parts(e); e.lu_tj = tj; }
     return OCFD_OK;
 }
@@ -867,13 +874,13 @@ int engine_set_lu_schedule(Engine& e, int schedule) {
     return OCFD_OK;
 }
 
-// The LU-SGS tile-shape autotuner: niter ordinary iterations with each tile shape (4x16, 8x8,
-// 16x4 (j,k) columns), timing the two sweeps of each with HIP events, then the fastest shape is
+// The LU-SGS tile-shape autotuner: niter ordinary iterations with each tile shape (4x4, 8x2,
+// 16x1 (j,k) columns), timing the two sweeps of each with HIP events, then the fastest shape is
 // kept.  Every shape gives the same result bit for bit, so the solve advances exactly as by
 // 3 niter plain iterations.
 int engine_autotune(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, int niter, int* best, double* ms3) {
     if (e.lu_schedule != OCFD_LU_PIPELINED) return fail(OCFD_EARG, "tile shapes apply to the pipelined LU-SGS schedule");
-    if (e.per_block) return fail(OCFD_EARG, "the per-block launch mode keeps 8x8 tiles");
+    if (e.per_block) return fail(OCFD_EARG, "the per-block launch mode keeps 8x2 tiles");
     if (niter < 1) return fail(OCFD_EARG, "niter < 1");
     static const int shapes[3] = {4, 8, 16};
     double t[3];

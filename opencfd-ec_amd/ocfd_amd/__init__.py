@@ -354,7 +354,7 @@ class Solver:
     def set_lu_fail_waits(self, on: bool): _check(lib().ocfd_set_lu_fail_waits(self._h, int(bool(on))))
 
     def set_per_block(self, on: bool):
-        """Plain launch mode: every kernel once per block, eagerly, 8x8 LU-SGS tiles."""
+        """Plain launch mode: every kernel once per block, eagerly, 8x2 LU-SGS tiles."""
         _check(lib().ocfd_set_per_block(self._h, int(bool(on))))
 
     def lu_tile(self) -> int:

@@ -107,15 +107,13 @@ class Server:
     @staticmethod
     def lu_bytes(case) -> int:
         """Device bytes of a request's share of the batch's tables: the LU-SGS sweep storage
-        (4 NVAR + 21 doubles per lane and step of every 64-column (j,k) tile, a tile marching
-        nx - 1 + tj + tk - 2 steps; the widest tile shape) and 16 MB for the launch tables."""
-        nv = C.nvar_of(case.params)
-        steps = 0
-        for b in case.blocks:
-            nx, ny, nz = b.dims
-            tiles = -(-(ny - 1) // 4) * -(-(nz - 1) // 16)
-            steps += max(tiles, -(-(ny - 1) // 16) * -(-(nz - 1) // 4)) * (nx - 1 + 18)
-        return int(steps * 64 * (4 * nv + 21) * 8 + 16e6)
+        (44, 51 or 54 doubles per column and step of every 16-column (j,k) tile for 5, 6 and 7
+        equations, a tile marching nx - 1 + tj + tk - 2 steps; the largest over the tile shapes) and
+        16 MB for the launch tables."""
+        words = {5: 44, 6: 51, 7: 54}[C.nvar_of(case.params)]
+        steps = max(sum(-(-(ny - 1) // tj) * -(-(nz - 1) // (16 // tj)) * (nx - 3 + tj + 16 // tj)
+                        for nx, ny, nz in (b.dims for b in case.blocks)) for tj in (4, 8, 16))
+        return int((steps + 48) * 16 * words * 8 + 16e6)
 
     @staticmethod
     def rms1(s) -> float:
