@@ -225,8 +225,8 @@ __global__ void __launch_bounds__(LU_NT) k_lusgs_sweep(const Blk* __restrict__ b
 // direction waves cost more than the arithmetic: 0.69 us per step with them, 0.36 without); and the
 // pressure and the reciprocals that do not depend on DU are formed once per cell by the pack.  A
 // step takes 0.42 us against 1.05 to 1.35 us with 64 columns per wave and all components per lane:
-// forward sweep of the 257x97x33 C-grid (SA) 528 -> 262 us, of the 97x33x9 channel 137 -> 85, of the
-// 24-block wing with 6.3 M cells 1085 -> 746.  A tile trails its upstream tile by about 3 us beyond
+// forward sweep of the 257x97x33 C-grid (SA) 528 -> 238 us, of the 97x33x9 channel 137 -> 78, of the
+// 24-block wing with 6.3 M cells 1085 -> 732.  A tile trails its upstream tile by about 2 us beyond
 // its own width, so long chains of narrow tiles lose (16x1 tiles), and a launch starts its tiles in
 // the order in which they can run (lusgs_start_order): block after block, the wing's sweep took
 // 1560 us instead of 1120 with the same kernel, most resident tiles waiting.
@@ -467,7 +467,7 @@ __device__ __forceinline__ void team_barrier() {
 // step q's piece of the tile's run (R to N forward, NBR to DUF backward) and, for the lanes at the
 // tile's upstream edges, the NBR (and backward SG) chunks that step q + 1 reads of the upstream
 // tiles.  du: the three direction waves' neighbour terms, double-buffered by step parity.
-constexpr int LU_RING = 6, LU_FAR = LU_RING - 1;      // slots, and how many steps ahead the loader writes
+constexpr int LU_RING = 4, LU_FAR = LU_RING - 1;      // slots, and how many steps ahead the loader writes
 template <int NV, bool FWD, int TJ> struct TeamLds {
     using F = Pk<NV>;
     static constexpr int BASE = FWD ? F::R : F::NBR;                 // first double of a run's piece
@@ -720,11 +720,12 @@ __device__ void team_sweep(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask&
     };
 
     // The loop is unrolled over the ring's slots.  The inputs of step q + 1 are read during step q,
-    // an upstream tile's DU is loaded LU_AHEAD steps before its use.  The last step of a round
+    // an upstream tile's DU is loaded LU_AHEAD steps before its use: every step more adds a step to
+    // the lag of each tile hop (257x97x33 C-grid, forward: 232, 263 and 292 us for 1, 2 and 3).  The last step of a round
     // checks whether a wave gave up (an LDS read after the barrier that the others skip): that wave
     // has set the error flag, so the waits of the steps in between give up within 256 polls and
     // their values are discarded, and all waves leave at the same barrier.
-    constexpr int LU_AHEAD = 2;
+    constexpr int LU_AHEAD = 1;
     static_assert(LU_RING % 2 == 0, "the step parity is fixed per unrolled step");
     TeamIn in[2];
     double Da[LU_RING], Db[LU_RING];

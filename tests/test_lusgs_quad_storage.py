@@ -14,7 +14,7 @@ import random
 
 import pytest
 
-COLS, PARTS, PK_W, PAD, RING, AHEAD = 16, 4, 32, 24, 6, 2
+COLS, PARTS, PK_W, PAD, RING, AHEAD = 16, 4, 32, 24, 4, 1
 FAR = RING - 1
 TILES = (4, 8, 16)
 SHAPES = [[(17, 17, 9)], [(33, 20, 13), (9, 5, 18)], [(65, 25, 9)], [(12, 40, 7), (20, 3, 3)], [(9, 65, 17)], [(3, 3, 3)]]
