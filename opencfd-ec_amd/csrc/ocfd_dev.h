@@ -26,7 +26,6 @@ struct Blk {
     double *dt, *mu, *muf, *mut;        // mu: Sutherland; muf: mu after the turbulence-model (x*Re)/Re round trip
     double *prim[7];                     // rho u v w p T c (per iteration; limiter snapshot afterwards)
     double *Lc[3], *Lv[3];
-    double *al[3];                       // du_LU_SGS's diagonal of the cell pass (one, or three for SA), for the sweeps
     double *vol, *S[3], *nv[9], *met[4][9], *dw, *dtm, *x, *y, *z, *xc, *yc, *zc;
     double *F[3][5];                     // inviscid face flux, m = 1..5
     double *Fv[3][4];                    // viscous face flux, m = 2..5

@@ -5,6 +5,7 @@
 
 #include "ocfd_dev.h"
 #include "ocfd_launch.h"
+#include "ocfd_pack.h"
 #include "ocfd_phys.h"
 
 namespace ocfd {
@@ -655,7 +656,7 @@ __device__ __forceinline__ void cell_assemble(const Blk& b, const Par& p, int i,
     }
 }
 
-// the cell pass in box order: Res, Lc, Lv and dt into the block arrays
+// the cell pass in box order, for the schedules that sweep the block arrays: Res, Lc, Lv and dt
 template <typename T>
 __global__ void __launch_bounds__(64) k_cell(BSet S) {
     OCFD_LOCATE(SP_CELL)
@@ -665,21 +666,92 @@ __global__ void __launch_bounds__(64) k_cell(BSet S) {
         b, p, i, j, k, s, [&](int m, double r) { b.Res[m][s] = r; },
         [&](int dir, double lc, double lv) { b.Lc[dir][s] = lc; b.Lv[dir][s] = lv; }, Lc, Lv, dt);
     b.dt[s] = dt;
-    // du_LU_SGS's diagonal (sub_LU_SGS.f90:27-37 forward, :81-90 backward): of components 1..5 (and
-    // 6, 7 of SST), and for SA of the SA component in the forward and in the backward sweep, which
-    // sum the viscous radii in different orders
-    const double vol = b.vol[s];
-    const double sumLc = (Lc[0] + Lc[1]) + Lc[2], sumLv = (Lv[0] + Lv[1]) + Lv[2];
-    double alfa = vol / dt + p.w_LU * sumLc;
-    if (p.visc == 1) alfa = alfa + 2.0 * sumLv;
-    b.al[0][s] = alfa + 0.0 * vol;
-    if (p.NV == 6) {
-        const double a1 = p.visc == 1 ? alfa + sumLv : alfa, a2 = p.visc == 1 ? ((alfa + Lv[0]) + Lv[1]) + Lv[2] : alfa;
-        b.al[1][s] = a1 + 0.0 * vol;
-        b.al[2][s] = a2 + 0.0 * vol;
-    }
 }
 
+// The cell pass of an iteration with the pipelined sweeps: one sweep tile's cells of an i-window
+// per workgroup, a thread per cell.  Res and dt go to the block arrays (for the host), and the
+// sweeps' inputs straight into sweep order, a group of fields at a time through one LDS buffer (35
+// KB for SA, so four workgroups share a CU): Res; du_LU_SGS's diagonal (sub_LU_SGS.f90:27-37
+// forward, :81-90 backward: of components 1..5, and 6, 7 of SST, and for SA of the SA component in
+// the forward and in the backward sweep, which sum the viscous radii in different orders) with its
+// reciprocals; the spectral radii; U with its pressure and reciprocal density.  The DU arrays get
+// the sentinel.  Bound by memory: against a cell pass in box order and a pack of its own, Lc, Lv
+// and the diagonal are not written and read back, nor Res read back (200 B per cell less), cell
+// pass and pack of the 24-block wing with 6.3 M cells 2020 -> 1750 us, of the 257x97x33 C-grid
+// 218 -> 203, of six serving solves 839 -> 759.  The register cap for six waves per SIMD makes it:
+// uncapped (130 VGPRs) one workgroup of eight waves fills a CU and the wing takes 2150 us, with four
+// waves 1780, with seven 1770.
+template <int NV, int TJ, typename T>
+__global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, const LuTask* __restrict__ tiles, double* __restrict__ pk,
+                                                  const int2* __restrict__ wins) {
+    using F = Pk<NV>;
+    __shared__ double buf[NV + 2][LU_COLS][PK_W + 2];
+    const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];     // (tile, i-window), windows fastest
+    const LuTask T_ = tiles[wn.x];
+    const Blk& b = S.blk[T_.blk];
+    const Par& p = S.par[T_.blk];
+    const int i0 = wn.y, W = min(PK_W, b.nx - i0);
+    const PackTile<NV, TJ> P{buf, T_, b, pk + T_.pofs + (long long)(i0 - 1) * F::RUN, i0, W};
+    P.sentinel();
+    const int x = (int)threadIdx.x % PK_W, c = (int)threadIdx.x / PK_W, jl = c % TJ, kl = c / TJ;
+    const int i = i0 + x, j = T_.j0 + jl, k = T_.k0 + kl;
+    const bool live = jl < T_.tj && kl < T_.tk && x < W;
+    const size_t s = IX(b, i, j, k);
+    double Lc[3], Lv[3], al[3] = {1.0, 1.0, 1.0};
+    if (live) {
+        double dt;
+        cell_assemble<T>(
+            b, p, i, j, k, s, [&](int m, double r) { b.Res[m][s] = r; buf[m][c][x] = r; }, [](int, double, double) {}, Lc, Lv, dt);
+        if constexpr (NV == 7) { buf[5][c][x] = b.Res[5][s]; buf[6][c][x] = b.Res[6][s]; }
+        b.dt[s] = dt;
+        const double vol = b.vol[s];
+        const double sumLc = (Lc[0] + Lc[1]) + Lc[2], sumLv = (Lv[0] + Lv[1]) + Lv[2];
+        double alfa = vol / dt + p.w_LU * sumLc;
+        if (p.visc == 1) alfa = alfa + 2.0 * sumLv;
+        al[0] = alfa + 0.0 * vol;
+        if (NV == 6) {
+            const double a1 = p.visc == 1 ? alfa + sumLv : alfa, a2 = p.visc == 1 ? ((alfa + Lv[0]) + Lv[1]) + Lv[2] : alfa;
+            al[1] = a1 + 0.0 * vol;
+            al[2] = a2 + 0.0 * vol;
+        }
+    }
+    __syncthreads();
+    P.template put<NV>([](int w, int& v, int& cc) { F::vec_at(w, v, cc); }, [](int w, int, int) { return F::R + w; });
+    __syncthreads();
+    if (live) {
+#pragma unroll
+        for (int m = 0; m < F::NAL; m++) { buf[2 * m][c][x] = al[m]; buf[2 * m + 1][c][x] = recip_nr(al[m]); }
+    }
+    __syncthreads();
+    P.template put<F::CA>([](int w, int& v, int& cc) { cc = w / F::CA; v = w % F::CA; }, [](int w, int, int) { return F::AL + w; });
+    __syncthreads();
+    if (live) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) { buf[d][c][x] = Lc[d]; buf[3 + d][c][x] = Lv[d]; }
+    }
+    __syncthreads();
+    P.template put<6>([](int w, int& v, int& cc) { cc = w / 6; v = w % 6; }, [](int, int v, int cc) { return F::NBR + cc * F::CS + F::LC + v; });
+    __syncthreads();
+    if (live) {
+        double u[NV];
+#pragma unroll
+        for (int m = 0; m < NV; m++) u[m] = b.U[m][s];
+        // comput_DFn's pressure of the undisturbed state, limit_vt's clamp
+        const double r = recip_nr(u[0]);
+        buf[NV][c][x] = (p.gamma - 1.0) * (u[4] - div_nr(0.5 * ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3]), u[0], r));
+        buf[NV + 1][c][x] = r;
+#pragma unroll
+        for (int m = 0; m < NV; m++) buf[m][c][x] = m > 4 && u[m] < 0.0 ? 0.0 : u[m];
+    }
+    __syncthreads();
+    P.template put<NV + 2>(
+        [](int w, int& v, int& cc) {
+            const int m = w % (NV + 2);
+            cc = w / (NV + 2);
+            v = m < 4 ? m + 1 : m == 4 ? 0 : m;
+        },
+        [](int w, int, int cc) { return F::NBR + cc * F::CS + w % (NV + 2); });
+}
 
 // ---------------------------------------------------------------------------------------------
 // du_LU_SGS (sub_LU_SGS.f90:4-129): cells of hyperplane i+j+k = plane, one thread per (j,k)
@@ -1447,6 +1519,28 @@ void set_viscous_dt(const SetPlan& P, hipStream_t st) {
     else viscous_dt_t<double>(P, st);
 }
 
+
+template <int NV, int TJ>
+static void cell_pk(const SetPlan& P, const LuPlan& L, hipStream_t st) {
+    if (L.nwins <= 0) return;
+    if (P.p0.mixed)
+        hipLaunchKernelGGL((k_cell_pk<NV, TJ, float>), dim3((unsigned)L.nwins), dim3(PK_T), 0, st, bset(P, SP_CELL), L.fwd, L.pk, L.win);
+    else
+        hipLaunchKernelGGL((k_cell_pk<NV, TJ, double>), dim3((unsigned)L.nwins), dim3(PK_T), 0, st, bset(P, SP_CELL), L.fwd, L.pk, L.win);
+}
+void set_viscous_dt_pack(const SetPlan& P, const LuPlan& L, hipStream_t st) {
+    switch (P.p0.NV * 100 + L.tj) {
+    case 504: cell_pk<5, 4>(P, L, st); break;
+    case 508: cell_pk<5, 8>(P, L, st); break;
+    case 516: cell_pk<5, 16>(P, L, st); break;
+    case 604: cell_pk<6, 4>(P, L, st); break;
+    case 608: cell_pk<6, 8>(P, L, st); break;
+    case 616: cell_pk<6, 16>(P, L, st); break;
+    case 704: cell_pk<7, 4>(P, L, st); break;
+    case 708: cell_pk<7, 8>(P, L, st); break;
+    default: cell_pk<7, 16>(P, L, st); break;
+    }
+}
 
 // limit_flow_U's replacement and limit_flow_SA after the update
 static void limit_after_update(const SetPlan& P, hipStream_t st) {

@@ -38,6 +38,8 @@ struct SetPlan {
 void set_pre(const SetPlan& P, hipStream_t st);
 void set_inviscid(const SetPlan& P, hipStream_t st);
 void set_viscous_dt(const SetPlan& P, hipStream_t st);
+// the same with the sweeps' inputs of the iteration written in sweep order
+void set_viscous_dt_pack(const SetPlan& P, const LuPlan& L, hipStream_t st);
 void set_update_limit(const SetPlan& P, hipStream_t st);
 // the update taking DU from the pipelined sweeps' storage
 void set_update_limit_sweep_order(const SetPlan& P, const LuPlan& L, hipStream_t st);
@@ -71,8 +73,6 @@ int lusgs_run(int NV);
 // (forward tile, first i) of every i-window of the tiles, tile after tile in storage order
 std::vector<int2> lusgs_window_list(const std::vector<Blk>& blks, const std::vector<LuTask>& fwd);
 void launch_lusgs_pack_geometry(const LuPlan& L, const Par& p, hipStream_t st);
-// the sweeps' per-iteration inputs (U, Res, Lc, Lv, the diagonal) into sweep order
-void launch_lusgs_pack(const LuPlan& L, const Par& p, hipStream_t st);
 void launch_lusgs_reset(const LuPlan& L, int NV, hipStream_t st);
 // the backward sweep's DU from the sweep-ordered storage into the block arrays (valid from the
 // end of the backward sweep until the next pack)

@@ -21,6 +21,7 @@
 
 #include "ocfd_dev.h"
 #include "ocfd_launch.h"
+#include "ocfd_pack.h"
 #include "ocfd_phys.h"
 
 namespace ocfd {
@@ -251,113 +252,32 @@ __device__ __forceinline__ double ld_coherent(const double* p) {
 }
 
 
-constexpr int PK_T = 256;
-
-// what a workgroup of the pack takes along: the neighbour data, Res, the diagonal, the sentinel
-// into DUF and DUB, and (once per plan) the areas and normals
-enum PackGroup { PG_NBR = 0, PG_R, PG_AL, PG_SENT_F, PG_SENT_B, PG_S, PG_N, PG_END };
-
-// box -> sweep order for one tile, one i-window of PK_W cells and one group of fields, through LDS
-// so both sides move in contiguous runs: NS fields are read (value src(v, s) at box index s), fin
-// completes a cell's column of the buffer, and the N fields are written: element w (of N LU_COLS)
-// of a step, field v of column c after at(w, v, c), goes to the run's element base + pos(w, v, c).  The LDS pitch of
-// PK_W + 2 keeps the skewed reads of a step's elements on different banks.
-template <int NV, int TJ, int NS, int N, typename Src, typename Fin, typename At, typename Pos>
-__device__ __forceinline__ void pack_group(double (*buf)[LU_COLS][PK_W + 2], const LuTask& T, const Blk& b, double* pk, int i0, int W,
-                                           int base, Src&& src, Fin&& fin, At&& at, Pos&& pos) {
-    constexpr int TK = LU_COLS / TJ;
-    const int t = (int)threadIdx.x, nsteps = b.nx - 1 + T.tj + T.tk - 2;
-    for (int e = t; e < NS * LU_COLS * PK_W; e += PK_T) {
-        const int x = e % PK_W, c = (e / PK_W) % LU_COLS, v = e / (PK_W * LU_COLS), jl = c % TJ, kl = c / TJ;
-        if (jl < T.tj && kl < T.tk && x < W) buf[v][c][x] = src(v, IX(b, i0 + x, T.j0 + jl, T.k0 + kl));
-    }
-    __syncthreads();
-    if constexpr (NS < N) {
-        for (int e = t; e < LU_COLS * PK_W; e += PK_T) fin(e / PK_W, e % PK_W);
-        __syncthreads();
-    }
-    for (int e = t; e < (W + TJ + TK - 2) * (N * LU_COLS); e += PK_T) {
-        const int q = i0 - 1 + e / (N * LU_COLS), w = e % (N * LU_COLS);
-        int v, c;
-        at(w, v, c);
-        const int jl = c % TJ, kl = c / TJ, x = q - jl - kl + 1 - i0;
-        if (jl < T.tj && kl < T.tk && x >= 0 && x < W && q < nsteps) pk[(size_t)T.pofs + (size_t)q * Pk<NV>::RUN + base + pos(w, v, c)] = buf[v][c][x];
-    }
-}
-
-// The pack of one group (grid z, from group g0 on).  Neighbouring i-windows of a tile share the
-// step runs at their boundary (each writes some columns of them), so a tile's windows run back to
-// back on one XCD, where the L2 merges those partial lines before they go to memory.  A DU group's
-// workgroup reads nothing and puts the sentinel into every element of its window's cells.
+// the geometry the sweeps read (S, n), into sweep order once per plan
 template <int NV, int TJ>
-__global__ void __launch_bounds__(PK_T) k_lu_transpose(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
-                                                       double* __restrict__ pk, const int2* __restrict__ wins, int g0, double gamma) {
+__global__ void __launch_bounds__(PK_T) k_lu_pack_geometry(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
+                                                           double* __restrict__ pk, const int2* __restrict__ wins) {
     using F = Pk<NV>;
-    __shared__ double buf[NV + 2][LU_COLS][PK_W + 2];
-    const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];     // (tile, i-window), windows fastest
+    __shared__ double buf[3][LU_COLS][PK_W + 2];
+    const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
     const LuTask T = tiles[wn.x];
     const Blk& b = blks[T.blk];
-    const int i0 = wn.y, W = min(PK_W, b.nx - 1 - i0 + 1);
-    const int g = g0 + (int)blockIdx.z;
-    auto none = [](int, int) {};
-    auto vec = [](int w, int& v, int& c) { F::vec_at(w, v, c); };
-    auto lin = [](int w, int, int) { return w; };
-    switch (g) {
-    case PG_NBR:
-        pack_group<NV, TJ, NV, NV + 2>(
-            buf, T, b, pk, i0, W, F::NBR, [&](int v, size_t s) { const double u = b.U[v][s]; return v > 4 && u < 0.0 ? 0.0 : u; },
-            [&](int c, int x) {
-                // comput_DFn's pressure of the undisturbed state
-                const double d = buf[0][c][x], m1 = buf[1][c][x], m2 = buf[2][c][x], m3 = buf[3][c][x], r = recip_nr(d);
-                buf[NV][c][x] = (gamma - 1.0) * (buf[4][c][x] - div_nr(0.5 * ((m1 * m1 + m2 * m2) + m3 * m3), d, r));
-                buf[NV + 1][c][x] = r;
-            },
-            [](int w, int& v, int& c) {
-                const int m = w % (NV + 2);
-                c = w / (NV + 2);
-                v = m < 4 ? m + 1 : m == 4 ? 0 : m;
-            },
-            [](int w, int, int c) { return c * F::CS + w % (NV + 2); });
-        __syncthreads();
-        pack_group<NV, TJ, 6, 6>(
-            buf, T, b, pk, i0, W, F::NBR, [&](int v, size_t s) { return v < 3 ? b.Lc[v][s] : b.Lv[v - 3][s]; }, none,
-            [](int w, int& v, int& c) { c = w / 6; v = w % 6; }, [](int, int v, int c) { return c * F::CS + F::LC + v; });
-        break;
-    case PG_R:
-        pack_group<NV, TJ, NV, NV>(buf, T, b, pk, i0, W, F::R, [&](int v, size_t s) { return b.Res[v][s]; }, none, vec, lin);
-        break;
-    case PG_AL:
-        pack_group<NV, TJ, F::NAL, 2 * F::NAL>(
-            buf, T, b, pk, i0, W, F::AL, [&](int v, size_t s) { return b.al[v][s]; },
-            [&](int c, int x) {
+    const PackTile<NV, TJ> P{buf, T, b, pk + T.pofs + (long long)(wn.y - 1) * F::RUN, wn.y, min(PK_W, b.nx - wn.y)};
+    auto third = [](int w, int& v, int& c) { c = w / 3; v = w % 3; };
+    P.template get<3>([&](size_t s, double* u) {
 #pragma unroll
-                for (int v = 0; v < F::NAL; v++) buf[F::NAL + v][c][x] = recip_nr(buf[v][c][x]);
-            },
-            [](int w, int& v, int& c) { const int m = w % F::CA; c = w / F::CA; v = (m & 1) * F::NAL + m / 2; }, lin);
-        break;
-    case PG_S:
-        pack_group<NV, TJ, 3, 3>(buf, T, b, pk, i0, W, F::SG, [&](int v, size_t s) { return b.S[v][s]; }, none,
-                                 [](int w, int& v, int& c) { c = w / 3; v = w % 3; }, [](int, int v, int c) { return 4 * c + v; });
-        break;
-    case PG_SENT_F:
-    case PG_SENT_B: {
-        constexpr int M = NV * LU_COLS;
-        const int nsteps = b.nx - 1 + T.tj + T.tk - 2, base = g == PG_SENT_F ? F::DUF : F::DUB;
-        for (int e = (int)threadIdx.x; e < (W + TJ + LU_COLS / TJ - 2) * M; e += PK_T) {
-            const int q = i0 - 1 + e / M, w = e % M;
-            int v, c;
-            F::vec_at(w, v, c);
-            const int x = q - c % TJ - c / TJ + 1 - i0;
-            if (x >= 0 && x < W && q < nsteps) pk[(size_t)T.pofs + (size_t)q * F::RUN + base + w] = sentinel_value();
-        }
-        break;
-    }
-    default:          // the normals, a direction at a time
-        for (int d = 0; d < 3; d++) {
-            if (d > 0) __syncthreads();
-            pack_group<NV, TJ, 3, 3>(buf, T, b, pk, i0, W, F::N, [&](int v, size_t s) { return b.nv[3 * d + v][s]; }, none,
-                                     [](int w, int& v, int& c) { c = w / 3; v = w % 3; }, [&](int, int v, int c) { return 9 * c + 3 * d + v; });
-        }
+        for (int d = 0; d < 3; d++) u[d] = b.S[d][s];
+    });
+    __syncthreads();
+    P.template put<3>(third, [](int, int v, int c) { return F::SG + 4 * c + v; });
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        __syncthreads();
+        P.template get<3>([&](size_t s, double* u) {
+#pragma unroll
+            for (int r = 0; r < 3; r++) u[r] = b.nv[3 * d + r][s];
+        });
+        __syncthreads();
+        P.template put<3>(third, [=](int, int v, int c) { return F::N + 9 * c + 3 * d + v; });
     }
 }
 
@@ -872,21 +792,6 @@ static void sweep_nv(const LuPlan& L, const Par& p, bool forward, bool fenced, h
                            L.blks, L.bwd, L.prog_bwd, L.prog_fwd, L.n_fwd, L.err, p);
 }
 
-// this iteration's sweep inputs into sweep order: U, Res, Lc, Lv and the diagonal, and the sentinel
-// into the DU elements the sweeps wait on
-template <int NV, int TJ>
-static void pack_nv(const LuPlan& L, const Par& p, hipStream_t st) {
-    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(PG_S - PG_NBR)), dim3(PK_T), 0, st, L.blks, L.fwd,
-                       L.pk, L.win, PG_NBR, p.gamma);
-}
-
-// the geometry the sweeps read (S, n), into sweep order once per plan
-template <int NV, int TJ>
-static void pack_geometry_nv(const LuPlan& L, const Par& p, hipStream_t st) {
-    hipLaunchKernelGGL((k_lu_transpose<NV, TJ>), dim3((unsigned)L.nwins, 1u, (unsigned)(PG_END - PG_S)), dim3(PK_T), 0, st, L.blks, L.fwd,
-                       L.pk, L.win, PG_S, p.gamma);
-}
-
 // NVAR and the plan's tile width as template arguments
 template <template <int, int> class K, typename... A>
 static void by_shape(int NV, int tj, A&&... a) {
@@ -903,8 +808,11 @@ static void by_shape(int NV, int tj, A&&... a) {
     }
 }
 template <int NV, int TJ> struct SweepK { static void run(const LuPlan& L, const Par& p, bool f, bool fe, hipStream_t st) { sweep_nv<NV, TJ>(L, p, f, fe, st); } };
-template <int NV, int TJ> struct PackK { static void run(const LuPlan& L, const Par& p, hipStream_t st) { pack_nv<NV, TJ>(L, p, st); } };
-template <int NV, int TJ> struct GeoK { static void run(const LuPlan& L, const Par& p, hipStream_t st) { pack_geometry_nv<NV, TJ>(L, p, st); } };
+template <int NV, int TJ> struct GeoK {
+    static void run(const LuPlan& L, hipStream_t st) {
+        hipLaunchKernelGGL((k_lu_pack_geometry<NV, TJ>), dim3((unsigned)L.nwins), dim3(PK_T), 0, st, L.blks, L.fwd, L.pk, L.win);
+    }
+};
 template <int NV, int TJ> struct DuBoxK {
     static void run(const LuPlan& L, hipStream_t st) {
         hipLaunchKernelGGL((k_lu_du_to_box<NV, TJ>), dim3((unsigned)L.nwins), dim3(PK_T), 0, st, L.blks, L.fwd, L.pk, L.win);
@@ -938,10 +846,7 @@ static void reset_nv(const LuPlan& L, hipStream_t st) {
 }
 
 void launch_lusgs_pack_geometry(const LuPlan& L, const Par& p, hipStream_t st) {
-    if (L.nwins > 0) by_shape<GeoK>(p.NV, L.tj, L, p, st);
-}
-void launch_lusgs_pack(const LuPlan& L, const Par& p, hipStream_t st) {
-    if (L.nwins > 0) by_shape<PackK>(p.NV, L.tj, L, p, st);
+    if (L.nwins > 0) by_shape<GeoK>(p.NV, L.tj, L, st);
 }
 void launch_lusgs_du_to_box(const LuPlan& L, int NV, hipStream_t st) {
     if (L.nwins > 0) by_shape<DuBoxK>(NV, L.tj, L, st);

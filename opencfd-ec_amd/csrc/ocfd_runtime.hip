@@ -159,7 +159,6 @@ int carve_block(ocfd_ctx* c, HostBlock& hb) {
     for (double** q : one) if ((r = dalloc(hb, q, n))) return r;
     for (int q = 0; q < 7; q++) if ((r = dalloc(hb, &b.prim[q], n))) return r;
     for (int q = 0; q < 3; q++) if ((r = dalloc(hb, &b.Lc[q], n)) || (r = dalloc(hb, &b.Lv[q], n)) || (r = dalloc(hb, &b.S[q], n))) return r;
-    for (int q = 0; q < (NV == 6 ? 3 : 1); q++) if ((r = dalloc(hb, &b.al[q], n))) return r;
     for (int q = 0; q < 9; q++) if ((r = dalloc(hb, &b.nv[q], n))) return r;
     for (int s = 1; s < 4; s++) for (int q = 0; q < 9; q++) if ((r = dalloc(hb, &b.met[s][q], n))) return r;
     if (turb) {
@@ -352,9 +351,9 @@ void enqueue_stage(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, 
         set_inviscid(P, e.st);
         break;
     case OCFD_STAGE_VISCOUS_DT:
-        set_viscous_dt(P, e.st);
         // the pipelined sweeps read their inputs in sweep order
-        if (e.lu_schedule == OCFD_LU_PIPELINED && e.lu.fwd) launch_lusgs_pack(e.lu, p0, e.st);
+        if (e.lu_schedule == OCFD_LU_PIPELINED && e.lu.fwd) set_viscous_dt_pack(P, e.lu, e.st);
+        else set_viscous_dt(P, e.st);
         break;
     case OCFD_STAGE_LU_FORWARD:
     case OCFD_STAGE_LU_BACKWARD:
