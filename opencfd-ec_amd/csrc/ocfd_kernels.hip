@@ -13,25 +13,72 @@ namespace ocfd {
 #define GRID1(n, bs) dim3((unsigned)(((n) + (bs) - 1) / (bs))), dim3(bs)
 
 // ---------------------------------------------------------------------------------------------
-// get_viscous's Sutherland viscosity of temperature T (sub_Residual.f90:1355-1383); muf keeps the
-// value left after the turbulence model's mu*Re ... mu/Re round trip (sub_turbulence_SA.f90:41,262)
-__device__ __forceinline__ void visc_cell(const Blk& b, const Par& p, size_t s, double T) {
+// get_viscous's Sutherland viscosity of temperature T (sub_Residual.f90:1355-1383)
+__device__ __forceinline__ double visc_of(const Par& p, double T) {
     double Tsb = 110.4 / p.T_inf;
-    double mu = ((1.0 / p.Re) * (1.0 + Tsb)) * sqrt((T * T) * T) / (Tsb + T);
+    return ((1.0 / p.Re) * (1.0 + Tsb)) * sqrt((T * T) * T) / (Tsb + T);
+}
+// muf keeps the value left after the turbulence model's mu*Re ... mu/Re round trip
+// (sub_turbulence_SA.f90:41,262)
+__device__ __forceinline__ void put_visc(const Blk& b, const Par& p, size_t s, double mu) {
     b.mu[s] = mu;
     b.muf[s] = (p.turb == 2 || p.turb == 3) ? (mu * p.Re) / p.Re : mu;
 }
+__device__ __forceinline__ double pw3(double x) { return (x * x) * x; }
+// mu_t of SA from viscosity, density and U6 (clamped by limit_vt) with both limit_mut passes
+// (sub_Residual.f90:1387-1408) folded in
+__device__ __forceinline__ double sa_mut(const Par& p, double mu, double d, double U6) {
+    const double Cv1_3 = pw3(7.1);
+    double mu_sa = mu * p.Re;
+    double vt = U6 < 0.0 ? 0.0 : U6;
+    double X = d * vt / mu_sa;
+    double fv1 = pw3(X) / (pw3(X) + Cv1_3);
+    double m1 = (fv1 * d) * vt;
+    if (m1 < 0.0) m1 = 0.0;
+    if (p.MUT_MAX >= 0.0 && m1 > p.MUT_MAX * mu_sa) m1 = p.MUT_MAX * mu_sa;
+    double m2 = m1 / p.Re;
+    double muf = (mu * p.Re) / p.Re;
+    if (m2 < 0.0) m2 = 0.0;
+    if (p.MUT_MAX >= 0.0 && m2 > p.MUT_MAX * muf) m2 = p.MUT_MAX * muf;
+    return m2;
+}
 
-// comput_duvtpc (sub_Residual.f90:1417-1456): primitives on the whole LAP box; for a viscous case
-// also get_viscous on the interior cells, from T in registers
+// density, velocity and temperature of cell s (comput_duvtpc)
+__device__ __forceinline__ void prims_of(const Blk& b, const Par& p, size_t s, double& d, double& u, double& v, double& w, double& T) {
+    d = b.U[0][s];
+    const double rd = recip_nr(d);
+    u = div_nr(b.U[1][s], d, rd); v = div_nr(b.U[2][s], d, rd); w = div_nr(b.U[3][s], d, rd);
+    T = (b.U[4][s] - (0.5 * d) * ((u * u + v * v) + w * w)) / (p.Cv * d);
+}
+
+// whether the ghost cell (i,j,k), ghost in one direction only (one index 0 or n, the others inside),
+// lies beyond a wall; sn is the index of the cell it borders.  False for every other cell (sn = s)
+__device__ __forceinline__ bool face_ghost(const Blk& b, int i, int j, int k, size_t s, size_t& sn, bool& wall) {
+    const bool ii = i >= 1 && i <= b.nx - 1, jj = j >= 1 && j <= b.ny - 1, kk = k >= 1 && k <= b.nz - 1;
+    const bool gi = i == 0 || i == b.nx, gj = j == 0 || j == b.ny, gk = k == 0 || k == b.nz;
+    sn = s;
+    wall = false;
+    if (gi && jj && kk) { sn = IX(b, i == 0 ? 1 : b.nx - 1, j, k); wall = b.bcf[0][JK(b, j, k)] & (i == 0 ? BCF_WALL : BCF_WALL << 1); }
+    else if (ii && gj && kk) { sn = IX(b, i, j == 0 ? 1 : b.ny - 1, k); wall = b.bcf[1][IK(b, i, k)] & (j == 0 ? BCF_WALL : BCF_WALL << 1); }
+    else if (ii && jj && gk) { sn = IX(b, i, j, k == 0 ? 1 : b.nz - 1); wall = b.bcf[2][IJ(b, i, j)] & (k == 0 ? BCF_WALL : BCF_WALL << 1); }
+    else return false;
+    return true;
+}
+
+// comput_duvtpc (sub_Residual.f90:1417-1456): primitives on the whole LAP box.  For a viscous case
+// also get_viscous on the cells, its copy into the first ghost layer, and for SA mu_t over 0..n
+// with Amut_boundary's sign change beyond walls (sub_turbulence_SA.f90:36-48,282-368): a ghost
+// cell's thread takes its neighbour's T from U, so no pass of its own reads them back
+// (with the passes merged, the kernels before the faces take 17 instead of 26 us on a 65x25x9 SA
+// grid and 44 instead of 55 us on 257x97x33; HBM bound on large ones).  The first thread of a block clears its limiter counters, the launch's first thread the set's.
 __global__ void __launch_bounds__(64) k_prims(BSet S) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *S.limited = 0;
     OCFD_LOCATE(SP_BOX)
     size_t s = IX(b, i, j, k);
+    if (i == -3 && j == -3 && k == -3) { b.flags[1] = 0; b.flags[2] = 0; }
     double p00 = 1.0 / (p.gamma * p.Ma * p.Ma);
-    double d = b.U[0][s];
-    const double rd = recip_nr(d);
-    double u = div_nr(b.U[1][s], d, rd), v = div_nr(b.U[2][s], d, rd), w = div_nr(b.U[3][s], d, rd);
-    double T = (b.U[4][s] - (0.5 * d) * ((u * u + v * v) + w * w)) / (p.Cv * d);
+    double d, u, v, w, T;
+    prims_of(b, p, s, d, u, v, w, T);
     b.prim[0][s] = d; b.prim[1][s] = u; b.prim[2][s] = v; b.prim[3][s] = w;
     b.prim[4][s] = (p00 * d) * T; b.prim[5][s] = T; b.prim[6][s] = sqrt(T) / p.Ma;
     if (p.turb == 3) {
@@ -44,30 +91,26 @@ __global__ void __launch_bounds__(64) k_prims(BSet S) {
         b.primf[0][s] = (float)d; b.primf[1][s] = (float)u; b.primf[2][s] = (float)v; b.primf[3][s] = (float)w;
         b.primf[4][s] = (float)((p00 * d) * T); b.primf[5][s] = (float)T;
     }
-    if (p.visc == 1 && i >= 1 && i <= b.nx - 1 && j >= 1 && j <= b.ny - 1 && k >= 1 && k <= b.nz - 1) visc_cell(b, p, s, T);
-}
-
-// mu and muf of the first cells of each face copied into its first ghost layer; one task per block
-// and face, tiles of 64 cells along the face's first tangential direction
-__global__ void __launch_bounds__(64) k_visc_ghost(SubSet S) {
-    OCFD_SUB_LOCATE
-    (void)p; (void)B;
-    if (a >= T_.n0) return;
-    const int f = T_.arg, u = a + 1, v = c + 1;
-    const int nx = b.nx, ny = b.ny, nz = b.nz;
-    size_t d, s;
-    if (f < 2) { d = IX(b, f == 0 ? 0 : nx, u, v); s = IX(b, f == 0 ? 1 : nx - 1, u, v); }
-    else if (f < 4) { d = IX(b, u, f == 2 ? 0 : ny, v); s = IX(b, u, f == 2 ? 1 : ny - 1, v); }
-    else { d = IX(b, u, v, f == 4 ? 0 : nz); s = IX(b, u, v, f == 4 ? 1 : nz - 1); }
-    b.mu[d] = b.mu[s];
-    b.muf[d] = b.muf[s];
+    if (p.visc != 1 || i < 0 || i > b.nx || j < 0 || j > b.ny || k < 0 || k > b.nz) return;
+    const bool cell = i >= 1 && i <= b.nx - 1 && j >= 1 && j <= b.ny - 1 && k >= 1 && k <= b.nz - 1;
+    size_t sn = s;
+    bool wall = false;
+    double dn = d, mu;
+    if (cell) { mu = visc_of(p, T); put_visc(b, p, s, mu); }
+    else if (face_ghost(b, i, j, k, s, sn, wall)) {
+        double un, vn, wn, Tn;
+        prims_of(b, p, sn, dn, un, vn, wn, Tn);
+        mu = visc_of(p, Tn);
+        put_visc(b, p, s, mu);
+    } else mu = b.mu[s];        // edges and corners keep the initial value
+    if (p.turb == 2) b.mut[s] = !cell && wall ? -sa_mut(p, mu, dn, b.U[5][sn]) : sa_mut(p, mu, d, b.U[5][s]);
+    else if (p.turb != 3 && !cell && wall) b.mut[s] = -b.mut[sn];
 }
 
 // ---------------------------------------------------------------------------------------------
 // Spalart-Allmaras (sub_turbulence_SA.f90:8-273).  U6 is read through limit_vt's clamp
 // (sub_time_advance.f90:420-428): negative values act as zero.
 __device__ __forceinline__ double vt_of(const Blk& b, size_t s) { double v = b.U[5][s]; return v < 0.0 ? 0.0 : v; }
-__device__ __forceinline__ double pw3(double x) { return (x * x) * x; }
 __device__ __forceinline__ double pw6(double x) { return ((((x * x) * x) * x) * x) * x; }   // flang expansion order
 
 // Storage of the compute type T of the residual: FP64 (the drop-in) or FP32 (the mixed mode's
@@ -100,25 +143,6 @@ template <typename T> __device__ __forceinline__ double get_Fv(const Blk& b, int
 }
 template <typename T> __device__ __forceinline__ double get_Fsa(const Blk& b, int d, int m, size_t s) {
     if constexpr (sizeof(T) == 8) return b.Fsa[d][m][s]; else return (double)b.Fsaf[d][m][s];
-}
-
-// mu_t over 0..n with both limit_mut passes (sub_Residual.f90:1387-1408) folded in
-__global__ void __launch_bounds__(64) k_sa_mut(BSet S) {
-    OCFD_LOCATE(SP_N0)
-    size_t s = IX(b, i, j, k);
-    const double Cv1_3 = pw3(7.1);
-    double mu_sa = b.mu[s] * p.Re;
-    double d = b.prim[0][s], vt = vt_of(b, s);
-    double X = d * vt / mu_sa;
-    double fv1 = pw3(X) / (pw3(X) + Cv1_3);
-    double m1 = (fv1 * d) * vt;
-    if (m1 < 0.0) m1 = 0.0;
-    if (p.MUT_MAX >= 0.0 && m1 > p.MUT_MAX * mu_sa) m1 = p.MUT_MAX * mu_sa;
-    double m2 = m1 / p.Re;
-    double muf = (b.mu[s] * p.Re) / p.Re;
-    if (m2 < 0.0) m2 = 0.0;
-    if (p.MUT_MAX >= 0.0 && m2 > p.MUT_MAX * muf) m2 = p.MUT_MAX * muf;
-    b.mut[s] = m2;
 }
 
 // SA constants (sub_turbulence_SA.f90:18-33)
@@ -228,6 +252,13 @@ __device__ __forceinline__ void d_amut(const Blk& b, const Sub& B, int a, int c)
         int kg = B.face == 3 ? 0 : B.ke, kk = B.face == 3 ? 1 : B.ke - 1; b.mut[IX(b, i, j, kg)] = -b.mut[IX(b, i, j, kk)]; break; }
     }
 }
+// Wall subfaces that do not lie on their block's face; the others' ghost cells are set by the kernels
+// that form mu_t
+__global__ void __launch_bounds__(64) k_amut(SubSet S) {
+    OCFD_SUB_LOCATE
+    (void)p;
+    d_amut(b, B, a, c);
+}
 
 // ---------------------------------------------------------------------------------------------
 // Menter SST (sub_turbulence_SST.f90:7-348).  f1 on the last face of each direction reads the
@@ -283,19 +314,30 @@ __global__ void __launch_bounds__(64) k_sst_cell(BSet S) {
     T vol = T(b.vol[s]);
     b.Res[5][s] = (double)(Qk * vol);
     b.Res[6][s] = (double)(Qw * vol);
-    b.mut[s] = (double)mutc;      // Re-scaled value, divided by Re in k_sst_finish
+    b.mut[s] = (double)mutc;      // Re-scaled value, divided by Re in k_sst_res
     b.aux[s] = (double)f1;
 }
 
-// mu_t ghost copies over the whole -1:n+1 extent (sub_turbulence_SST.f90:170-175): face f in
-// order i-, i+, j-, j+, k-, k+ launched one after the other
-__global__ void k_sst_ghost(BSet S, int f) {
-    const Blk& b = S.blk[blockIdx.z];
-    int a = blockIdx.x * blockDim.x + threadIdx.x - 1, c = blockIdx.y - 1;
-    int nx = b.nx, ny = b.ny, nz = b.nz;
-    if (f < 2) { if (a > ny + 1 || c > nz + 1) return; b.mut[IX(b, f == 0 ? 0 : nx, a, c)] = b.mut[IX(b, f == 0 ? 1 : nx - 1, a, c)]; }
-    else if (f < 4) { if (a > nx + 1 || c > nz + 1) return; b.mut[IX(b, a, f == 2 ? 0 : ny, c)] = b.mut[IX(b, a, f == 2 ? 1 : ny - 1, c)]; }
-    else { if (a > nx + 1 || c > ny + 1) return; b.mut[IX(b, a, c, f == 4 ? 0 : nz)] = b.mut[IX(b, a, c, f == 4 ? 1 : nz - 1)]; }
+// mu_t of the first ghost layer (sub_turbulence_SST.f90:170-175): the reference copies face after
+// face in the order i-, i+, j-, j+, k-, k+, which leaves every ghost cell of 0..n with the value of
+// the cell that each of its ghost indices moved inside gives; Amut_boundary's sign change beyond
+// walls follows.  One task per block and face, over the face's cells with their ghost rows.
+__global__ void __launch_bounds__(64) k_sst_ghost(SubSet S) {
+    OCFD_SUB_LOCATE
+    (void)p; (void)B;
+    if (a >= T_.n0) return;
+    const int f = T_.arg, nx = b.nx, ny = b.ny, nz = b.nz;
+    int i, j, k;
+    if (f < 2) { i = f == 0 ? 0 : nx; j = a; k = c; }
+    else if (f < 4) { i = a; j = f == 2 ? 0 : ny; k = c; }
+    else { i = a; j = c; k = f == 4 ? 0 : nz; }
+    const int ci = min(max(i, 1), nx - 1), cj = min(max(j, 1), ny - 1), ck = min(max(k, 1), nz - 1);
+    const size_t s = IX(b, i, j, k);
+    size_t sn;
+    bool wall;
+    face_ghost(b, i, j, k, s, sn, wall);
+    const double m = b.mut[IX(b, ci, cj, ck)];
+    b.mut[s] = wall ? -m : m;
 }
 
 // k and omega flux through face (i,j,k) of direction DIR, between cells (i,j,k) - e_DIR and
@@ -303,8 +345,7 @@ __global__ void k_sst_ghost(BSet S, int f) {
 // omega; one thread per face, each face evaluated once for both of its cells; compute type T,
 // stored in FP64
 template <int DIR, typename T>
-__global__ void __launch_bounds__(64) k_sst_face(BSet S) {
-    OCFD_LOCATE(SP_FI + DIR)
+__device__ __forceinline__ void sst_face(const Blk& b, const Par& p, int i, int j, int k) {
     const T sigma_k1 = T(0.85), sigma_w1 = T(0.5), sigma_k2 = T(1.0), sigma_w2 = T(0.856);
     const T Re = T(p.Re);
     const T *uu = prim_of<T>(b, 1), *vv = prim_of<T>(b, 2), *ww = prim_of<T>(b, 3);
@@ -354,31 +395,43 @@ __global__ void __launch_bounds__(64) k_sst_face(BSet S) {
     b.Fsa[DIR][0][f] = (double)((-kfi + muk * ((ktx * s1x + kty * s1y) + ktz * s1z)) * Sf);
     b.Fsa[DIR][1][f] = (double)((-wfi + muw * ((wtx * s1x + wty * s1y) + wtz * s1z)) * Sf);
 }
-
-// the face fluxes accumulated into Res(6:7) per direction in i, j, k order
-__global__ void __launch_bounds__(64) k_sst_res(BSet S) {
-    OCFD_LOCATE(SP_CELL)
-    size_t s = IX(b, i, j, k);
-    const size_t sp[3] = {s + 1, s + (size_t)b.NI, s + (size_t)b.NI * b.NJ};
-    double r6 = b.Res[5][s], r7 = b.Res[6][s];
-#pragma unroll
-    for (int dir = 0; dir < 3; dir++) {
-        r6 = (r6 + b.Fsa[dir][0][sp[dir]]) - b.Fsa[dir][0][s];
-        r7 = (r7 + b.Fsa[dir][1][sp[dir]]) - b.Fsa[dir][1][s];
+// the three directions in one launch
+template <typename T>
+__global__ void __launch_bounds__(64) k_sst_face(FaceSet S) {
+    int bi, i, j, k;
+    switch (locate_face(S, bi, i, j, k)) {
+    case 0: sst_face<0, T>(S.blk[bi], S.par[bi], i, j, k); break;
+    case 1: sst_face<1, T>(S.blk[bi], S.par[bi], i, j, k); break;
+    case 2: sst_face<2, T>(S.blk[bi], S.par[bi], i, j, k); break;
     }
-    b.Res[5][s] = r6;
-    b.Res[6][s] = r7;
 }
 
-// mu_t/Re and the limit_mut pass of Residual (sub_turbulence_SST.f90:333-340; sub_Residual.f90:1387-1408)
-__global__ void __launch_bounds__(64) k_sst_finish(BSet S) {
+// The face fluxes accumulated into Res(6:7) per direction in i, j, k order, and over 0..n mu_t/Re
+// with the limit_mut pass of Residual (sub_turbulence_SST.f90:333-340; sub_Residual.f90:1387-1408)
+// and Amut_boundary again: a ghost cell beyond a wall holds minus its neighbour's mu_t and the
+// neighbour's mu, so its thread forms the neighbour's final value from them.
+__global__ void __launch_bounds__(64) k_sst_res(BSet S) {
     OCFD_LOCATE(SP_N0)
     size_t s = IX(b, i, j, k);
-    double m2 = b.mut[s] / p.Re;
+    if (i >= 1 && i <= b.nx - 1 && j >= 1 && j <= b.ny - 1 && k >= 1 && k <= b.nz - 1) {
+        const size_t sp[3] = {s + 1, s + (size_t)b.NI, s + (size_t)b.NI * b.NJ};
+        double r6 = b.Res[5][s], r7 = b.Res[6][s];
+#pragma unroll
+        for (int dir = 0; dir < 3; dir++) {
+            r6 = (r6 + b.Fsa[dir][0][sp[dir]]) - b.Fsa[dir][0][s];
+            r7 = (r7 + b.Fsa[dir][1][sp[dir]]) - b.Fsa[dir][1][s];
+        }
+        b.Res[5][s] = r6;
+        b.Res[6][s] = r7;
+    }
+    size_t sn;
+    bool wall;
+    face_ghost(b, i, j, k, s, sn, wall);
+    double m2 = (wall ? -b.mut[s] : b.mut[s]) / p.Re;
     double muf = (b.mu[s] * p.Re) / p.Re;
     if (m2 < 0.0) m2 = 0.0;
     if (p.MUT_MAX >= 0.0 && m2 > p.MUT_MAX * muf) m2 = p.MUT_MAX * muf;
-    b.mut[s] = m2;
+    b.mut[s] = wall ? -m2 : m2;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -402,8 +455,8 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int 
     int nd = DIR == 0 ? b.nx : DIR == 1 ? b.ny : b.nz;
     int scheme = p.scheme;
     uint8_t fl = DIR == 0 ? b.bcf[0][JK(b, j, k)] : DIR == 1 ? b.bcf[1][IK(b, i, k)] : b.bcf[2][IJ(b, i, j)];
-    if (fl & 1) { if (pos == 1) scheme = S_CD2; else if (pos < LAP) scheme = p.bscheme; }
-    if (fl & 2) { if (pos == nd) scheme = S_CD2; else if (pos > nd - LAP + 1) scheme = p.bscheme; }
+    if (fl & BCF_PHYS) { if (pos == 1) scheme = S_CD2; else if (pos < LAP) scheme = p.bscheme; }
+    if (fl & BCF_PHYS << 1) { if (pos == nd) scheme = S_CD2; else if (pos > nd - LAP + 1) scheme = p.bscheme; }
     if (b.flags[0] == 1) scheme = S_UD1;
     T s1x = nv_of<T>(b, 3 * DIR)[s], s1y = nv_of<T>(b, 3 * DIR + 1)[s], s1z = nv_of<T>(b, 3 * DIR + 2)[s];
     T t1x, t1y, t1z;
@@ -490,12 +543,9 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int 
     put_F(b, DIR, 4, s, -F0[4] * Sf);
 }
 
-// explicit average-state flux on a physical k subface (sub_Residual.f90:667-688)
+// explicit average-state flux on a physical k face (sub_Residual.f90:667-688)
 template <typename T>
-__global__ void __launch_bounds__(64) k_inv_kbc(SubSet S) {
-    OCFD_SUB_LOCATE
-    int i = B.ib + a, j = B.jb + c, k = B.kb;
-    if (i > B.ie - 1 || j > B.je - 1) return;
+__device__ __forceinline__ void inv_kbc(const Blk& b, const Par& p, int i, int j, int k) {
     size_t s = IX(b, i, j, k), t = IX(b, i, j, k - 1);
     double g = p.gamma;
     double d0 = (b.prim[0][s] + b.prim[0][t]) * 0.5, uu0 = (b.prim[1][s] + b.prim[1][t]) * 0.5, v0 = (b.prim[2][s] + b.prim[2][t]) * 0.5;
@@ -509,6 +559,15 @@ __global__ void __launch_bounds__(64) k_inv_kbc(SubSet S) {
     put_F(b, 2, 2, s, T(-((d0 * un) * v0 + p0 * n2) * Sk));
     put_F(b, 2, 3, s, T(-((d0 * un) * w0 + p0 * n3) * Sk));
     put_F(b, 2, 4, s, T(-((E0 + p0) * un) * Sk));
+}
+
+// k subfaces inside a block, after the faces
+template <typename T>
+__global__ void __launch_bounds__(64) k_inv_kbc(SubSet S) {
+    OCFD_SUB_LOCATE
+    int i = B.ib + a, j = B.jb + c;
+    if (i > B.ie - 1 || j > B.je - 1) return;
+    inv_kbc<T>(b, p, i, j, B.kb);
 }
 
 // flux_viscous_i/j/k (sub_Residual.f90:712-1247) of face (i,j,k) of direction DIR, stored
@@ -596,8 +655,7 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int
 // viscous flux, mostly loads of the face's gradient stencil and metrics, overlaps the inviscid
 // flux's arithmetic in the same kernel.
 template <int DIR, typename T, int RECON, int FLUX>
-__global__ void __launch_bounds__(64) k_face(BSet S) {
-    OCFD_LOCATE(SP_FI + DIR)
+__device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, int k) {
     if (p.turb == 2) {
         const size_t s = IX(b, i, j, k);
         T fv, f2;
@@ -605,8 +663,24 @@ __global__ void __launch_bounds__(64) k_face(BSet S) {
         put_Fsa(b, DIR, 0, s, fv);
         put_Fsa(b, DIR, 1, s, f2);
     }
-    inv_face<DIR, T, RECON, FLUX>(b, p, i, j, k);
+    if (DIR == 2 && ((k == 1 && (b.bcf[2][IJ(b, i, j)] & BCF_KBC)) || (k == b.nz && (b.bcf[2][IJ(b, i, j)] & BCF_KBC << 1))))
+        inv_kbc<T>(b, p, i, j, k);
+    else inv_face<DIR, T, RECON, FLUX>(b, p, i, j, k);
     if (p.visc == 1) visc_face<DIR, T>(b, p, i, j, k);
+}
+// The three directions' faces in one launch.  On small grids, where a direction's tiles do not fill
+// the GPU and a launch costs more than its work, they run side by side (97x33x9 without viscosity:
+// 22 us instead of 37 in three launches; 257x97x33 SA: 271 against 306); on large ones the
+// directions share the primitives in L2 (face_tile; a batch of 6 with 1.9 M cells: 835 against
+// 930 us, 24 blocks with 6.3 M cells: 2090 against 2200).
+template <typename T, int RECON, int FLUX>
+__global__ void __launch_bounds__(64) k_face(FaceSet S) {
+    int bi, i, j, k;
+    switch (locate_face(S, bi, i, j, k)) {
+    case 0: face<0, T, RECON, FLUX>(S.blk[bi], S.par[bi], i, j, k); break;
+    case 1: face<1, T, RECON, FLUX>(S.blk[bi], S.par[bi], i, j, k); break;
+    case 2: face<2, T, RECON, FLUX>(S.blk[bi], S.par[bi], i, j, k); break;
+    }
 }
 
 // Res(1:5): inviscid i, j, k then viscous i, j, k face differences, in the reference order
@@ -846,18 +920,19 @@ __device__ __forceinline__ bool lim_out(const Par& p, double d1, double u1, doub
     return d1 < p.Ldmin || p1 < p.Lpmin || d1 > p.Ldmax || p1 > p.Lpmax || fabs(u1) > p.Lumax || fabs(v1) > p.Lumax || fabs(w1) > p.Lumax;
 }
 
-__device__ __forceinline__ void update_cell(const Blk& b, const Par& p, int i, int j, int k, size_t s, const double* DU) {
+__device__ __forceinline__ void update_cell(const BSet& S, const Blk& b, const Par& p, int i, int j, int k, size_t s, const double* DU) {
     double U[MAXV];
     for (int m = 0; m < p.NV; m++) { U[m] = b.U[m][s] + DU[m]; b.U[m][s] = U[m]; }
     if (p.limit_flow != 1) return;
     double d1, u1, v1, w1, p1;
     lim_prims(U, p.gamma, d1, u1, v1, w1, p1);
-    if (lim_out(p, d1, u1, v1, w1, p1)) atomicAdd(&b.flags[1], 1);
+    if (lim_out(p, d1, u1, v1, w1, p1)) { atomicAdd(&b.flags[1], 1); *S.limited = 1; }
     if (p.NV == 6) {
         const double v = U[5];
         b.prim[5][s] = v;
         if (v > p.LSAmax) {
             atomicAdd(&b.flags[2], 1);
+            *S.limited = 1;
             long c = sa_cell_index(b, i, j, k);
             atomicOr(&b.samask[c >> 6], 1ull << (c & 63));
         } else if (v < 1.0e-8) {
@@ -873,7 +948,7 @@ __global__ void __launch_bounds__(64) k_update_detect(BSet S) {
     const size_t s = IX(b, i, j, k);
     double DU[MAXV];
     for (int m = 0; m < p.NV; m++) DU[m] = b.DU[m][s];
-    update_cell(b, p, i, j, k, s, DU);
+    update_cell(S, b, p, i, j, k, s, DU);
 }
 
 // The update of an iteration with the pipelined sweeps: the backward sweep's DU comes from the
@@ -912,7 +987,7 @@ __global__ void __launch_bounds__(UP_T) k_update_pk(BSet S, const LuTask* __rest
         double DU[MAXV];
 #pragma unroll
         for (int m = 0; m < NV; m++) DU[m] = buf[m][c][x];
-        update_cell(b, p, i, j, k, IX(b, i, j, k), DU);
+        update_cell(S, b, p, i, j, k, IX(b, i, j, k), DU);
     }
 }
 
@@ -926,9 +1001,8 @@ __device__ __forceinline__ bool lim_cell(const Blk& b, const Par& p, size_t s, d
 // limit_flow_U replacement step (sub_limitflow.f90:84-150): bad cells take the mean of the valid
 // 3x3x3 neighbours' primitive states, or their own clamped state; sets the IF_OverLimit latch.
 // The states come from U after the update: the valid cells keep it through the step, and the
-// new U of a bad cell goes to prim[0..4] (free after the residual) until k_limit_commit, once
-// every bad cell has read its neighbours.  (One launch of a few thousand workgroups looping over
-// the cell tiles: when no block has a bad cell, the usual case, it ends within microseconds.)
+// new U of a bad cell goes to prim[0..4] (free after the residual) until k_limit_finish, once
+// every bad cell has read its neighbours.
 __device__ __forceinline__ void limit_apply_cell(const Blk& b, const Par& p, int i, int j, int k) {
     if (i == 1 && j == 1 && k == 1) b.flags[0] = 1;
     size_t s = IX(b, i, j, k);
@@ -959,35 +1033,19 @@ __device__ __forceinline__ void limit_apply_cell(const Blk& b, const Par& p, int
     b.prim[4][s] = p0 / (p.gamma - 1.0) + (0.5 * d0) * ((u0 * u0 + v0 * v0) + w0 * w0);
 }
 
-// the cell tiles of the blocks whose flag word `which` is nonzero, spread over the grid: every
-// workgroup walks the block list (uniform, scalar loads) and skips an unflagged block whole
+// the cell tiles of the blocks whose flag word `which` is nonzero, every step-th from the first-th
+// on: a workgroup walks the block list (uniform, scalar loads) and skips an unflagged block whole
 template <typename F>
-__device__ __forceinline__ void flagged_tiles(const BSet& S, int nb, int ntiles, int which, F&& f) {
+__device__ __forceinline__ void flagged_tiles(const BSet& S, int nb, int ntiles, int first, int step, int lane, int which, F&& f) {
     for (int bi = 0; bi < nb; bi++) {
         const Blk& b = S.blk[bi];
         if (b.flags[which] == 0) continue;
         const int t1 = bi + 1 < nb ? S.tile0[bi + 1] : ntiles;
-        for (int t = S.tile0[bi] + (int)blockIdx.x; t < t1; t += (int)gridDim.x) {
+        for (int t = S.tile0[bi] + first; t < t1; t += step) {
             int bj, i, j, k;
-            if (locate_tile<SP_CELL>(S, t, bj, i, j, k)) f(b, S.par[bi], i, j, k);
+            if (locate_tile<SP_CELL>(S, t, bj, i, j, k, lane)) f(b, S.par[bi], i, j, k);
         }
     }
-}
-
-__global__ void __launch_bounds__(64) k_limit_apply(BSet S, int nb, int ntiles) {
-    if (halted(S)) return;
-    flagged_tiles(S, nb, ntiles, 1, [](const Blk& b, const Par& p, int i, int j, int k) { limit_apply_cell(b, p, i, j, k); });
-}
-
-// the new U of the bad cells, once every bad cell has read its neighbours
-__global__ void __launch_bounds__(64) k_limit_commit(BSet S, int nb, int ntiles) {
-    if (halted(S)) return;
-    flagged_tiles(S, nb, ntiles, 1, [](const Blk& b, const Par& p, int i, int j, int k) {
-        const size_t s = IX(b, i, j, k);
-        double d1, u1, v1, w1, p1;
-        if (lim_cell(b, p, s, d1, u1, v1, w1, p1))
-            for (int m = 0; m < 5; m++) b.U[m][s] = b.prim[m][s];
-    });
 }
 
 // limit_flow_SA (sub_limitflow.f90:182-231).  The reference clamps and averages in place in
@@ -1032,18 +1090,23 @@ __device__ __forceinline__ void limit_sa_isolated_cell(const Blk& b, const Par& 
     atomicAnd(&b.samask[c >> 6], ~(1ull << (c & 63)));
 }
 
-__global__ void __launch_bounds__(64) k_limit_sa_isolated(BSet S, int nb, int ntiles) {
-    if (halted(S)) return;
-    flagged_tiles(S, nb, ntiles, 2, [](const Blk& b, const Par& p, int i, int j, int k) { limit_sa_isolated_cell(b, p, i, j, k); });
+// The limiter after the update in two launches: k_limit replaces limit_flow_U's bad cells into
+// prim[0..4] and the isolated flagged cells of SA (the two work on different variables), and
+// k_limit_finish commits the former and replaces the clustered flagged cells in order.  When no
+// cell of the set is out of the limits, the usual case, one word sends every workgroup home (with
+// the walk of the block list, the update and limiter of 8 small solves took 109 us, now 60).
+__global__ void __launch_bounds__(64) k_limit(BSet S, int nb, int ntiles) {
+    if (*S.limited == 0 || halted(S)) return;
+    flagged_tiles(S, nb, ntiles, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, 1,
+                  [](const Blk& b, const Par& p, int i, int j, int k) { limit_apply_cell(b, p, i, j, k); });
+    flagged_tiles(S, nb, ntiles, (int)blockIdx.x, (int)gridDim.x, (int)threadIdx.x, 2,
+                  [](const Blk& b, const Par& p, int i, int j, int k) { limit_sa_isolated_cell(b, p, i, j, k); });
 }
 
-// one workgroup per block: the flagged cells left by the isolated pass, by increasing w over the
-// box that bounds them; clears the mask
+// the flagged cells of block b left by the isolated pass, by increasing w over the box that bounds
+// them, by one workgroup of SA_ORD_T threads; clears the mask
 constexpr int SA_ORD_T = 256;
-__global__ void __launch_bounds__(SA_ORD_T) k_limit_sa_ordered(BSet S) {
-    if (halted(S)) return;
-    const Blk& b = S.blk[blockIdx.x];
-    const Par& p = S.par[blockIdx.x];
+__device__ __forceinline__ void limit_sa_ordered(const Blk& b, const Par& p) {
     if (b.flags[2] == 0) return;
     const int nxm = b.nx - 1, nym = b.ny - 1;
     const long ncell = (long)nxm * nym * (b.nz - 1);
@@ -1084,17 +1147,21 @@ __global__ void __launch_bounds__(SA_ORD_T) k_limit_sa_ordered(BSet S) {
         if (b.samask[wi]) b.samask[wi] = 0ull;
 }
 
-__global__ void k_reset_flags(BSet S) {
-    const Blk& b = S.blk[blockIdx.x];
-    if (threadIdx.x == 0) { b.flags[1] = 0; b.flags[2] = 0; }
-}
-
-// force_vt_kw (sub_time_advance.f90:27-61)
-__global__ void __launch_bounds__(64) k_force_vt_kw(BSet S) {
-    if (halted(S)) return;
-    OCFD_LOCATE(SP_CELL)
-    size_t s = IX(b, i, j, k);
-    for (int m = 5; m < p.NV; m++) if (b.U[m][s] < 0) b.U[m][s] = 1.0e-10;
+__global__ void __launch_bounds__(SA_ORD_T) k_limit_finish(BSet S, int nb, int ntiles) {
+    if (*S.limited == 0 || halted(S)) return;
+    if ((int)blockIdx.x < nb) {        // a workgroup per block
+        if (S.par[blockIdx.x].NV == 6) limit_sa_ordered(S.blk[blockIdx.x], S.par[blockIdx.x]);
+        return;
+    }
+    // the new U of the bad cells, once every bad cell has read its neighbours: a wave per tile
+    const int wave = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
+    flagged_tiles(S, nb, ntiles, ((int)blockIdx.x - nb) * (SA_ORD_T / 64) + wave, ((int)gridDim.x - nb) * (SA_ORD_T / 64), lane, 1,
+                  [](const Blk& b, const Par& p, int i, int j, int k) {
+                      const size_t s = IX(b, i, j, k);
+                      double d1, u1, v1, w1, p1;
+                      if (lim_cell(b, p, s, d1, u1, v1, w1, p1))
+                          for (int m = 0; m < 5; m++) b.U[m][s] = b.prim[m][s];
+                  });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1242,13 +1309,6 @@ __global__ void __launch_bounds__(64) k_bc(SubSet S) {
     }
 }
 
-// Amut_boundary on every wall subface of the set
-__global__ void __launch_bounds__(64) k_amut(SubSet S) {
-    OCFD_SUB_LOCATE
-    (void)p;
-    d_amut(b, B, a, c);
-}
-
 // Umessage_send_mpi local copy (sub_update_buffer_mpi.f90:42-141): LAP ghost layers of the
 // neighbour block from this block's interior, with the L1..L3 axis permutation and order.
 __device__ __forceinline__ void d_halo(const Blk& src, const Blk& dst, const HaloMap& h, int NV, int t) {
@@ -1295,6 +1355,9 @@ __device__ __forceinline__ void d_corner_edges(const Blk& b, int NV, int t, int 
     (void)NV;
 }
 
+// FRESH: the edge cells are formed here from the faces' ghost cells, as d_corner_edges forms them,
+// so edges and vertices need no order between them
+template <bool FRESH>
 __device__ __forceinline__ void d_corner_vertices(const Blk& b, int c, int m) {
     if (c >= 8) return;
     int nx = b.nx, ny = b.ny, nz = b.nz;
@@ -1302,25 +1365,43 @@ __device__ __forceinline__ void d_corner_vertices(const Blk& b, int c, int m) {
     auto V = [&](int i, int j, int k) { return U[IX(b, i, j, k)]; };
     int I = (c & 1) ? nx : 0, J = (c & 2) ? ny : 0, K = (c & 4) ? nz : 0;
     int Ii = (c & 1) ? nx - 1 : 1, Jj = (c & 2) ? ny - 1 : 1, Kk = (c & 4) ? nz - 1 : 1;
-    double r = (2.0 * ((V(Ii, J, K) + V(I, Jj, K)) + V(I, J, Kk)) - ((V(Ii, Jj, K) + V(Ii, J, Kk)) + V(I, Jj, Kk))) / 3.0;
+    double eI, eJ, eK;
+    if (FRESH) {
+        eI = (V(Ii, Jj, K) + V(Ii, J, Kk)) * 0.5;
+        eJ = (V(Ii, Jj, K) + V(I, Jj, Kk)) * 0.5;
+        eK = (V(Ii, J, Kk) + V(I, Jj, Kk)) * 0.5;
+    } else { eI = V(Ii, J, K); eJ = V(I, Jj, K); eK = V(I, J, Kk); }
+    double r = (2.0 * ((eI + eJ) + eK) - ((V(Ii, Jj, K) + V(Ii, J, Kk)) + V(I, Jj, Kk))) / 3.0;
     U[IX(b, I, J, K)] = r;
 }
 
-// edges then vertices of every block of the set (blockIdx.y: edge, blockIdx.z: block x variable);
-// a workgroup walks its whole edge
-__global__ void k_corner_edges(BSet S, int NV) {
-    const Blk& b = S.blk[blockIdx.z / NV];
-    const int len = max(b.nx, max(b.ny, b.nz));
-    for (int t = (int)threadIdx.x; t < len; t += (int)blockDim.x) d_corner_edges(b, NV, t, blockIdx.y, blockIdx.z % NV);
-}
-__global__ void k_corner_vertices(BSet S, int NV) {
-    d_corner_vertices(S.blk[blockIdx.x / NV], threadIdx.x, blockIdx.x % NV);
+// The launch that ends an iteration: edges and vertices of every block (get_U_conner) and
+// force_vt_kw (sub_time_advance.f90:27-61), which changes cells that no edge or vertex reads.
+// Workgroup 13 (NV block + variable) + edge walks an edge, + 12 forms the vertices, which take the
+// edge cells they need from the faces' ghost cells, as the edges do; the cells' tiles follow.
+// (nb 0: no edges and vertices.)
+__global__ void __launch_bounds__(64) k_corner_force(BSet S, int nb, int NV) {
+    const int nc = 13 * nb * NV;
+    if ((int)blockIdx.x < nc) {
+        const int e = (int)blockIdx.x % 13, m = (int)blockIdx.x / 13 % NV;
+        const Blk& b = S.blk[(int)blockIdx.x / (13 * NV)];
+        const int len = max(b.nx, max(b.ny, b.nz));
+        if (e < 12) { for (int t = (int)threadIdx.x; t < len; t += 64) d_corner_edges(b, NV, t, e, m); }
+        else d_corner_vertices<true>(b, threadIdx.x, m);
+        return;
+    }
+    if (halted(S)) return;
+    int bi, i, j, k;
+    if (!locate_tile<SP_CELL>(S, (int)blockIdx.x - nc, bi, i, j, k, (int)threadIdx.x)) return;
+    const Blk& b = S.blk[bi];
+    const size_t s = IX(b, i, j, k);
+    for (int m = 5; m < NV; m++) if (b.U[m][s] < 0) b.U[m][s] = 1.0e-10;
 }
 // single-block forms, used while the geometry is set up
 __global__ void k_corner_edges1(Blk b, int NV) {
     d_corner_edges(b, NV, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, blockIdx.z);
 }
-__global__ void k_corner_vertices1(Blk b) { d_corner_vertices(b, threadIdx.x, blockIdx.x); }
+__global__ void k_corner_vertices1(Blk b) { d_corner_vertices<false>(b, threadIdx.x, blockIdx.x); }
 
 // ---------------------------------------------------------------------------------------------
 // comput_max_Res_onemesh (sub_time_advance.f90:330-380): per block, component and part (a fixed
@@ -1434,7 +1515,7 @@ __global__ void k_force_final(int nparts, const double* part, double* out9) {
 // host launchers.  Every launch covers all blocks of the set; the per-block conditions of the
 // reference (turbulence model, limiter, NVAR) are uniform over a set.
 static inline dim3 g3(int n0, int n1, int n2, int bs) { return dim3((unsigned)((n0 + bs - 1) / bs), (unsigned)n1, (unsigned)n2); }
-static inline BSet bset(const SetPlan& P, int sp) { return BSet{P.blk, P.par, P.tile_blk[sp], P.tile0[sp], P.halt}; }
+static inline BSet bset(const SetPlan& P, int sp) { return BSet{P.blk, P.par, P.tile_blk[sp], P.tile0[sp], P.halt, P.limited}; }
 
 template <int SP>
 static void launch_space(void (*kern)(BSet), const SetPlan& P, hipStream_t st) {
@@ -1445,44 +1526,36 @@ static void launch_subs(void (*kern)(SubSet), const SetPlan& P, const SubList& L
     if (L.ntiles > 0) hipLaunchKernelGGL(kern, dim3((unsigned)L.ntiles), dim3(64), 0, st, SubSet{P.blk, P.par, L.t, L.tile_task});
 }
 
+static void launch_faces(void (*kern)(FaceSet), const SetPlan& P, hipStream_t st) {
+    FaceSet S{P.blk, P.par, {}, {}, {}};
+    for (int d = 0; d < 3; d++) {
+        S.tile_blk[d] = P.tile_blk[SP_FI + d];
+        S.tile0[d] = P.tile0[SP_FI + d];
+        S.n[d] = P.ntiles[SP_FI + d];
+    }
+    const int n = face_grid(S.n);
+    if (n > 0) hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64), 0, st, S);
+}
+
 void set_pre(const SetPlan& P, hipStream_t st) {
     const Par& p = P.p0;
-    hipLaunchKernelGGL(k_reset_flags, dim3((unsigned)P.nb), dim3(64), 0, st, bset(P, SP_CELL));
-    launch_space<SP_BOX>(k_prims, P, st);      // with get_viscous on the interior cells
+    launch_space<SP_BOX>(k_prims, P, st);
     if (p.visc != 1) return;
-    launch_subs(k_visc_ghost, P, P.vghost, st);
-    if (p.turb == 2) {
-        launch_space<SP_N0>(k_sa_mut, P, st);
-        launch_subs(k_amut, P, P.amut, st);
-    } else if (p.turb == 3) {
+    if (p.turb == 3) {
         if (p.mixed) launch_space<SP_CELL>(k_sst_cell<float>, P, st);
         else launch_space<SP_CELL>(k_sst_cell<double>, P, st);
-        int m3 = P.mx + 3;
-        for (int f = 0; f < 6; f++)
-            hipLaunchKernelGGL(k_sst_ghost, dim3((unsigned)((m3 + 63) / 64), (unsigned)m3, (unsigned)P.nb), dim3(64), 0, st, bset(P, SP_CELL), f);
+        launch_subs(k_sst_ghost, P, P.sghost, st);
         launch_subs(k_amut, P, P.amut, st);
-        if (p.mixed) {
-            launch_space<SP_FI>(k_sst_face<0, float>, P, st);
-            launch_space<SP_FJ>(k_sst_face<1, float>, P, st);
-            launch_space<SP_FK>(k_sst_face<2, float>, P, st);
-        } else {
-            launch_space<SP_FI>(k_sst_face<0, double>, P, st);
-            launch_space<SP_FJ>(k_sst_face<1, double>, P, st);
-            launch_space<SP_FK>(k_sst_face<2, double>, P, st);
-        }
-        launch_space<SP_CELL>(k_sst_res, P, st);
-        launch_space<SP_N0>(k_sst_finish, P, st);
-        launch_subs(k_amut, P, P.amut, st);
-    } else {
-        launch_subs(k_amut, P, P.amut, st);
+        if (p.mixed) launch_faces(k_sst_face<float>, P, st);
+        else launch_faces(k_sst_face<double>, P, st);
+        launch_space<SP_N0>(k_sst_res, P, st);
     }
+    launch_subs(k_amut, P, P.amut, st);
 }
 
 template <typename T, int R, int FL>
 static void faces_rf(const SetPlan& P, hipStream_t st) {
-    launch_space<SP_FI>(k_face<0, T, R, FL>, P, st);
-    launch_space<SP_FJ>(k_face<1, T, R, FL>, P, st);
-    launch_space<SP_FK>(k_face<2, T, R, FL>, P, st);
+    launch_faces(k_face<T, R, FL>, P, st);
 }
 // the reconstruction variable set (IFlag_Reconstruction) and, for the primitive-variable
 // reconstruction, the 1-D flux as template arguments: each kernel holds only its own
@@ -1547,13 +1620,8 @@ static void limit_after_update(const SetPlan& P, hipStream_t st) {
     if (P.p0.limit_flow != 1) return;
     const int n = P.ntiles[SP_CELL];
     if (n <= 0) return;
-    const dim3 grid((unsigned)std::min(n, 4096));
-    hipLaunchKernelGGL(k_limit_apply, grid, dim3(64), 0, st, bset(P, SP_CELL), P.nb, n);
-    hipLaunchKernelGGL(k_limit_commit, grid, dim3(64), 0, st, bset(P, SP_CELL), P.nb, n);
-    if (P.p0.NV == 6) {
-        hipLaunchKernelGGL(k_limit_sa_isolated, grid, dim3(64), 0, st, bset(P, SP_CELL), P.nb, n);
-        hipLaunchKernelGGL(k_limit_sa_ordered, dim3((unsigned)P.nb), dim3(SA_ORD_T), 0, st, bset(P, SP_CELL));
-    }
+    hipLaunchKernelGGL(k_limit, dim3((unsigned)std::min(n, 4096)), dim3(64), 0, st, bset(P, SP_CELL), P.nb, n);
+    hipLaunchKernelGGL(k_limit_finish, dim3((unsigned)(P.nb + std::min((n + 3) / 4, 1024))), dim3(SA_ORD_T), 0, st, bset(P, SP_CELL), P.nb, n);
 }
 
 void set_update_limit(const SetPlan& P, hipStream_t st) {
@@ -1584,19 +1652,27 @@ void set_update_limit_sweep_order(const SetPlan& P, const LuPlan& L, hipStream_t
 
 void set_bc(const SetPlan& P, hipStream_t st) { launch_subs(k_bc, P, P.bc, st); }
 
-void set_halo(const SetPlan& P, hipStream_t st) {
-    if (P.halo.ntiles > 0)
-        hipLaunchKernelGGL(k_halo_set, dim3((unsigned)P.halo.ntiles), dim3(256), 0, st, HaloSet{P.blk, P.halo.t, P.halo.tile_task}, P.p0.NV);
-    hipLaunchKernelGGL(k_corner_edges, dim3(1, 12, (unsigned)(P.p0.NV * P.nb)), dim3(64), 0, st, bset(P, SP_CELL), P.p0.NV);
-    hipLaunchKernelGGL(k_corner_vertices, dim3((unsigned)(P.p0.NV * P.nb)), dim3(64), 0, st, bset(P, SP_CELL), P.p0.NV);
-}
-
 // force_vt_kw (sub_time_advance.f90:27-61): U6 (and U7) below 0 set to 1e-10 in the cells.  With SA
 // and the limiter on, the update has already raised every cell's U6 below 1e-8 to 1e-8 and the SA
-// replacement writes positive values only, so the pass cannot change anything and is not launched.
-void set_force_vt_kw(const SetPlan& P, hipStream_t st) {
-    if (P.p0.NV == 6 && P.p0.limit_flow == 1) return;
-    if (P.p0.NV >= 6) launch_space<SP_CELL>(k_force_vt_kw, P, st);
+// replacement writes positive values only, so the pass cannot change anything and is left out.
+static void corner_force(const SetPlan& P, bool corners, bool force, hipStream_t st) {
+    const int nb = corners ? P.nb : 0, NV = P.p0.NV;
+    const int nf = force && NV >= 6 && !(NV == 6 && P.p0.limit_flow == 1) ? P.ntiles[SP_CELL] : 0;
+    const int n = 13 * nb * NV + nf;
+    if (n > 0) hipLaunchKernelGGL(k_corner_force, dim3((unsigned)n), dim3(64), 0, st, bset(P, SP_CELL), nb, NV);
+}
+static void halo_copy(const SetPlan& P, hipStream_t st) {
+    if (P.halo.ntiles > 0)
+        hipLaunchKernelGGL(k_halo_set, dim3((unsigned)P.halo.ntiles), dim3(256), 0, st, HaloSet{P.blk, P.halo.t, P.halo.tile_task}, P.p0.NV);
+}
+void set_halo(const SetPlan& P, hipStream_t st) {
+    halo_copy(P, st);
+    corner_force(P, true, false, st);
+}
+void set_force_vt_kw(const SetPlan& P, hipStream_t st) { corner_force(P, false, true, st); }
+void set_halo_force(const SetPlan& P, hipStream_t st) {
+    halo_copy(P, st);
+    corner_force(P, true, true, st);
 }
 
 void launch_norms(const NormBlk* tab, int nb, int NV, double* part, double* out, hipStream_t st) {

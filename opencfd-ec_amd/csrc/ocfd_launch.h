@@ -28,10 +28,11 @@ struct SetPlan {
     int* tile_blk[SP_COUNT] = {};
     int* tile0[SP_COUNT] = {};
     int ntiles[SP_COUNT] = {};
-    SubList bc, amut, kbc, force;   // force: the wall (bc 2) subfaces, one thread per face
-    SubList vghost;                  // the six faces of every block (k_visc_ghost)
+    SubList bc, force;               // force: the wall (bc 2) subfaces, one thread per face
+    SubList amut, kbc;               // wall and k subfaces that do not lie on their block's face (usually none)
+    SubList sghost;                  // SST: the six faces of every block with their ghost rows (k_sst_ghost)
     HaloList halo;
-    int mx = 0;                      // max over blocks of max(nx, ny, nz)
+    int* limited = nullptr;          // set by the update when a cell of the set needs the limiter
     const int* halt = nullptr;       // the LU-SGS error word of the engine's sweeps (or null)
 };
 
@@ -46,6 +47,8 @@ void set_update_limit_sweep_order(const SetPlan& P, const LuPlan& L, hipStream_t
 void set_bc(const SetPlan& P, hipStream_t st);
 void set_halo(const SetPlan& P, hipStream_t st);
 void set_force_vt_kw(const SetPlan& P, hipStream_t st);
+// set_halo followed by set_force_vt_kw
+void set_halo_force(const SetPlan& P, hipStream_t st);
 // the residual norms of a table of blocks: parts (nb x NV x norms_parts() x 3 doubles), then
 // out (3 NV doubles: max, sum of squares, NaN flag per component)
 constexpr int NORMS_PARTS = 64;

@@ -274,13 +274,25 @@ Par to_par(const ocfd_params& h) {
     return p;
 }
 
+// whether a subface lies on the block face that its face id names
+static bool on_face(const HostBlock& hb, const Sub& B) {
+    const int lo[3] = {B.ib, B.jb, B.kb}, hi[3] = {B.ie, B.je, B.ke}, n[3] = {hb.nx, hb.ny, hb.nz};
+    const int d = (B.face - 1) % 3, at = B.face <= 3 ? 1 : n[d];
+    return lo[d] == at && hi[d] == at;
+}
+
 // boundary indicators BcI/BcJ/BcK (set_BcK, sub_init.f90:545-577) as per-row bit flags
 int upload_bcflags(HostBlock& hb) {
     const Blk& b = hb.d;
     std::vector<uint8_t> fi((size_t)b.NJ * b.NK, 0), fj((size_t)b.NI * b.NK, 0), fk((size_t)b.NI * b.NJ, 0);
     for (const Sub& B : hb.subs) {
         if (B.bc < 0) continue;
-        uint8_t bit = B.face <= 3 ? 1 : 2;
+        uint8_t bit = BCF_PHYS;
+        if (on_face(hb, B)) {
+            if (B.bc == 2) bit |= BCF_WALL;
+            if (B.bc > 0 && B.face % 3 == 0) bit |= BCF_KBC;
+        }
+        if (B.face > 3) bit <<= 1;
         if (B.face == 1 || B.face == 4) { for (int k = B.kb; k <= B.ke - 1; k++) for (int j = B.jb; j <= B.je - 1; j++) fi[JK(b, j, k)] |= bit; }
         else if (B.face == 2 || B.face == 5) { for (int k = B.kb; k <= B.ke - 1; k++) for (int i = B.ib; i <= B.ie - 1; i++) fj[IK(b, i, k)] |= bit; }
         else { for (int j = B.jb; j <= B.je - 1; j++) for (int i = B.ib; i <= B.ie - 1; i++) fk[IJ(b, i, j)] |= bit; }
@@ -368,8 +380,7 @@ void enqueue_stage(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, 
         break;
     case OCFD_STAGE_BC_HALO:
         set_bc(P, e.st);
-        set_halo(P, e.st);
-        set_force_vt_kw(P, e.st);
+        set_halo_force(P, e.st);
         break;
     }
 }
@@ -719,7 +730,6 @@ int build_set_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) 
     for (int bi = 0; bi < P.nb; bi++) {
         const HostBlock& hb = *refs[bi].hb;
         const Par& p = *refs[bi].p;
-        P.mx = std::max(P.mx, std::max(hb.nx, std::max(hb.ny, hb.nz)));
         for (const Sub& B : hb.subs) {
             SubTask t{};
             t.blk = bi; t.B = B;
@@ -733,7 +743,7 @@ int build_set_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) 
                 else t.kind = SUB_EXT;
                 bc.push_back(t);
                 if (B.bc == 2) {
-                    SubTask a = t; a.kind = SUB_AMUT; amut.push_back(a);
+                    if (!on_face(hb, B)) { SubTask a = t; a.kind = SUB_AMUT; amut.push_back(a); }
                     // comput_force's face loop: cells of the two tangential directions
                     SubTask fo = t;
                     const int d = (B.face - 1) % 3;
@@ -741,7 +751,7 @@ int build_set_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) 
                     fo.n1 = d == 2 ? B.je - B.jb : B.ke - B.kb;
                     if (fo.n0 > 0 && fo.n1 > 0) force.push_back(fo);
                 }
-                if (B.face == 3 || B.face == 6) {
+                if ((B.face == 3 || B.face == 6) && !on_face(hb, B)) {
                     SubTask k = t;
                     k.kind = SUB_KBC; k.n0 = B.ie - B.ib; k.n1 = std::max(1, B.je - B.jb);
                     kbc.push_back(k);
@@ -755,20 +765,21 @@ int build_set_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) 
             }
         }
     }
-    std::vector<SubTask> vghost;
-    for (int bi = 0; bi < P.nb; bi++) {
+    std::vector<SubTask> sghost;
+    for (int bi = 0; bi < P.nb && p0.turb == 3; bi++) {
         const Blk& b = blks[bi];
         for (int f = 0; f < 6; f++) {
             SubTask t{};
             t.blk = bi; t.arg = f;
-            t.n0 = f < 2 ? b.ny - 1 : b.nx - 1;
-            t.n1 = f < 4 ? b.nz - 1 : b.ny - 1;
-            vghost.push_back(t);
+            t.n0 = f < 2 ? b.ny + 1 : b.nx + 1;
+            t.n1 = f < 4 ? b.nz + 1 : b.ny + 1;
+            sghost.push_back(t);
         }
     }
     if ((r = build_sub_list(e.set_allocs, bc, P.bc)) || (r = build_sub_list(e.set_allocs, amut, P.amut)) ||
         (r = build_sub_list(e.set_allocs, kbc, P.kbc)) || (r = build_sub_list(e.set_allocs, force, P.force)) ||
-        (r = build_sub_list(e.set_allocs, vghost, P.vghost)))
+        (r = build_sub_list(e.set_allocs, sghost, P.sghost)) ||
+        (r = upload_table(e.set_allocs, std::vector<int>(1, 0), &P.limited)))
         return r;
     P.halo.ntiles = (int)halo_tile.size();
     if ((r = upload_table(e.set_allocs, halo, &P.halo.t)) || (r = upload_table(e.set_allocs, halo_tile, &P.halo.tile_task))) return r;
