@@ -12,6 +12,37 @@ namespace ocfd {
 constexpr int LAP = 4;
 constexpr int MAXV = 7;
 
+// A pointer to device memory in a table that kernels read.  A plain pointer loaded from memory could
+// point anywhere, so the compiler uses flat accesses: a 64-bit address in vector registers for each,
+// and waits that cover LDS too.  In device code this one says that it points to global memory.
+template <typename T>
+struct gptr {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(1))) T* ptr;
+#else
+    typedef T* ptr;
+#endif
+    ptr p;
+    __host__ __device__ __forceinline__ operator T*() const { return (T*)p; }
+    __host__ __device__ __forceinline__ gptr& operator=(T* q) { p = (ptr)q; return *this; }
+    // element s of a box: the base stays in scalar registers and a lane's address is one 32-bit byte
+    // offset, shared by the arrays of a block.  A box array stays below 4 GiB: a block has 95 of them
+    // or more, and a device 288 GB.
+    __host__ __device__ __forceinline__ T& operator[](size_t s) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return *(T*)(ptr)((__attribute__((address_space(1))) const char*)p + (uint32_t)((uint32_t)s * (uint32_t)sizeof(T)));
+#else
+        return p[s];
+#endif
+    }
+    __host__ __device__ __forceinline__ T& operator[](uint32_t s) const { return (*this)[(size_t)s]; }
+    __host__ __device__ __forceinline__ T& operator[](long s) const { return ((T*)p)[s]; }
+    __host__ __device__ __forceinline__ T& operator[](int s) const { return ((T*)p)[s]; }
+    // the array shifted by an offset that is the same in all lanes (a stencil's neighbour): at(o)[s]
+    // is element s + o
+    __host__ __device__ __forceinline__ gptr at(long o) const { return gptr{p + o}; }
+};
+
 struct Par {                 // control parameters after set_const_para (sub_read_parameter.f90:371-429)
     double Ma, Re, gamma, Cv, Cp, PrL, PrT, T_inf, Twall, AoA, A_alfa, A_beta, P_outlet;
     double CFL, dtmax, dtmin, dt_global, w_LU, MUT_MAX, Kt_inf, Wt_inf;
@@ -22,27 +53,27 @@ struct Par {                 // control parameters after set_const_para (sub_rea
 
 struct Blk {
     int nx, ny, nz, NI, NJ, NK;
-    double *U[MAXV], *Res[MAXV], *DU[MAXV];
-    double *dt, *mu, *muf, *mut;        // mu: Sutherland; muf: mu after the turbulence-model (x*Re)/Re round trip
-    double *prim[7];                     // rho u v w p T c (per iteration; limiter snapshot afterwards)
-    double *Lc[3], *Lv[3];
-    double *vol, *S[3], *nv[9], *met[4][9], *dw, *dtm, *x, *y, *z, *xc, *yc, *zc;
-    double *F[3][5];                     // inviscid face flux, m = 1..5
-    double *Fv[3][4];                    // viscous face flux, m = 2..5
-    double *Fsa[3][2];                   // SA face terms: convection+diffusion flux, grad(vt).n S; SST: k and omega fluxes
+    gptr<double> U[MAXV], Res[MAXV], DU[MAXV];
+    gptr<double> dt, mu, muf, mut;        // mu: Sutherland; muf: mu after the turbulence-model (x*Re)/Re round trip
+    gptr<double> prim[7]; // rho u v w p T c (per iteration; limiter snapshot afterwards)
+    gptr<double> Lc[3], Lv[3];
+    gptr<double> vol, S[3], nv[9], met[4][9], dw, dtm, x, y, z, xc, yc, zc;
+    gptr<double> F[3][5]; // inviscid face flux, m = 1..5
+    gptr<double> Fv[3][4]; // viscous face flux, m = 2..5
+    gptr<double> Fsa[3][2]; // SA face terms: convection+diffusion flux, grad(vt).n S; SST: k and omega fluxes
     // mixed precision: FP32 primitives (rho u v w p T) and FP32 face terms; the face arrays share
     // the memory of their FP64 counterparts
-    float *primf[6], *Ff[3][5], *Fvf[3][4], *Fsaf[3][2];
+    gptr<float> primf[6], Ff[3][5], Fvf[3][4], Fsaf[3][2];
     // mixed precision: FP32 copies of the geometry the FP32 kernels read (face normals, areas,
     // metrics, and per direction the node difference t1 of the inviscid flux's face frame), made
     // once per block from the FP64 arrays
-    float *nvf[9], *Sf[3], *metf[4][9], *t1f[3][3];
-    double *aux;                         // turbulence scratch (SST f1)
-    double *kt, *wt;                     // SST: k and omega per unit mass, max(U, 0) / rho, on the box
-    uint8_t *bcf[3];                     // face-row flags (BcFlag; the upper face's bit is the lower's << 1)
-    double *surf[6][3];                  // Surf1..6 (wall viscous force of the i-/j-/k-/i+/j+/k+ faces)
-    int *flags;                          // [0] IF_OverLimit latch, [1] limited cells this iteration, [2] SA cells above LSAmax
-    unsigned long long *samask;          // SA cells above LSAmax, one bit per cell in (i,j,k) order (SA only)
+    gptr<float> nvf[9], Sf[3], metf[4][9], t1f[3][3];
+    gptr<double> aux; // turbulence scratch (SST f1)
+    gptr<double> kt, wt; // SST: k and omega per unit mass, max(U, 0) / rho, on the box
+    gptr<uint8_t> bcf[3]; // face-row flags (BcFlag; the upper face's bit is the lower's << 1)
+    gptr<double> surf[6][3]; // Surf1..6 (wall viscous force of the i-/j-/k-/i+/j+/k+ faces)
+    gptr<int> flags; // [0] IF_OverLimit latch, [1] limited cells this iteration, [2] SA cells above LSAmax
+    gptr<unsigned long long> samask;          // SA cells above LSAmax, one bit per cell in (i,j,k) order (SA only)
 };
 
 // per face row of a direction: the lower face is physical, lies on a wall, takes the explicit flux
@@ -50,15 +81,17 @@ struct Blk {
 enum BcFlag : int { BCF_PHYS = 1, BCF_WALL = 4, BCF_KBC = 16 };
 
 __device__ __host__ __forceinline__ size_t IX(const Blk& b, int i, int j, int k) {
-    return (size_t)(i + 3) + (size_t)b.NI * ((size_t)(j + 3) + (size_t)b.NJ * (size_t)(k + 3));
+    return (uint32_t)(i + 3) + (uint32_t)b.NI * ((uint32_t)(j + 3) + (uint32_t)b.NJ * (uint32_t)(k + 3));
 }
-__device__ __host__ __forceinline__ size_t JK(const Blk& b, int j, int k) { return (size_t)(j + 3) + (size_t)b.NJ * (size_t)(k + 3); }
-__device__ __host__ __forceinline__ size_t IK(const Blk& b, int i, int k) { return (size_t)(i + 3) + (size_t)b.NI * (size_t)(k + 3); }
-__device__ __host__ __forceinline__ size_t IJ(const Blk& b, int i, int j) { return (size_t)(i + 3) + (size_t)b.NI * (size_t)(j + 3); }
+__device__ __host__ __forceinline__ size_t JK(const Blk& b, int j, int k) { return (uint32_t)(j + 3) + (uint32_t)b.NJ * (uint32_t)(k + 3); }
+__device__ __host__ __forceinline__ size_t IK(const Blk& b, int i, int k) { return (uint32_t)(i + 3) + (uint32_t)b.NI * (uint32_t)(k + 3); }
+__device__ __host__ __forceinline__ size_t IJ(const Blk& b, int i, int j) { return (uint32_t)(i + 3) + (uint32_t)b.NI * (uint32_t)(j + 3); }
+// the distance between a cell and its neighbour (di, dj, dk) away
+__device__ __host__ __forceinline__ long OFF(const Blk& b, int di, int dj, int dk) { return di + (long)b.NI * (dj + (long)b.NJ * dk); }
 
 // what the residual norms read of a block
 struct NormBlk {
-    const double* res[MAXV];
+    gptr<const double> res[MAXV];
     int nx, ny, nz, NI, NJ;
 };
 

@@ -78,7 +78,7 @@ __global__ void k_geo_centres(Blk b) {
     }
 }
 
-__device__ __forceinline__ void metric_store(double* const* mt, size_t s, double xi, double yi, double zi, double xj, double yj,
+__device__ __forceinline__ void metric_store(const gptr<double>* mt, size_t s, double xi, double yi, double zi, double xj, double yj,
                                              double zj, double xk, double yk, double zk) {
     double Jac1 = ((((xi * yj * zk + yi * zj * xk) + zi * xj * yk) - xi * zj * yk) - yi * xj * zk) - zi * yj * xk;
     if (fabs(Jac1) < 1.0e-20) Jac1 = 1.0e-20;

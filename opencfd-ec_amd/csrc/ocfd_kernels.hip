@@ -110,39 +110,40 @@ __global__ void __launch_bounds__(64) k_prims(BSet S) {
 // ---------------------------------------------------------------------------------------------
 // Spalart-Allmaras (sub_turbulence_SA.f90:8-273).  U6 is read through limit_vt's clamp
 // (sub_time_advance.f90:420-428): negative values act as zero.
-__device__ __forceinline__ double vt_of(const Blk& b, size_t s) { double v = b.U[5][s]; return v < 0.0 ? 0.0 : v; }
+// limit_vt's clamp of U6 at the element o away from s
+__device__ __forceinline__ double vt_of(const Blk& b, size_t s, long o) { double v = b.U[5].at(o)[s]; return v < 0.0 ? 0.0 : v; }
 __device__ __forceinline__ double pw6(double x) { return ((((x * x) * x) * x) * x) * x; }   // flang expansion order
 
 // Storage of the compute type T of the residual: FP64 (the drop-in) or FP32 (the mixed mode's
 // reconstruction, fluxes and turbulence source, whose face fluxes the FP64 assembly reads).
-template <typename T> __device__ __forceinline__ const T* prim_of(const Blk& b, int m);
-template <> __device__ __forceinline__ const double* prim_of<double>(const Blk& b, int m) { return b.prim[m]; }
-template <> __device__ __forceinline__ const float* prim_of<float>(const Blk& b, int m) { return b.primf[m]; }
+template <typename T> __device__ __forceinline__ gptr<T> prim_of(const Blk& b, int m);
+template <> __device__ __forceinline__ gptr<double> prim_of<double>(const Blk& b, int m) { return b.prim[m]; }
+template <> __device__ __forceinline__ gptr<float> prim_of<float>(const Blk& b, int m) { return b.primf[m]; }
 // the geometry in the compute type: for FP32 the copies converted once per block, which hold the
 // values a conversion of the FP64 arrays at every read gives
-template <typename T> __device__ __forceinline__ const T* nv_of(const Blk& b, int q);
-template <> __device__ __forceinline__ const double* nv_of<double>(const Blk& b, int q) { return b.nv[q]; }
-template <> __device__ __forceinline__ const float* nv_of<float>(const Blk& b, int q) { return b.nvf[q]; }
-template <typename T> __device__ __forceinline__ const T* S_of(const Blk& b, int d);
-template <> __device__ __forceinline__ const double* S_of<double>(const Blk& b, int d) { return b.S[d]; }
-template <> __device__ __forceinline__ const float* S_of<float>(const Blk& b, int d) { return b.Sf[d]; }
-template <typename T> __device__ __forceinline__ const T* met_of(const Blk& b, int m, int q);
-template <> __device__ __forceinline__ const double* met_of<double>(const Blk& b, int m, int q) { return b.met[m][q]; }
-template <> __device__ __forceinline__ const float* met_of<float>(const Blk& b, int m, int q) { return b.metf[m][q]; }
+template <typename T> __device__ __forceinline__ gptr<T> nv_of(const Blk& b, int q);
+template <> __device__ __forceinline__ gptr<double> nv_of<double>(const Blk& b, int q) { return b.nv[q]; }
+template <> __device__ __forceinline__ gptr<float> nv_of<float>(const Blk& b, int q) { return b.nvf[q]; }
+template <typename T> __device__ __forceinline__ gptr<T> S_of(const Blk& b, int d);
+template <> __device__ __forceinline__ gptr<double> S_of<double>(const Blk& b, int d) { return b.S[d]; }
+template <> __device__ __forceinline__ gptr<float> S_of<float>(const Blk& b, int d) { return b.Sf[d]; }
+template <typename T> __device__ __forceinline__ gptr<T> met_of(const Blk& b, int m, int q);
+template <> __device__ __forceinline__ gptr<double> met_of<double>(const Blk& b, int m, int q) { return b.met[m][q]; }
+template <> __device__ __forceinline__ gptr<float> met_of<float>(const Blk& b, int m, int q) { return b.metf[m][q]; }
 __device__ __forceinline__ void put_F(const Blk& b, int d, int m, size_t s, double v) { b.F[d][m][s] = v; }
 __device__ __forceinline__ void put_F(const Blk& b, int d, int m, size_t s, float v) { b.Ff[d][m][s] = v; }
 __device__ __forceinline__ void put_Fv(const Blk& b, int d, int m, size_t s, double v) { b.Fv[d][m][s] = v; }
 __device__ __forceinline__ void put_Fv(const Blk& b, int d, int m, size_t s, float v) { b.Fvf[d][m][s] = v; }
 __device__ __forceinline__ void put_Fsa(const Blk& b, int d, int m, size_t s, double v) { b.Fsa[d][m][s] = v; }
 __device__ __forceinline__ void put_Fsa(const Blk& b, int d, int m, size_t s, float v) { b.Fsaf[d][m][s] = v; }
-template <typename T> __device__ __forceinline__ double get_F(const Blk& b, int d, int m, size_t s) {
-    if constexpr (sizeof(T) == 8) return b.F[d][m][s]; else return (double)b.Ff[d][m][s];
+template <typename T> __device__ __forceinline__ double get_F(const Blk& b, int d, int m, size_t s, long o) {
+    if constexpr (sizeof(T) == 8) return b.F[d][m].at(o)[s]; else return (double)b.Ff[d][m].at(o)[s];
 }
-template <typename T> __device__ __forceinline__ double get_Fv(const Blk& b, int d, int m, size_t s) {
-    if constexpr (sizeof(T) == 8) return b.Fv[d][m][s]; else return (double)b.Fvf[d][m][s];
+template <typename T> __device__ __forceinline__ double get_Fv(const Blk& b, int d, int m, size_t s, long o) {
+    if constexpr (sizeof(T) == 8) return b.Fv[d][m].at(o)[s]; else return (double)b.Fvf[d][m].at(o)[s];
 }
-template <typename T> __device__ __forceinline__ double get_Fsa(const Blk& b, int d, int m, size_t s) {
-    if constexpr (sizeof(T) == 8) return b.Fsa[d][m][s]; else return (double)b.Fsaf[d][m][s];
+template <typename T> __device__ __forceinline__ double get_Fsa(const Blk& b, int d, int m, size_t s, long o) {
+    if constexpr (sizeof(T) == 8) return b.Fsa[d][m].at(o)[s]; else return (double)b.Fsaf[d][m].at(o)[s];
 }
 
 // SA constants (sub_turbulence_SA.f90:18-33)
@@ -152,42 +153,45 @@ struct SAc {
 };
 
 // nu-tilde face flux of the SA equation on face (fi,fj,fk) of direction DIR (I-1/2 convention):
+// a face's normal, area and metrics
+template <typename T> struct FaceGeo { T n[3], S, m[9]; };
+
 // fv = (-upwind convection + (1+cb2)/sigma (vt+mu/rho)/Re grad(vt).n) S and f2 = grad(vt).n S
 // (sub_turbulence_SA.f90:60-174)
 template <int DIR, typename T>
-__device__ __forceinline__ void sa_face(const Blk& b, const Par& p, int fi, int fj, int fk, T& fv, T& f2) {
+__device__ __forceinline__ void sa_face(const Blk& b, const Par& p, const FaceGeo<T>& g, int fi, int fj, int fk, T& fv, T& f2) {
     constexpr int di = DIR == 0, dj = DIR == 1, dk = DIR == 2;
     const T c_v0 = T((0.5 * (1.0 + SAc::Cb2)) / SAc::sigma);
     const T Re = T(p.Re);
-    const T* d = prim_of<T>(b, 0);
-    const T *uu = prim_of<T>(b, 1), *vv = prim_of<T>(b, 2), *ww = prim_of<T>(b, 3);
-    size_t f = IX(b, fi, fj, fk), fm = IX(b, fi - di, fj - dj, fk - dk);
-    T s1x = nv_of<T>(b, 3 * DIR)[f], s1y = nv_of<T>(b, 3 * DIR + 1)[f], s1z = nv_of<T>(b, 3 * DIR + 2)[f];
+    const gptr<T> d = prim_of<T>(b, 0), uu = prim_of<T>(b, 1), vv = prim_of<T>(b, 2), ww = prim_of<T>(b, 3);
+    const size_t f = IX(b, fi, fj, fk);
+    const long m = -OFF(b, di, dj, dk);
+    T s1x = g.n[0], s1y = g.n[1], s1z = g.n[2];
     T gi, gj, gk;
-    auto VT = [&](int a, int bb, int cc) { return T(vt_of(b, IX(b, a, bb, cc))); };
+    auto VT = [&](int a, int bb, int cc) { return T(vt_of(b, f, OFF(b, a, bb, cc))); };
     if (DIR == 0) {
-        gi = VT(fi, fj, fk) - VT(fi - 1, fj, fk);
-        gj = T(0.25) * (((VT(fi, fj + 1, fk) - VT(fi, fj - 1, fk)) + VT(fi - 1, fj + 1, fk)) - VT(fi - 1, fj - 1, fk));
-        gk = T(0.25) * (((VT(fi, fj, fk + 1) - VT(fi, fj, fk - 1)) + VT(fi - 1, fj, fk + 1)) - VT(fi - 1, fj, fk - 1));
+        gi = VT(0, 0, 0) - VT(-1, 0, 0);
+        gj = T(0.25) * (((VT(0, 1, 0) - VT(0, -1, 0)) + VT(-1, 1, 0)) - VT(-1, -1, 0));
+        gk = T(0.25) * (((VT(0, 0, 1) - VT(0, 0, -1)) + VT(-1, 0, 1)) - VT(-1, 0, -1));
     } else if (DIR == 1) {
-        gi = T(0.25) * (((VT(fi + 1, fj, fk) - VT(fi - 1, fj, fk)) + VT(fi + 1, fj - 1, fk)) - VT(fi - 1, fj - 1, fk));
-        gj = VT(fi, fj, fk) - VT(fi, fj - 1, fk);
-        gk = T(0.25) * (((VT(fi, fj, fk + 1) - VT(fi, fj, fk - 1)) + VT(fi, fj - 1, fk + 1)) - VT(fi, fj - 1, fk - 1));
+        gi = T(0.25) * (((VT(1, 0, 0) - VT(-1, 0, 0)) + VT(1, -1, 0)) - VT(-1, -1, 0));
+        gj = VT(0, 0, 0) - VT(0, -1, 0);
+        gk = T(0.25) * (((VT(0, 0, 1) - VT(0, 0, -1)) + VT(0, -1, 1)) - VT(0, -1, -1));
     } else {
-        gi = T(0.25) * (((VT(fi + 1, fj, fk) - VT(fi - 1, fj, fk)) + VT(fi + 1, fj, fk - 1)) - VT(fi - 1, fj, fk - 1));
-        gj = T(0.25) * (((VT(fi, fj + 1, fk) - VT(fi, fj - 1, fk)) + VT(fi, fj + 1, fk - 1)) - VT(fi, fj - 1, fk - 1));
-        gk = VT(fi, fj, fk) - VT(fi, fj, fk - 1);
+        gi = T(0.25) * (((VT(1, 0, 0) - VT(-1, 0, 0)) + VT(1, 0, -1)) - VT(-1, 0, -1));
+        gj = T(0.25) * (((VT(0, 1, 0) - VT(0, -1, 0)) + VT(0, 1, -1)) - VT(0, -1, -1));
+        gk = VT(0, 0, 0) - VT(0, 0, -1);
     }
-    auto M = [&](int q) { return met_of<T>(b, DIR + 1, q)[f]; };
+    auto M = [&](int q) { return g.m[q]; };
     T vtx = (gi * M(0) + gj * M(3)) + gk * M(6);
     T vty = (gi * M(1) + gj * M(4)) + gk * M(7);
     T vtz = (gi * M(2) + gj * M(5)) + gk * M(8);
-    T v0 = c_v0 * (((T(vt_of(b, f)) + (T(b.mu[f]) * Re) / d[f]) + T(vt_of(b, fm))) + (T(b.mu[fm]) * Re) / d[fm]);
-    T vn1 = (uu[fm] * s1x + vv[fm] * s1y) + ww[fm] * s1z;
+    T v0 = c_v0 * (((T(vt_of(b, f, 0)) + (T(b.mu[f]) * Re) / d[f]) + T(vt_of(b, f, m))) + (T(b.mu.at(m)[f]) * Re) / d.at(m)[f]);
+    T vn1 = (uu.at(m)[f] * s1x + vv.at(m)[f] * s1y) + ww.at(m)[f] * s1z;
     T vn2 = (uu[f] * s1x + vv[f] * s1y) + ww[f] * s1z;
-    T vfi = T(0.5) * ((vn1 + fabs(vn1)) * T(vt_of(b, fm)) + (vn2 - fabs(vn2)) * T(vt_of(b, f)));
+    T vfi = T(0.5) * ((vn1 + fabs(vn1)) * T(vt_of(b, f, m)) + (vn2 - fabs(vn2)) * T(vt_of(b, f, 0)));
     T gn = (vtx * s1x + vty * s1y) + vtz * s1z;
-    T Sf = S_of<T>(b, DIR)[f];
+    T Sf = g.S;
     fv = (-vfi + (v0 / Re) * gn) * Sf;
     f2 = gn * Sf;
 }
@@ -199,26 +203,25 @@ __device__ __forceinline__ double sa_residual(const Blk& b, const Par& p, int i,
     const double Cw1 = SAc::Cb1 / (SAc::k * SAc::k) + (1.0 + SAc::Cb2) / SAc::sigma;
     const double Cv1_3 = pw3(7.1), Cw3_6 = pw6(SAc::Cw3);
     const double Re = p.Re;
-    const double* d = b.prim[0];
-    const T* dt_ = prim_of<T>(b, 0);
-    const T *ut = prim_of<T>(b, 1), *vtt = prim_of<T>(b, 2), *wt = prim_of<T>(b, 3);
-    double vt_c = vt_of(b, s), mu_c = b.mu[s] * Re;
+    const gptr<double> d = b.prim[0];
+    const gptr<T> dt_ = prim_of<T>(b, 0), ut = prim_of<T>(b, 1), vtt = prim_of<T>(b, 2), wt = prim_of<T>(b, 3);
+    double vt_c = vt_of(b, s, 0), mu_c = b.mu[s] * Re;
     double v0c = ((vt_c + mu_c / d[s]) * SAc::Cb2) / SAc::sigma;
-    const size_t sp[3] = {s + 1, s + (size_t)b.NI, s + (size_t)b.NI * b.NJ};
+    const long sp[3] = {1, OFF(b, 0, 1, 0), OFF(b, 0, 0, 1)};
     double res = 0.0;
 #pragma unroll
     for (int dir = 0; dir < 3; dir++) {
-        double fv0 = get_Fsa<T>(b, dir, 0, s), fv1 = get_Fsa<T>(b, dir, 0, sp[dir]);
-        double f20 = get_Fsa<T>(b, dir, 1, s), f21 = get_Fsa<T>(b, dir, 1, sp[dir]);
+        double fv0 = get_Fsa<T>(b, dir, 0, s, 0), fv1 = get_Fsa<T>(b, dir, 0, s, sp[dir]);
+        double f20 = get_Fsa<T>(b, dir, 1, s, 0), f21 = get_Fsa<T>(b, dir, 1, s, sp[dir]);
         if (dir == 0) res = (fv1 - fv0) - (v0c / Re) * (f21 - f20);
         else res = ((res + fv1) - fv0) - (v0c / Re) * (f21 - f20);
     }
-    auto UU = [&](int a, int bb, int cc) { return ut[IX(b, a, bb, cc)]; };
-    auto VV = [&](int a, int bb, int cc) { return vtt[IX(b, a, bb, cc)]; };
-    auto WW = [&](int a, int bb, int cc) { return wt[IX(b, a, bb, cc)]; };
-    T ui = UU(i + 1, j, k) - UU(i - 1, j, k), vi = VV(i + 1, j, k) - VV(i - 1, j, k), wi = WW(i + 1, j, k) - WW(i - 1, j, k);
-    T uj = UU(i, j + 1, k) - UU(i, j - 1, k), vj = VV(i, j + 1, k) - VV(i, j - 1, k), wj = WW(i, j + 1, k) - WW(i, j - 1, k);
-    T uk = UU(i, j, k + 1) - UU(i, j, k - 1), vk = VV(i, j, k + 1) - VV(i, j, k - 1), wk = WW(i, j, k + 1) - WW(i, j, k - 1);
+    auto UU = [&](int a, int bb, int cc) { return ut.at(OFF(b, a, bb, cc))[s]; };
+    auto VV = [&](int a, int bb, int cc) { return vtt.at(OFF(b, a, bb, cc))[s]; };
+    auto WW = [&](int a, int bb, int cc) { return wt.at(OFF(b, a, bb, cc))[s]; };
+    T ui = UU(1, 0, 0) - UU(-1, 0, 0), vi = VV(1, 0, 0) - VV(-1, 0, 0), wi = WW(1, 0, 0) - WW(-1, 0, 0);
+    T uj = UU(0, 1, 0) - UU(0, -1, 0), vj = VV(0, 1, 0) - VV(0, -1, 0), wj = WW(0, 1, 0) - WW(0, -1, 0);
+    T uk = UU(0, 0, 1) - UU(0, 0, -1), vk = VV(0, 0, 1) - VV(0, 0, -1), wk = WW(0, 0, 1) - WW(0, 0, -1);
     auto M0 = [&](int q) { return met_of<T>(b, 0, q)[s]; };
     T ix = M0(0), iy = M0(1), iz = M0(2), jx = M0(3), jy = M0(4), jz = M0(5), kx = M0(6), ky = M0(7), kz = M0(8);
     T vx = (vi * ix + vj * jx) + vk * kx, wx = (wi * ix + wj * jx) + wk * kx;
@@ -263,9 +266,6 @@ __global__ void __launch_bounds__(64) k_amut(SubSet S) {
 // ---------------------------------------------------------------------------------------------
 // Menter SST (sub_turbulence_SST.f90:7-348).  f1 on the last face of each direction reads the
 // never-written cell (nx,.,.)/(.,ny,.)/(.,.,nz); here that storage holds zero.
-// k and omega per unit mass, max(U, 0) / rho, as k_prims stores them for the iteration
-__device__ __forceinline__ double kt_of(const Blk& b, size_t s) { return b.kt[s]; }
-__device__ __forceinline__ double wt_of(const Blk& b, size_t s) { return b.wt[s]; }
 
 // cell pass: mu_t, f1, sources into Res(6:7), in the compute type T (FP64, or FP32 in the mixed
 // mode, where the velocities come from the FP32 primitives); stored in FP64
@@ -275,11 +275,11 @@ __global__ void __launch_bounds__(64) k_sst_cell(BSet S) {
     const T sigma_w2 = T(0.856), beta1 = T(0.075), Cw1s = T(0.533), beta2 = T(0.0828), Cw2s = T(0.440);
     const T a1 = T(0.31), betas = T(0.09), c009 = T((double)0.09f);
     const T Re = T(p.Re);
-    const T *uu = prim_of<T>(b, 1), *vv = prim_of<T>(b, 2), *ww = prim_of<T>(b, 3);
+    const gptr<T> uu = prim_of<T>(b, 1), vv = prim_of<T>(b, 2), ww = prim_of<T>(b, 3);
     size_t s = IX(b, i, j, k);
-    auto DIFF = [&](const T* a, int di, int dj, int dk) { return a[IX(b, i + di, j + dj, k + dk)] - a[IX(b, i - di, j - dj, k - dk)]; };
-    auto DK = [&](int di, int dj, int dk) { return T(kt_of(b, IX(b, i + di, j + dj, k + dk))) - T(kt_of(b, IX(b, i - di, j - dj, k - dk))); };
-    auto DW = [&](int di, int dj, int dk) { return T(wt_of(b, IX(b, i + di, j + dj, k + dk))) - T(wt_of(b, IX(b, i - di, j - dj, k - dk))); };
+    auto DIFF = [&](gptr<T> a, int di, int dj, int dk) { const long o = OFF(b, di, dj, dk); return a.at(o)[s] - a.at(-o)[s]; };
+    auto DK = [&](int di, int dj, int dk) { const long o = OFF(b, di, dj, dk); return T(b.kt.at(o)[s]) - T(b.kt.at(-o)[s]); };
+    auto DW = [&](int di, int dj, int dk) { const long o = OFF(b, di, dj, dk); return T(b.wt.at(o)[s]) - T(b.wt.at(-o)[s]); };
     T ui = DIFF(uu, 1, 0, 0), vi = DIFF(vv, 1, 0, 0), wi = DIFF(ww, 1, 0, 0), kti = DK(1, 0, 0), wti = DW(1, 0, 0);
     T uj = DIFF(uu, 0, 1, 0), vj = DIFF(vv, 0, 1, 0), wj = DIFF(ww, 0, 1, 0), ktj = DK(0, 1, 0), wtj = DW(0, 1, 0);
     T uk = DIFF(uu, 0, 0, 1), vk = DIFF(vv, 0, 0, 1), wk = DIFF(ww, 0, 0, 1), ktk = DK(0, 0, 1), wtk = DW(0, 0, 1);
@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(64) k_sst_cell(BSet S) {
     T uz = (ui * iz + uj * jz) + uk * kz, vz = (vi * iz + vj * jz) + vk * kz;
     T ktz = (kti * iz + ktj * jz) + ktk * kz, wtz = (wti * iz + wtj * jz) + wtk * kz;
     T omega = sqrt((sq(wy - vz) + sq(uz - wx)) + sq(vx - uy));
-    T d = T(b.prim[0][s]), mu = T(b.mu[s] * p.Re), dw = T(b.dw[s]), kt = T(kt_of(b, s)), wt = T(wt_of(b, s));
+    T d = T(b.prim[0][s]), mu = T(b.mu[s] * p.Re), dw = T(b.dw[s]), kt = T(b.kt[s]), wt = T(b.wt[s]);
     T a2a = T(2) * sqrt(fabs(kt)) / (((c009 * wt) * dw) * Re);
     T a2b = (T(500) * mu) / ((((d * wt) * sq(dw)) * Re) * Re);
     T arg2 = a2a > a2b ? a2a : a2b;
@@ -348,49 +348,49 @@ template <int DIR, typename T>
 __device__ __forceinline__ void sst_face(const Blk& b, const Par& p, int i, int j, int k) {
     const T sigma_k1 = T(0.85), sigma_w1 = T(0.5), sigma_k2 = T(1.0), sigma_w2 = T(0.856);
     const T Re = T(p.Re);
-    const T *uu = prim_of<T>(b, 1), *vv = prim_of<T>(b, 2), *ww = prim_of<T>(b, 3);
-    const int di = DIR == 0, dj = DIR == 1, dk = DIR == 2;
-    const int fi = i, fj = j, fk_ = k;
-    size_t f = IX(b, fi, fj, fk_), fm = IX(b, fi - di, fj - dj, fk_ - dk);
+    const gptr<T> uu = prim_of<T>(b, 1), vv = prim_of<T>(b, 2), ww = prim_of<T>(b, 3);
+    constexpr int di = DIR == 0, dj = DIR == 1, dk = DIR == 2;
+    const size_t f = IX(b, i, j, k);
+    const long m = -OFF(b, di, dj, dk);
     T f1 = T(b.aux[f]);
     T skk = f1 * sigma_k1 + (T(1) - f1) * sigma_k2, sww = f1 * sigma_w1 + (T(1) - f1) * sigma_w2;
-    T mua = T(b.mu[fm] * p.Re), mub = T(b.mu[f] * p.Re), mta = T(b.mut[fm]), mtb = T(b.mut[f]);
+    T mua = T(b.mu.at(m)[f] * p.Re), mub = T(b.mu[f] * p.Re), mta = T(b.mut.at(m)[f]), mtb = T(b.mut[f]);
     T muk = (((mua + mub) + skk * (mta + mtb)) * T(0.5)) / Re;
     T muw = (((mua + mub) + sww * (mta + mtb)) * T(0.5)) / Re;
-    auto K = [&](int a, int bb, int cc) { return T(kt_of(b, IX(b, a, bb, cc))); };
-    auto W = [&](int a, int bb, int cc) { return T(wt_of(b, IX(b, a, bb, cc))); };
+    auto K = [&](int a, int bb, int cc) { return T(b.kt.at(OFF(b, a, bb, cc))[f]); };
+    auto W = [&](int a, int bb, int cc) { return T(b.wt.at(OFF(b, a, bb, cc))[f]); };
     const T q = T(0.25);
     T kti, ktj, ktk, wti, wtj, wtk;
     if constexpr (DIR == 0) {
-        kti = K(fi, fj, fk_) - K(fi - 1, fj, fk_); wti = W(fi, fj, fk_) - W(fi - 1, fj, fk_);
-        ktj = q * (((K(fi, fj + 1, fk_) - K(fi, fj - 1, fk_)) + K(fi - 1, fj + 1, fk_)) - K(fi - 1, fj - 1, fk_));
-        wtj = q * (((W(fi, fj + 1, fk_) - W(fi, fj - 1, fk_)) + W(fi - 1, fj + 1, fk_)) - W(fi - 1, fj - 1, fk_));
-        ktk = q * (((K(fi, fj, fk_ + 1) - K(fi, fj, fk_ - 1)) + K(fi - 1, fj, fk_ + 1)) - K(fi - 1, fj, fk_ - 1));
-        wtk = q * (((W(fi, fj, fk_ + 1) - W(fi, fj, fk_ - 1)) + W(fi - 1, fj, fk_ + 1)) - W(fi - 1, fj, fk_ - 1));
+        kti = K(0, 0, 0) - K(-1, 0, 0); wti = W(0, 0, 0) - W(-1, 0, 0);
+        ktj = q * (((K(0, 1, 0) - K(0, -1, 0)) + K(-1, 1, 0)) - K(-1, -1, 0));
+        wtj = q * (((W(0, 1, 0) - W(0, -1, 0)) + W(-1, 1, 0)) - W(-1, -1, 0));
+        ktk = q * (((K(0, 0, 1) - K(0, 0, -1)) + K(-1, 0, 1)) - K(-1, 0, -1));
+        wtk = q * (((W(0, 0, 1) - W(0, 0, -1)) + W(-1, 0, 1)) - W(-1, 0, -1));
     } else if constexpr (DIR == 1) {
-        kti = q * (((K(fi + 1, fj, fk_) - K(fi - 1, fj, fk_)) + K(fi + 1, fj - 1, fk_)) - K(fi - 1, fj - 1, fk_));
-        ktj = K(fi, fj, fk_) - K(fi, fj - 1, fk_);
-        ktk = q * (((K(fi, fj, fk_ + 1) - K(fi, fj, fk_ - 1)) + K(fi, fj - 1, fk_ + 1)) - K(fi, fj - 1, fk_ - 1));
-        wti = q * (((W(fi + 1, fj, fk_) - W(fi - 1, fj, fk_)) + W(fi + 1, fj - 1, fk_)) - W(fi - 1, fj - 1, fk_));
-        wtj = W(fi, fj, fk_) - W(fi, fj - 1, fk_);
-        wtk = q * (((W(fi, fj, fk_ + 1) - W(fi, fj, fk_ - 1)) + W(fi, fj - 1, fk_ + 1)) - W(fi, fj - 1, fk_ - 1));
+        kti = q * (((K(1, 0, 0) - K(-1, 0, 0)) + K(1, -1, 0)) - K(-1, -1, 0));
+        ktj = K(0, 0, 0) - K(0, -1, 0);
+        ktk = q * (((K(0, 0, 1) - K(0, 0, -1)) + K(0, -1, 1)) - K(0, -1, -1));
+        wti = q * (((W(1, 0, 0) - W(-1, 0, 0)) + W(1, -1, 0)) - W(-1, -1, 0));
+        wtj = W(0, 0, 0) - W(0, -1, 0);
+        wtk = q * (((W(0, 0, 1) - W(0, 0, -1)) + W(0, -1, 1)) - W(0, -1, -1));
     } else {
-        kti = q * (((K(fi + 1, fj, fk_) - K(fi - 1, fj, fk_)) + K(fi + 1, fj, fk_ - 1)) - K(fi - 1, fj, fk_ - 1));
-        ktj = q * (((K(fi, fj + 1, fk_) - K(fi, fj - 1, fk_)) + K(fi, fj + 1, fk_ - 1)) - K(fi, fj - 1, fk_ - 1));
-        ktk = K(fi, fj, fk_) - K(fi, fj, fk_ - 1);
-        wti = q * (((W(fi + 1, fj, fk_) - W(fi - 1, fj, fk_)) + W(fi + 1, fj, fk_ - 1)) - W(fi - 1, fj, fk_ - 1));
-        wtj = q * (((W(fi, fj + 1, fk_) - W(fi, fj - 1, fk_)) + W(fi, fj + 1, fk_ - 1)) - W(fi, fj - 1, fk_ - 1));
-        wtk = W(fi, fj, fk_) - W(fi, fj, fk_ - 1);
+        kti = q * (((K(1, 0, 0) - K(-1, 0, 0)) + K(1, 0, -1)) - K(-1, 0, -1));
+        ktj = q * (((K(0, 1, 0) - K(0, -1, 0)) + K(0, 1, -1)) - K(0, -1, -1));
+        ktk = K(0, 0, 0) - K(0, 0, -1);
+        wti = q * (((W(1, 0, 0) - W(-1, 0, 0)) + W(1, 0, -1)) - W(-1, 0, -1));
+        wtj = q * (((W(0, 1, 0) - W(0, -1, 0)) + W(0, 1, -1)) - W(0, -1, -1));
+        wtk = W(0, 0, 0) - W(0, 0, -1);
     }
     auto M = [&](int c) { return met_of<T>(b, DIR + 1, c)[f]; };
     T ktx = (kti * M(0) + ktj * M(3)) + ktk * M(6), wtx = (wti * M(0) + wtj * M(3)) + wtk * M(6);
     T kty = (kti * M(1) + ktj * M(4)) + ktk * M(7), wty = (wti * M(1) + wtj * M(4)) + wtk * M(7);
     T ktz = (kti * M(2) + ktj * M(5)) + ktk * M(8), wtz = (wti * M(2) + wtj * M(5)) + wtk * M(8);
     T s1x = nv_of<T>(b, 3 * DIR)[f], s1y = nv_of<T>(b, 3 * DIR + 1)[f], s1z = nv_of<T>(b, 3 * DIR + 2)[f];
-    T vn1 = (uu[fm] * s1x + vv[fm] * s1y) + ww[fm] * s1z;
+    T vn1 = (uu.at(m)[f] * s1x + vv.at(m)[f] * s1y) + ww.at(m)[f] * s1z;
     T vn2 = (uu[f] * s1x + vv[f] * s1y) + ww[f] * s1z;
-    T kfi = T(0.5) * ((vn1 + fabs(vn1)) * K(fi - di, fj - dj, fk_ - dk) + (vn2 - fabs(vn2)) * K(fi, fj, fk_));
-    T wfi = T(0.5) * ((vn1 + fabs(vn1)) * W(fi - di, fj - dj, fk_ - dk) + (vn2 - fabs(vn2)) * W(fi, fj, fk_));
+    T kfi = T(0.5) * ((vn1 + fabs(vn1)) * K(-di, -dj, -dk) + (vn2 - fabs(vn2)) * K(0, 0, 0));
+    T wfi = T(0.5) * ((vn1 + fabs(vn1)) * W(-di, -dj, -dk) + (vn2 - fabs(vn2)) * W(0, 0, 0));
     T Sf = S_of<T>(b, DIR)[f];
     b.Fsa[DIR][0][f] = (double)((-kfi + muk * ((ktx * s1x + kty * s1y) + ktz * s1z)) * Sf);
     b.Fsa[DIR][1][f] = (double)((-wfi + muw * ((wtx * s1x + wty * s1y) + wtz * s1z)) * Sf);
@@ -414,12 +414,12 @@ __global__ void __launch_bounds__(64) k_sst_res(BSet S) {
     OCFD_LOCATE(SP_N0)
     size_t s = IX(b, i, j, k);
     if (i >= 1 && i <= b.nx - 1 && j >= 1 && j <= b.ny - 1 && k >= 1 && k <= b.nz - 1) {
-        const size_t sp[3] = {s + 1, s + (size_t)b.NI, s + (size_t)b.NI * b.NJ};
+        const long sp[3] = {1, OFF(b, 0, 1, 0), OFF(b, 0, 0, 1)};
         double r6 = b.Res[5][s], r7 = b.Res[6][s];
 #pragma unroll
         for (int dir = 0; dir < 3; dir++) {
-            r6 = (r6 + b.Fsa[dir][0][sp[dir]]) - b.Fsa[dir][0][s];
-            r7 = (r7 + b.Fsa[dir][1][sp[dir]]) - b.Fsa[dir][1][s];
+            r6 = (r6 + b.Fsa[dir][0].at(sp[dir])[s]) - b.Fsa[dir][0][s];
+            r7 = (r7 + b.Fsa[dir][1].at(sp[dir])[s]) - b.Fsa[dir][1][s];
         }
         b.Res[5][s] = r6;
         b.Res[6][s] = r7;
@@ -449,7 +449,7 @@ __device__ __forceinline__ void riemann_t(const T* QL, const T* QR, T* F, T gamm
 
 // flux_inviscous_i/j/k (sub_Residual.f90:182-705) of face (i,j,k) of direction DIR, stored
 template <int DIR, typename T, int RECON, int FLUX>
-__device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int j, int k) {
+__device__ __forceinline__ void inv_face(const Blk& b, const Par& p, const FaceGeo<T>& g, int i, int j, int k) {
     size_t s = IX(b, i, j, k);
     int pos = DIR == 0 ? i : DIR == 1 ? j : k;
     int nd = DIR == 0 ? b.nx : DIR == 1 ? b.ny : b.nz;
@@ -458,12 +458,12 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int 
     if (fl & BCF_PHYS) { if (pos == 1) scheme = S_CD2; else if (pos < LAP) scheme = p.bscheme; }
     if (fl & BCF_PHYS << 1) { if (pos == nd) scheme = S_CD2; else if (pos > nd - LAP + 1) scheme = p.bscheme; }
     if (b.flags[0] == 1) scheme = S_UD1;
-    T s1x = nv_of<T>(b, 3 * DIR)[s], s1y = nv_of<T>(b, 3 * DIR + 1)[s], s1z = nv_of<T>(b, 3 * DIR + 2)[s];
+    T s1x = g.n[0], s1y = g.n[1], s1z = g.n[2];
     T t1x, t1y, t1z;
     if constexpr (std::is_same<T, float>::value) { t1x = b.t1f[DIR][0][s]; t1y = b.t1f[DIR][1][s]; t1z = b.t1f[DIR][2][s]; }
-    else if (DIR == 0) { size_t a = IX(b, i, j + 1, k), c = IX(b, i, j, k + 1); t1x = T(b.x[a] - b.x[c]); t1y = T(b.y[a] - b.y[c]); t1z = T(b.z[a] - b.z[c]); }
-    else if (DIR == 1) { size_t a = IX(b, i + 1, j, k + 1); t1x = T(b.x[a] - b.x[s]); t1y = T(b.y[a] - b.y[s]); t1z = T(b.z[a] - b.z[s]); }
-    else { size_t a = IX(b, i + 1, j + 1, k); t1x = T(b.x[a] - b.x[s]); t1y = T(b.y[a] - b.y[s]); t1z = T(b.z[a] - b.z[s]); }
+    else if (DIR == 0) { const long a = OFF(b, 0, 1, 0), c = OFF(b, 0, 0, 1); t1x = T(b.x.at(a)[s] - b.x.at(c)[s]); t1y = T(b.y.at(a)[s] - b.y.at(c)[s]); t1z = T(b.z.at(a)[s] - b.z.at(c)[s]); }
+    else if (DIR == 1) { const long a = OFF(b, 1, 0, 1); t1x = T(b.x.at(a)[s] - b.x[s]); t1y = T(b.y.at(a)[s] - b.y[s]); t1z = T(b.z.at(a)[s] - b.z[s]); }
+    else { const long a = OFF(b, 1, 1, 0); t1x = T(b.x.at(a)[s] - b.x[s]); t1y = T(b.y.at(a)[s] - b.y[s]); t1z = T(b.z.at(a)[s] - b.z[s]); }
     T t10 = T(1) / sqrt((t1x * t1x + t1y * t1y) + t1z * t1z);
     T s2x = t1x * t10, s2y = t1y * t10, s2z = t1z * t10;
     T s3x = s1y * s2z - s1z * s2y, s3y = s1z * s2x - s1x * s2z, s3z = s1x * s2y - s1y * s2x;
@@ -471,10 +471,10 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int 
     T UL[5], UR[5];
     if constexpr (RECON == 0) {
         for (int m = 0; m < 5; m++) {
-            const T* a = prim_of<T>(b, m) + s;
+            const gptr<T> a = prim_of<T>(b, m);
             T u[8];
 #pragma unroll
-            for (int q = 0; q < 8; q++) u[q] = a[(q - 4) * st];     // u[q] = cell (face - 4 + q): u(q-3)
+            for (int q = 0; q < 8; q++) u[q] = a.at((q - 4) * st)[s];     // u[q] = cell (face - 4 + q): u(q-3)
             UL[m] = scheme_fP(u + 3, scheme);
             UR[m] = scheme_fm(u + 3, scheme);
         }
@@ -535,7 +535,7 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, int i, int 
     QR[0] = UR[0]; QR[1] = (UR[1] * s1x + UR[2] * s1y) + UR[3] * s1z; QR[2] = (UR[1] * s2x + UR[2] * s2y) + UR[3] * s2z;
     QR[3] = (UR[1] * s3x + UR[2] * s3y) + UR[3] * s3z; QR[4] = UR[4];
     riemann_t<FLUX, T>(QL, QR, F0, T(p.gamma), p.flux);
-    T Sf = S_of<T>(b, DIR)[s];
+    T Sf = g.S;
     put_F(b, DIR, 0, s, -F0[0] * Sf);
     put_F(b, DIR, 1, s, -((F0[1] * s1x + F0[2] * s2x) + F0[3] * s3x) * Sf);
     put_F(b, DIR, 2, s, -((F0[1] * s1y + F0[2] * s2y) + F0[3] * s3y) * Sf);
@@ -572,7 +572,7 @@ __global__ void __launch_bounds__(64) k_inv_kbc(SubSet S) {
 
 // flux_viscous_i/j/k (sub_Residual.f90:712-1247) of face (i,j,k) of direction DIR, stored
 template <int DIR, typename T>
-__device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int j, int k) {
+__device__ __forceinline__ void visc_face(const Blk& b, const Par& p, const FaceGeo<T>& g, int i, int j, int k) {
     constexpr int di = DIR == 0, dj = DIR == 1, dk = DIR == 2;
     const T tmp1 = T(4.0 / 3.0), tmp2 = T(2.0 / 3.0);
     size_t s = IX(b, i, j, k);
@@ -580,17 +580,17 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int
         int pos0 = DIR == 0 ? i : DIR == 1 ? j : k, nd0 = DIR == 0 ? b.nx : DIR == 1 ? b.ny : b.nz;
         if (pos0 == 1 || pos0 == nd0) {
             int f = DIR + (pos0 == 1 ? 0 : 3);
-            size_t m = DIR == 0 ? JK(b, j, k) : DIR == 1 ? IK(b, i, k) : IJ(b, i, j);
-            b.surf[f][0][m] = 0.0; b.surf[f][1][m] = 0.0; b.surf[f][2][m] = 0.0;
+            size_t r = DIR == 0 ? JK(b, j, k) : DIR == 1 ? IK(b, i, k) : IJ(b, i, j);
+            b.surf[f][0][r] = 0.0; b.surf[f][1][r] = 0.0; b.surf[f][2][r] = 0.0;
         }
         return;
     }
-    int im = i - di, jm = j - dj, km = k - dk;
-    size_t sm = IX(b, im, jm, km);
-    const T* Q[4] = {prim_of<T>(b, 1), prim_of<T>(b, 2), prim_of<T>(b, 3), prim_of<T>(b, 5)};
+    const long m = -OFF(b, di, dj, dk);
+    const gptr<T> Q[4] = {prim_of<T>(b, 1), prim_of<T>(b, 2), prim_of<T>(b, 3), prim_of<T>(b, 5)};
     // tangential directions: i-faces (j,k), j-faces (i,k), k-faces (i,j)
     constexpr int ai = DIR == 0 ? 0 : 1, aj = DIR == 0 ? 1 : 0;          // first tangential unit step
     constexpr int bj = DIR == 2 ? 1 : 0, bk = DIR == 2 ? 0 : 1;          // second tangential unit step
+    const long oa = OFF(b, ai, aj, 0), ob = OFF(b, 0, bj, bk);
     int pos = DIR == 0 ? i : DIR == 1 ? j : k;
     int nd = DIR == 0 ? b.nx : DIR == 1 ? b.ny : b.nz;
     int posA = DIR == 0 ? j : i, nA = DIR == 0 ? b.ny : b.nx;
@@ -600,23 +600,23 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int
     T gi[4], gj[4], gk[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const T* a = Q[q];
-        T dn = a[s] - a[sm];
+        const gptr<T> a = Q[q];
+        T dn = a[s] - a.at(m)[s];
         T ta1 = T(0), ta2 = T(0), tb1 = T(0), tb2 = T(0);
         if (!zeroA) {
-            ta1 = T(0.5) * (a[IX(b, i - ai, j - aj, k)] + a[IX(b, im - ai, jm - aj, km)]);
-            ta2 = T(0.5) * (a[IX(b, i + ai, j + aj, k)] + a[IX(b, im + ai, jm + aj, km)]);
+            ta1 = T(0.5) * (a.at(-oa)[s] + a.at(m - oa)[s]);
+            ta2 = T(0.5) * (a.at(oa)[s] + a.at(m + oa)[s]);
         }
         if (!zeroB) {
-            tb1 = T(0.5) * (a[IX(b, i, j - bj, k - bk)] + a[IX(b, im, jm - bj, km - bk)]);
-            tb2 = T(0.5) * (a[IX(b, i, j + bj, k + bk)] + a[IX(b, im, jm + bj, km + bk)]);
+            tb1 = T(0.5) * (a.at(-ob)[s] + a.at(m - ob)[s]);
+            tb2 = T(0.5) * (a.at(ob)[s] + a.at(m + ob)[s]);
         }
         T ga = T(0.5) * (ta2 - ta1), gb = T(0.5) * (tb2 - tb1);
         if (DIR == 0) { gi[q] = dn; gj[q] = ga; gk[q] = gb; }
         else if (DIR == 1) { gi[q] = ga; gj[q] = dn; gk[q] = gb; }
         else { gi[q] = ga; gj[q] = gb; gk[q] = dn; }
     }
-    auto M = [&](int q) { return met_of<T>(b, DIR + 1, q)[s]; };
+    auto M = [&](int q) { return g.m[q]; };
     T ix = M(0), iy = M(1), iz = M(2), jx = M(3), jy = M(4), jz = M(5), kx = M(6), ky = M(7), kz = M(8);
     T ux = (gi[0] * ix + gj[0] * jx) + gk[0] * kx, vx = (gi[1] * ix + gj[1] * jx) + gk[1] * kx;
     T wx = (gi[2] * ix + gj[2] * jx) + gk[2] * kx, Tx = (gi[3] * ix + gj[3] * jx) + gk[3] * kx;
@@ -624,18 +624,18 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int
     T wy = (gi[2] * iy + gj[2] * jy) + gk[2] * ky, Ty = (gi[3] * iy + gj[3] * jy) + gk[3] * ky;
     T uz = (gi[0] * iz + gj[0] * jz) + gk[0] * kz, vz = (gi[1] * iz + gj[1] * jz) + gk[1] * kz;
     T wz = (gi[2] * iz + gj[2] * jz) + gk[2] * kz, Tz = (gi[3] * iz + gj[3] * jz) + gk[3] * kz;
-    T mua = T(b.muf[s]), mub = T(b.muf[sm]), mta = T(b.mut[s]), mtb = T(b.mut[sm]);
+    T mua = T(b.muf[s]), mub = T(b.muf.at(m)[s]), mta = T(b.mut[s]), mtb = T(b.mut.at(m)[s]);
     T mu0 = T(0.5) * (((mua + mta) + mub) + mtb);
     T PrL = T(p.PrL), PrT = T(p.PrT);
     T k0 = (T(0.5) * T(p.Cp)) * (((mua / PrL + mta / PrT) + mub / PrL) + mtb / PrT);
     T s11 = mu0 * (tmp1 * ux - tmp2 * (vy + wz)), s12 = mu0 * (uy + vx), s13 = mu0 * (uz + wx);
     T s22 = mu0 * (tmp1 * vy - tmp2 * (ux + wz)), s23 = mu0 * (vz + wy), s33 = mu0 * (tmp1 * wz - tmp2 * (ux + vy));
-    T u1 = (Q[0][s] + Q[0][sm]) * T(0.5), v1 = (Q[1][s] + Q[1][sm]) * T(0.5), w1 = (Q[2][s] + Q[2][sm]) * T(0.5);
+    T u1 = (Q[0][s] + Q[0].at(m)[s]) * T(0.5), v1 = (Q[1][s] + Q[1].at(m)[s]) * T(0.5), w1 = (Q[2][s] + Q[2].at(m)[s]) * T(0.5);
     T E1 = ((u1 * s11 + v1 * s12) + w1 * s13) + k0 * Tx;
     T E2 = ((u1 * s12 + v1 * s22) + w1 * s23) + k0 * Ty;
     T E3 = ((u1 * s13 + v1 * s23) + w1 * s33) + k0 * Tz;
-    T s1x = nv_of<T>(b, 3 * DIR)[s], s1y = nv_of<T>(b, 3 * DIR + 1)[s], s1z = nv_of<T>(b, 3 * DIR + 2)[s];
-    T Sf = S_of<T>(b, DIR)[s];
+    T s1x = g.n[0], s1y = g.n[1], s1z = g.n[2];
+    T Sf = g.S;
     T f1 = ((s11 * s1x + s12 * s1y) + s13 * s1z) * Sf;
     T f2 = ((s12 * s1x + s22 * s1y) + s23 * s1z) * Sf;
     T f3 = ((s13 * s1x + s23 * s1y) + s33 * s1z) * Sf;
@@ -644,35 +644,47 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, int i, int
     // Surf1..6: viscous force on the first and last face of each direction
     if (pos == 1 || pos == nd) {
         int f = DIR + (pos == 1 ? 0 : 3);
-        size_t m = DIR == 0 ? JK(b, j, k) : DIR == 1 ? IK(b, i, k) : IJ(b, i, j);
-        b.surf[f][0][m] = f1; b.surf[f][1][m] = f2; b.surf[f][2][m] = f3;
+        size_t r = DIR == 0 ? JK(b, j, k) : DIR == 1 ? IK(b, i, k) : IJ(b, i, j);
+        b.surf[f][0][r] = f1; b.surf[f][1][r] = f2; b.surf[f][2][r] = f3;
     }
 }
 
-// Every flux through face (i,j,k) of direction DIR, one thread per face: the SA face terms
-// (sub_turbulence_SA.f90:60-174), the inviscid flux and the viscous flux, each stored for the cell
-// pass.  The SA terms go first, so their registers are free again for the reconstruction; the
-// viscous flux, mostly loads of the face's gradient stencil and metrics, overlaps the inviscid
-// flux's arithmetic in the same kernel.
+// Every flux through face (i,j,k) of direction DIR, one thread per face, each stored for the cell
+// pass: the SA face terms (sub_turbulence_SA.f90:60-174), the viscous flux and the inviscid flux.
+// The terms that share the metrics come first and the face's geometry is read once: a wave lives 25
+// us, in which an XCD's L2 is filled three times over, so a second read of a metric or a normal
+// later in the kernel came from memory again (24 blocks with 6.3 M cells: 7.0 -> 4.1 GB read, 2070 ->
+// 1880 us; a batch of 6 with 1.9 M cells 842 -> 737 us; 257x97x33: 264 -> 246).  What bounds it now
+// is FP64 arithmetic: the vector units are busy 64 % of the time at 4 waves per SIMD (118 VGPRs).
+// Slower: the viscous part in workgroups of its own (100 VGPRs, 1980 us; capped for 5 waves 1885),
+// one kernel capped for 5 waves (spills, 2225), non-temporal flux stores and metric loads (1910).
 template <int DIR, typename T, int RECON, int FLUX>
 __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, int k) {
-    if (p.turb == 2) {
-        const size_t s = IX(b, i, j, k);
+    const size_t s = IX(b, i, j, k);
+    FaceGeo<T> g;
+#pragma unroll
+    for (int q = 0; q < 3; q++) g.n[q] = nv_of<T>(b, 3 * DIR + q)[s];
+    g.S = S_of<T>(b, DIR)[s];
+    if (p.visc == 1) {
+#pragma unroll
+        for (int q = 0; q < 9; q++) g.m[q] = met_of<T>(b, DIR + 1, q)[s];
         T fv, f2;
-        sa_face<DIR, T>(b, p, i, j, k, fv, f2);
-        put_Fsa(b, DIR, 0, s, fv);
-        put_Fsa(b, DIR, 1, s, f2);
+        if (p.turb == 2) sa_face<DIR, T>(b, p, g, i, j, k, fv, f2);
+        visc_face<DIR, T>(b, p, g, i, j, k);
+        if (p.turb == 2) {
+            put_Fsa(b, DIR, 0, s, fv);
+            put_Fsa(b, DIR, 1, s, f2);
+        }
     }
     if (DIR == 2 && ((k == 1 && (b.bcf[2][IJ(b, i, j)] & BCF_KBC)) || (k == b.nz && (b.bcf[2][IJ(b, i, j)] & BCF_KBC << 1))))
         inv_kbc<T>(b, p, i, j, k);
-    else inv_face<DIR, T, RECON, FLUX>(b, p, i, j, k);
-    if (p.visc == 1) visc_face<DIR, T>(b, p, i, j, k);
+    else inv_face<DIR, T, RECON, FLUX>(b, p, g, i, j, k);
 }
 // The three directions' faces in one launch.  On small grids, where a direction's tiles do not fill
 // the GPU and a launch costs more than its work, they run side by side (97x33x9 without viscosity:
 // 22 us instead of 37 in three launches; 257x97x33 SA: 271 against 306); on large ones the
 // directions share the primitives in L2 (face_tile; a batch of 6 with 1.9 M cells: 835 against
-// 930 us, 24 blocks with 6.3 M cells: 2090 against 2200).
+// 930 us, 24 blocks with 6.3 M cells: 2090 against 2200, before the metrics were read once).
 template <typename T, int RECON, int FLUX>
 __global__ void __launch_bounds__(64) k_face(FaceSet S) {
     int bi, i, j, k;
@@ -691,17 +703,17 @@ __global__ void __launch_bounds__(64) k_face(FaceSet S) {
 template <typename T, typename ResSink, typename LamSink>
 __device__ __forceinline__ void cell_assemble(const Blk& b, const Par& p, int i, int j, int k, size_t s, ResSink&& res,
                                               LamSink&& lam, double* Lc, double* Lv, double& dt) {
-    size_t sp[3] = {s + 1, s + (size_t)b.NI, s + (size_t)b.NI * b.NJ};
+    const long sp[3] = {1, OFF(b, 0, 1, 0), OFF(b, 0, 0, 1)};
     bool visc = p.visc == 1 && b.flags[0] != 1;
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-        double r = get_F<T>(b, 0, m, sp[0]) - get_F<T>(b, 0, m, s);
-        r = (r + get_F<T>(b, 1, m, sp[1])) - get_F<T>(b, 1, m, s);
-        r = (r + get_F<T>(b, 2, m, sp[2])) - get_F<T>(b, 2, m, s);
+        double r = get_F<T>(b, 0, m, s, sp[0]) - get_F<T>(b, 0, m, s, 0);
+        r = (r + get_F<T>(b, 1, m, s, sp[1])) - get_F<T>(b, 1, m, s, 0);
+        r = (r + get_F<T>(b, 2, m, s, sp[2])) - get_F<T>(b, 2, m, s, 0);
         if (visc && m > 0) {
-            r = (r + get_Fv<T>(b, 0, m - 1, sp[0])) - get_Fv<T>(b, 0, m - 1, s);
-            r = (r + get_Fv<T>(b, 1, m - 1, sp[1])) - get_Fv<T>(b, 1, m - 1, s);
-            r = (r + get_Fv<T>(b, 2, m - 1, sp[2])) - get_Fv<T>(b, 2, m - 1, s);
+            r = (r + get_Fv<T>(b, 0, m - 1, s, sp[0])) - get_Fv<T>(b, 0, m - 1, s, 0);
+            r = (r + get_Fv<T>(b, 1, m - 1, s, sp[1])) - get_Fv<T>(b, 1, m - 1, s, 0);
+            r = (r + get_Fv<T>(b, 2, m - 1, s, sp[2])) - get_Fv<T>(b, 2, m - 1, s, 0);
         }
         res(m, r);
     }
@@ -712,9 +724,9 @@ __device__ __forceinline__ void cell_assemble(const Blk& b, const Par& p, int i,
     double vol = b.vol[s], vol1 = 1.0 / vol;
 #pragma unroll
     for (int dir = 0; dir < 3; dir++) {
-        double un = 0.5 * ((u * (b.nv[3 * dir][s] + b.nv[3 * dir][sp[dir]]) + v * (b.nv[3 * dir + 1][s] + b.nv[3 * dir + 1][sp[dir]]))
-                           + w * (b.nv[3 * dir + 2][s] + b.nv[3 * dir + 2][sp[dir]]));
-        double S0 = (b.S[dir][s] + b.S[dir][sp[dir]]) * 0.5;
+        double un = 0.5 * ((u * (b.nv[3 * dir][s] + b.nv[3 * dir].at(sp[dir])[s]) + v * (b.nv[3 * dir + 1][s] + b.nv[3 * dir + 1].at(sp[dir])[s]))
+                           + w * (b.nv[3 * dir + 2][s] + b.nv[3 * dir + 2].at(sp[dir])[s]));
+        double S0 = (b.S[dir][s] + b.S[dir].at(sp[dir])[s]) * 0.5;
         Lc[dir] = (fabs(un) + c) * S0;
         Lv[dir] = ((D0 * S0) * S0) * vol1;
         lam(dir, Lc[dir], Lv[dir]);

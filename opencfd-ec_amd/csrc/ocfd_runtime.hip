@@ -134,12 +134,12 @@ void* carve(HostBlock& hb, size_t n) {
     return hb.sizing ? nullptr : hb.slab + at;
 }
 
-int dalloc(HostBlock& hb, double** p, size_t n) {
+int dalloc(HostBlock& hb, gptr<double>* p, size_t n) {
     *p = (double*)carve(hb, n * sizeof(double));
     return OCFD_OK;
 }
 
-int balloc(HostBlock& hb, uint8_t** p, size_t n) {
+int balloc(HostBlock& hb, gptr<uint8_t>* p, size_t n) {
     *p = (uint8_t*)carve(hb, n);
     return OCFD_OK;
 }
@@ -155,8 +155,8 @@ int carve_block(ocfd_ctx* c, HostBlock& hb) {
     for (int m = 0; m < NV; m++) {
         if ((r = dalloc(hb, &b.U[m], n)) || (r = dalloc(hb, &b.Res[m], n)) || (r = dalloc(hb, &b.DU[m], n))) return r;
     }
-    double** one[] = {&b.dt, &b.mu, &b.muf, &b.mut, &b.vol, &b.dtm, &b.x, &b.y, &b.z, &b.xc, &b.yc, &b.zc, &b.aux};
-    for (double** q : one) if ((r = dalloc(hb, q, n))) return r;
+    gptr<double>* one[] = {&b.dt, &b.mu, &b.muf, &b.mut, &b.vol, &b.dtm, &b.x, &b.y, &b.z, &b.xc, &b.yc, &b.zc, &b.aux};
+    for (gptr<double>* q : one) if ((r = dalloc(hb, q, n))) return r;
     for (int q = 0; q < 7; q++) if ((r = dalloc(hb, &b.prim[q], n))) return r;
     for (int q = 0; q < 3; q++) if ((r = dalloc(hb, &b.Lc[q], n)) || (r = dalloc(hb, &b.Lv[q], n)) || (r = dalloc(hb, &b.S[q], n))) return r;
     for (int q = 0; q < 9; q++) if ((r = dalloc(hb, &b.nv[q], n))) return r;
@@ -173,16 +173,16 @@ int carve_block(ocfd_ctx* c, HostBlock& hb) {
     if (c->p.mixed) {
         // FP32 primitives in half-size slots; FP32 face terms in the first half of the FP64 arrays
         for (int q = 0; q < 6; q++) {
-            double* a = nullptr;
+            gptr<double> a;
             if ((r = dalloc(hb, &a, (n + 1) / 2))) return r;
-            b.primf[q] = reinterpret_cast<float*>(a);
+            b.primf[q] = (float*)(double*)a;
         }
         // FP32 geometry: normals, areas, the face metrics (and the cell metrics with a turbulence
         // model), the inviscid flux's node differences
-        auto falloc = [&](float** q) {
-            double* a = nullptr;
+        auto falloc = [&](gptr<float>* q) {
+            gptr<double> a;
             int rr = dalloc(hb, &a, (n + 1) / 2);
-            *q = reinterpret_cast<float*>(a);
+            *q = (float*)(double*)a;
             return rr;
         };
         for (int q = 0; q < 9; q++) if ((r = falloc(&b.nvf[q]))) return r;
@@ -190,9 +190,9 @@ int carve_block(ocfd_ctx* c, HostBlock& hb) {
         for (int m = turb ? 0 : 1; m < 4; m++) for (int q = 0; q < 9; q++) if ((r = falloc(&b.metf[m][q]))) return r;
         for (int dd = 0; dd < 3; dd++) for (int q = 0; q < 3; q++) if ((r = falloc(&b.t1f[dd][q]))) return r;
         for (int dd = 0; dd < 3; dd++) {
-            for (int m = 0; m < 5; m++) b.Ff[dd][m] = reinterpret_cast<float*>(b.F[dd][m]);
-            for (int m = 0; m < 4; m++) b.Fvf[dd][m] = reinterpret_cast<float*>(b.Fv[dd][m]);
-            for (int m = 0; m < 2; m++) b.Fsaf[dd][m] = reinterpret_cast<float*>(b.Fsa[dd][m]);
+            for (int m = 0; m < 5; m++) b.Ff[dd][m] = (float*)(double*)b.F[dd][m];
+            for (int m = 0; m < 4; m++) b.Fvf[dd][m] = (float*)(double*)b.Fv[dd][m];
+            for (int m = 0; m < 2; m++) b.Fsaf[dd][m] = (float*)(double*)b.Fsa[dd][m];
         }
     }
     size_t jk = (size_t)b.NJ * b.NK, ik = (size_t)b.NI * b.NK, ij = (size_t)b.NI * b.NJ;
@@ -202,9 +202,9 @@ int carve_block(ocfd_ctx* c, HostBlock& hb) {
     b.flags = (int*)carve(hb, 16 * sizeof(int));
     if (c->p.NV == 6) {
         size_t ncell = (size_t)(hb.nx - 1) * (hb.ny - 1) * (hb.nz - 1);
-        double* m = nullptr;
+        gptr<double> m;
         if ((r = dalloc(hb, &m, (ncell + 63) / 64))) return r;
-        b.samask = reinterpret_cast<unsigned long long*>(m);
+        b.samask = (unsigned long long*)(double*)m;
     }
     return OCFD_OK;
 }
