@@ -1391,8 +1391,10 @@ __device__ __forceinline__ void d_corner_vertices(const Blk& b, int c, int m) {
 // force_vt_kw (sub_time_advance.f90:27-61), which changes cells that no edge or vertex reads.
 // Workgroup 13 (NV block + variable) + edge walks an edge, + 12 forms the vertices, which take the
 // edge cells they need from the faces' ghost cells, as the edges do; the cells' tiles follow.
-// (nb 0: no edges and vertices.)
-__global__ void __launch_bounds__(64) k_corner_force(BSet S, int nb, int NV) {
+// (nb 0: no edges and vertices.)  The sweeps' error word goes to the host, so the host has it after
+// its wait for the stream and copies nothing.
+__global__ void __launch_bounds__(64) k_corner_force(BSet S, int nb, int NV, int* halt_host) {
+    if (halt_host && S.halt && blockIdx.x == 0 && threadIdx.x == 0) *halt_host = *S.halt;
     const int nc = 13 * nb * NV;
     if ((int)blockIdx.x < nc) {
         const int e = (int)blockIdx.x % 13, m = (int)blockIdx.x / 13 % NV;
@@ -1671,7 +1673,7 @@ static void corner_force(const SetPlan& P, bool corners, bool force, hipStream_t
     const int nb = corners ? P.nb : 0, NV = P.p0.NV;
     const int nf = force && NV >= 6 && !(NV == 6 && P.p0.limit_flow == 1) ? P.ntiles[SP_CELL] : 0;
     const int n = 13 * nb * NV + nf;
-    if (n > 0) hipLaunchKernelGGL(k_corner_force, dim3((unsigned)n), dim3(64), 0, st, bset(P, SP_CELL), nb, NV);
+    if (n > 0) hipLaunchKernelGGL(k_corner_force, dim3((unsigned)n), dim3(64), 0, st, bset(P, SP_CELL), nb, NV, P.halt_host);
 }
 static void halo_copy(const SetPlan& P, hipStream_t st) {
     if (P.halo.ntiles > 0)

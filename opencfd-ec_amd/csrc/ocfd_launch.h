@@ -33,6 +33,7 @@ struct SetPlan {
     SubList sghost;                  // SST: the six faces of every block with their ghost rows (k_sst_ghost)
     HaloList halo;
     int* limited = nullptr;          // set by the update when a cell of the set needs the limiter
+    int* halt_host = nullptr;        // pinned: the word's value at the end of an iteration
     const int* halt = nullptr;       // the LU-SGS error word of the engine's sweeps (or null)
 };
 

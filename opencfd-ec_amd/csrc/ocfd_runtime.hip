@@ -45,19 +45,20 @@ struct HostBlock {
 
 }  // namespace
 
-// Launch machinery of one block list: its stream, the per-stage graphs and the device tables
+// Launch machinery of one block list: its stream, the captured graphs and the device tables
 // of the batched launches and of the pipelined LU-SGS sweeps.  A context owns one for its own
 // blocks; a batch owns one for the blocks of all its member contexts.
 struct Engine {
     hipStream_t st = nullptr;
     bool use_graph = false;
-    hipGraphExec_t exec[OCFD_NSTAGES] = {};   // one captured graph per stage of the iteration
-    hipGraph_t graph[OCFD_NSTAGES] = {};
+    hipGraphExec_t exec[OCFD_NSTAGES + 1] = {};   // a captured graph per stage, the last of the whole iteration
+    hipGraph_t graph[OCFD_NSTAGES + 1] = {};
     std::vector<hipEvent_t> events;           // stage boundaries of ocfd_step_timed
     int lu_schedule = OCFD_LU_PIPELINED;     // LU-SGS sweep schedule
     int lu_tj = 8;                            // tile width of the pipelined sweep
     int lu_fail = 0;                          // 1: every sweep wait that has to poll gives up
     LuPlan lu{};                              // pipelined-sweep tables (built on first use)
+    int* err_host = nullptr;                  // pinned: the sweeps' error word after an iteration
     int lu_nv = 0;
     std::vector<void*> lu_allocs;
     SetPlan set{};                            // batched-launch tables (built on first use)
@@ -386,22 +387,34 @@ void enqueue_stage(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, 
 }
 
 void drop_graphs(Engine& e) {
-    for (int s = 0; s < OCFD_NSTAGES; s++) {
+    for (int s = 0; s <= OCFD_NSTAGES; s++) {
         if (e.exec[s]) { (void)hipGraphExecDestroy(e.exec[s]); e.exec[s] = nullptr; }
         if (e.graph[s]) { (void)hipGraphDestroy(e.graph[s]); e.graph[s] = nullptr; }
     }
 }
 
-// One stage of the iteration: eager launches, or the stage's graph (captured on first use).
+// stage OCFD_NSTAGES: all of them
+void enqueue_stages(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, int stage) {
+    const bool all = stage == OCFD_NSTAGES;
+    for (int s = all ? 0 : stage; s < (all ? OCFD_NSTAGES : stage + 1); s++) enqueue_stage(e, refs, p0, s);
+}
+
+// the graph of a stage or of the iteration, captured on first use
+int capture_stage(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, int stage) {
+    if (!e.use_graph || e.per_block || e.exec[stage]) return OCFD_OK;
+    HIPCHK(hipStreamBeginCapture(e.st, hipStreamCaptureModeThreadLocal));
+    enqueue_stages(e, refs, p0, stage);
+    HIPCHK(hipStreamEndCapture(e.st, &e.graph[stage]));
+    HIPCHK(hipGraphInstantiate(&e.exec[stage], e.graph[stage], nullptr, nullptr, 0));
+    return OCFD_OK;
+}
+
+// one stage of the iteration, or all of them: eager launches or the graph
 int run_stage(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, int stage) {
-    if (stage == OCFD_STAGE_UPDATE && e.lu_schedule == OCFD_LU_PIPELINED) e.du_pending = true;
-    if (!e.use_graph || e.per_block) { enqueue_stage(e, refs, p0, stage); return OCFD_OK; }
-    if (!e.exec[stage]) {
-        HIPCHK(hipStreamBeginCapture(e.st, hipStreamCaptureModeThreadLocal));
-        enqueue_stage(e, refs, p0, stage);
-        HIPCHK(hipStreamEndCapture(e.st, &e.graph[stage]));
-        HIPCHK(hipGraphInstantiate(&e.exec[stage], e.graph[stage], nullptr, nullptr, 0));
-    }
+    if ((stage == OCFD_NSTAGES || stage == OCFD_STAGE_UPDATE) && e.lu_schedule == OCFD_LU_PIPELINED) e.du_pending = true;
+    if (!e.use_graph || e.per_block) { enqueue_stages(e, refs, p0, stage); return OCFD_OK; }
+    int r = capture_stage(e, refs, p0, stage);
+    if (r) return r;
     HIPCHK(hipGraphLaunch(e.exec[stage], e.st));
     return OCFD_OK;
 }
@@ -649,11 +662,13 @@ int build_lu_plan_batch(ocfd_batch* b, const Par& p0) {
     return OCFD_OK;
 }
 
-// After a sweep gave up waiting: clear the flag and re-arm both counter sets.
-int check_lu_error(Engine& e) {
+// After a sweep gave up waiting: clear the flag and re-arm both counter sets.  iterated: the stream
+// has ended with an iteration's last launch, which left the word in err_host.
+int check_lu_error(Engine& e, bool iterated = false) {
     if (!e.lu.err) return OCFD_OK;
     int v = 0;
-    HIPCHK(hipMemcpy(&v, e.lu.err, sizeof(int), hipMemcpyDeviceToHost));
+    if (iterated && e.err_host) v = *(volatile int*)e.err_host;
+    else HIPCHK(hipMemcpy(&v, e.lu.err, sizeof(int), hipMemcpyDeviceToHost));
     if (v == 0) return OCFD_OK;
     std::vector<int> minus(std::max(e.lu.n_fwd, e.lu.n_bwd), -1);
     HIPCHK(hipMemcpy(e.lu.prog_fwd, minus.data(), e.lu.n_fwd * sizeof(int), hipMemcpyHostToDevice));
@@ -820,13 +835,13 @@ int engine_prepare(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, 
     return OCFD_OK;
 }
 
-int engine_finish(Engine& e) {
+int engine_finish(Engine& e, bool iterated = false) {
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e.st));
     int r = OCFD_OK;
     for (Engine& q : e.parts) { int rq = check_lu_error(q); if (rq && !r) r = rq; }
     if (r) { e.du_pending = false; return r; }     // the parts' storage holds no iteration's DU
-    return check_lu_error(e);
+    return check_lu_error(e, iterated);
 }
 
 // niter iterations; with stage_ms, HIP events at the stage boundaries (device ms per stage,
@@ -841,15 +856,27 @@ int engine_step(Engine& e, const std::vector<BlockRef>& refs, const Par& p0, int
             e.events.push_back(ev);
         }
     }
+    if (e.lu.err && !e.err_host) HIPCHK(hipHostMalloc((void**)&e.err_host, sizeof(int), hipHostMallocDefault));
+    e.set.halt_host = e.err_host;
+    // captured ahead of the first event, so no stage's time holds a capture
+    for (int s = 0; s < OCFD_NSTAGES && stage_ms; s++)
+        if ((r = capture_stage(e, refs, p0, s))) return r;
     for (int it = 0; it < niter; it++) {
-        hipEvent_t* ev = stage_ms ? e.events.data() + (size_t)it * (OCFD_NSTAGES + 1) : nullptr;
-        if (ev) HIPCHK(hipEventRecord(ev[0], e.st));
+        if (!stage_ms) {
+            // One graph launch per iteration; between the launches of a graph per stage the GPU idles
+            // for about 5 us each (97x33x9 channel 226 -> 195 us per iteration, 65x25x9 SA 208 -> 178,
+            // 257x97x33 1003 -> 972).
+            if ((r = run_stage(e, refs, p0, OCFD_NSTAGES))) return r;
+            continue;
+        }
+        hipEvent_t* ev = e.events.data() + (size_t)it * (OCFD_NSTAGES + 1);
+        HIPCHK(hipEventRecord(ev[0], e.st));
         for (int s = 0; s < OCFD_NSTAGES; s++) {
             if ((r = run_stage(e, refs, p0, s))) return r;
-            if (ev) HIPCHK(hipEventRecord(ev[s + 1], e.st));
+            HIPCHK(hipEventRecord(ev[s + 1], e.st));
         }
     }
-    if ((r = engine_finish(e))) return r;
+    if ((r = engine_finish(e, niter > 0 && !e.per_block))) return r;
     if (stage_ms) {
         for (int s = 0; s < OCFD_NSTAGES; s++) stage_ms[s] = 0.0;
         for (int it = 0; it < niter; it++) {
@@ -914,6 +941,8 @@ void engine_destroy(Engine& e) {
     drop_plans(e);
     for (hipEvent_t ev : e.events) (void)hipEventDestroy(ev);
     e.events.clear();
+    if (e.err_host) (void)hipHostFree(e.err_host);
+    e.err_host = nullptr;
     if (e.st) (void)hipStreamDestroy(e.st);
     e.st = nullptr;
 }

@@ -231,7 +231,7 @@ class Server:
                 if not active:
                     continue
                 if flags["recapture"]:
-                    # the batch captures its stage graphs in this round: no device calls from the
+                    # the batch captures its graphs in this round: no device calls from the
                     # preparing thread meanwhile
                     with st["dev"]:
                         batch.step(self.round_iters)
