@@ -38,9 +38,37 @@ struct gptr {
     __host__ __device__ __forceinline__ T& operator[](uint32_t s) const { return (*this)[(size_t)s]; }
     __host__ __device__ __forceinline__ T& operator[](long s) const { return ((T*)p)[s]; }
     __host__ __device__ __forceinline__ T& operator[](int s) const { return ((T*)p)[s]; }
+    // element s + o of an array that the kernel does not write (o the same in all lanes): the load may
+    // move ahead of the kernel's stores, which a plain load does not, since the compiler cannot tell
+    // the arrays of the table apart
+    __device__ __forceinline__ T ro(size_t s, long o = 0) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef __attribute__((address_space(4))) const char* cptr;
+        return *(__attribute__((address_space(4))) const T*)((cptr)(p + o) + (uint32_t)((uint32_t)s * (uint32_t)sizeof(T)));
+#else
+        return p[s + o];
+#endif
+    }
     // the array shifted by an offset that is the same in all lanes (a stencil's neighbour): at(o)[s]
     // is element s + o
     __host__ __device__ __forceinline__ gptr at(long o) const { return gptr{p + o}; }
+};
+
+// A table that no kernel writes (blocks, their parameters, tile maps), in the constant address space
+// in device code.  Through a plain pointer the compiler has to assume that a kernel's stores may
+// change the table: it then reads each array pointer with a vector load of its own, just before the
+// array's element and after the stores ahead of it.  From here the pointers come in scalar loads.
+template <typename T>
+struct ctab {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(4))) const T* ptr;
+#else
+    typedef const T* ptr;
+#endif
+    ptr p;
+    ctab() = default;
+    __host__ __device__ __forceinline__ ctab(const T* q) : p((ptr)q) {}
+    __host__ __device__ __forceinline__ const T& operator[](long i) const { return *(const T*)(p + i); }
 };
 
 struct Par {                 // control parameters after set_const_para (sub_read_parameter.f90:371-429)
@@ -122,10 +150,10 @@ __device__ __host__ __forceinline__ void space_dims(int sp, const Blk& b, int& n
 }
 
 struct BSet {
-    const Blk* blk;
-    const Par* par;
-    const int* tile_blk;     // for the launch's space
-    const int* tile0;
+    ctab<Blk> blk;
+    ctab<Par> par;
+    ctab<int> tile_blk;      // for the launch's space
+    ctab<int> tile0;
     const int* halt;         // nonzero *halt: an LU-SGS sweep of this iteration gave up; the update
                              // kernels then leave U as it is (may be null)
     int* limited;            // set by the update when a cell of any block needs the limiter
@@ -145,7 +173,7 @@ __device__ __forceinline__ int xcd_tile(int t, int n) {
 constexpr int ROW_CHUNK = 16;
 
 // point `lane` of tile t of iteration space sp
-__device__ __forceinline__ bool locate_point(int sp, const Blk* blk, const int* tile_blk, const int* tile0, int t, int& bi, int& i, int& j,
+__device__ __forceinline__ bool locate_point(int sp, const ctab<Blk>& blk, const ctab<int>& tile_blk, const ctab<int>& tile0, int t, int& bi, int& i, int& j,
                                              int& k, int lane) {
     bi = tile_blk[t];
     int n0, n1, n2, o0, o1, o2;
@@ -185,10 +213,10 @@ __device__ __forceinline__ bool locate(const BSet& S, int& bi, int& i, int& j, i
 
 // The faces of the three directions in one launch: n[d] tiles of direction d (space SP_FI + d).
 struct FaceSet {
-    const Blk* blk;
-    const Par* par;
-    const int* tile_blk[3];
-    const int* tile0[3];
+    ctab<Blk> blk;
+    ctab<Par> par;
+    ctab<int> tile_blk[3];
+    ctab<int> tile0[3];
     int n[3];
 };
 
@@ -232,10 +260,10 @@ struct SubTask {
     Sub B;
 };
 struct SubSet {
-    const Blk* blk;
-    const Par* par;
-    const SubTask* t;
-    const int* tile_task;
+    ctab<Blk> blk;
+    ctab<Par> par;
+    ctab<SubTask> t;
+    ctab<int> tile_task;
 };
 
 #define OCFD_SUB_LOCATE                                                      \
@@ -253,9 +281,9 @@ struct HaloTask {
     HaloMap h;
 };
 struct HaloSet {
-    const Blk* blk;
-    const HaloTask* t;
-    const int* tile_task;
+    ctab<Blk> blk;
+    ctab<HaloTask> t;
+    ctab<int> tile_task;
 };
 
 // one tile of the pipelined LU-SGS sweep: cells j0..j0+tj-1, k0..k0+tk-1 of block `blk`, all i

@@ -111,6 +111,7 @@ __global__ void __launch_bounds__(64) k_prims(BSet S) {
 // Spalart-Allmaras (sub_turbulence_SA.f90:8-273).  U6 is read through limit_vt's clamp
 // (sub_time_advance.f90:420-428): negative values act as zero.
 // limit_vt's clamp of U6 at the element o away from s
+__device__ __forceinline__ double vt_ro(const Blk& b, size_t s, long o = 0) { double v = b.U[5].ro(s, o); return v < 0.0 ? 0.0 : v; }
 __device__ __forceinline__ double vt_of(const Blk& b, size_t s, long o) { double v = b.U[5].at(o)[s]; return v < 0.0 ? 0.0 : v; }
 __device__ __forceinline__ double pw6(double x) { return ((((x * x) * x) * x) * x) * x; }   // flang expansion order
 
@@ -137,13 +138,13 @@ __device__ __forceinline__ void put_Fv(const Blk& b, int d, int m, size_t s, flo
 __device__ __forceinline__ void put_Fsa(const Blk& b, int d, int m, size_t s, double v) { b.Fsa[d][m][s] = v; }
 __device__ __forceinline__ void put_Fsa(const Blk& b, int d, int m, size_t s, float v) { b.Fsaf[d][m][s] = v; }
 template <typename T> __device__ __forceinline__ double get_F(const Blk& b, int d, int m, size_t s, long o) {
-    if constexpr (sizeof(T) == 8) return b.F[d][m].at(o)[s]; else return (double)b.Ff[d][m].at(o)[s];
+    if constexpr (sizeof(T) == 8) return b.F[d][m].ro(s, o); else return (double)b.Ff[d][m].ro(s, o);
 }
 template <typename T> __device__ __forceinline__ double get_Fv(const Blk& b, int d, int m, size_t s, long o) {
-    if constexpr (sizeof(T) == 8) return b.Fv[d][m].at(o)[s]; else return (double)b.Fvf[d][m].at(o)[s];
+    if constexpr (sizeof(T) == 8) return b.Fv[d][m].ro(s, o); else return (double)b.Fvf[d][m].ro(s, o);
 }
 template <typename T> __device__ __forceinline__ double get_Fsa(const Blk& b, int d, int m, size_t s, long o) {
-    if constexpr (sizeof(T) == 8) return b.Fsa[d][m].at(o)[s]; else return (double)b.Fsaf[d][m].at(o)[s];
+    if constexpr (sizeof(T) == 8) return b.Fsa[d][m].ro(s, o); else return (double)b.Fsaf[d][m].ro(s, o);
 }
 
 // SA constants (sub_turbulence_SA.f90:18-33)
@@ -205,8 +206,8 @@ __device__ __forceinline__ double sa_residual(const Blk& b, const Par& p, int i,
     const double Re = p.Re;
     const gptr<double> d = b.prim[0];
     const gptr<T> dt_ = prim_of<T>(b, 0), ut = prim_of<T>(b, 1), vtt = prim_of<T>(b, 2), wt = prim_of<T>(b, 3);
-    double vt_c = vt_of(b, s, 0), mu_c = b.mu[s] * Re;
-    double v0c = ((vt_c + mu_c / d[s]) * SAc::Cb2) / SAc::sigma;
+    double vt_c = vt_ro(b, s), mu_c = b.mu.ro(s) * Re;
+    double v0c = ((vt_c + mu_c / d.ro(s)) * SAc::Cb2) / SAc::sigma;
     const long sp[3] = {1, OFF(b, 0, 1, 0), OFF(b, 0, 0, 1)};
     double res = 0.0;
 #pragma unroll
@@ -216,20 +217,20 @@ __device__ __forceinline__ double sa_residual(const Blk& b, const Par& p, int i,
         if (dir == 0) res = (fv1 - fv0) - (v0c / Re) * (f21 - f20);
         else res = ((res + fv1) - fv0) - (v0c / Re) * (f21 - f20);
     }
-    auto UU = [&](int a, int bb, int cc) { return ut.at(OFF(b, a, bb, cc))[s]; };
-    auto VV = [&](int a, int bb, int cc) { return vtt.at(OFF(b, a, bb, cc))[s]; };
-    auto WW = [&](int a, int bb, int cc) { return wt.at(OFF(b, a, bb, cc))[s]; };
+    auto UU = [&](int a, int bb, int cc) { return ut.ro(s, OFF(b, a, bb, cc)); };
+    auto VV = [&](int a, int bb, int cc) { return vtt.ro(s, OFF(b, a, bb, cc)); };
+    auto WW = [&](int a, int bb, int cc) { return wt.ro(s, OFF(b, a, bb, cc)); };
     T ui = UU(1, 0, 0) - UU(-1, 0, 0), vi = VV(1, 0, 0) - VV(-1, 0, 0), wi = WW(1, 0, 0) - WW(-1, 0, 0);
     T uj = UU(0, 1, 0) - UU(0, -1, 0), vj = VV(0, 1, 0) - VV(0, -1, 0), wj = WW(0, 1, 0) - WW(0, -1, 0);
     T uk = UU(0, 0, 1) - UU(0, 0, -1), vk = VV(0, 0, 1) - VV(0, 0, -1), wk = WW(0, 0, 1) - WW(0, 0, -1);
-    auto M0 = [&](int q) { return met_of<T>(b, 0, q)[s]; };
+    auto M0 = [&](int q) { return met_of<T>(b, 0, q).ro(s); };
     T ix = M0(0), iy = M0(1), iz = M0(2), jx = M0(3), jy = M0(4), jz = M0(5), kx = M0(6), ky = M0(7), kz = M0(8);
     T vx = (vi * ix + vj * jx) + vk * kx, wx = (wi * ix + wj * jx) + wk * kx;
     T uy = (ui * iy + uj * jy) + uk * ky, wy = (wi * iy + wj * jy) + wk * ky;
     T uz = (ui * iz + uj * jz) + uk * kz, vz = (vi * iz + vj * jz) + vk * kz;
     T S = sqrt((sq(wy - vz) + sq(uz - wx)) + sq(vx - uy));
-    T dw = T(b.dw[s]);
-    T X = dt_[s] * T(vt_c) / T(mu_c);
+    T dw = T(b.dw.ro(s));
+    T X = dt_.ro(s) * T(vt_c) / T(mu_c);
     T fv1 = (X * X * X) / ((X * X * X) + T(Cv1_3));
     T fv2 = T(1) - X / (T(1) + X * fv1);
     T ft2 = T(SAc::Ct3) * exp(-((T(SAc::Ct4) * X) * X));
@@ -241,7 +242,7 @@ __device__ __forceinline__ double sa_residual(const Blk& b, const Par& p, int i,
     T fw = g * pow((T(1) + T(Cw3_6)) / ((((((g * g) * g) * g) * g) * g) + T(Cw3_6)), T(1.0 / 6.0));
     T Q3 = (T(SAc::Cb1) * ((T(1) - ft2) * fv2 + ft2)) / T(SAc::k * SAc::k) - T(Cw1) * fw;
     T Q_SA = ((T(SAc::Cb1) * (T(1) - ft2)) * S1) * T(vt_c) + (Q3 * sq(T(vt_c) / dw)) / T(Re);
-    return res + (double)(Q_SA * T(b.vol[s]));
+    return res + (double)(Q_SA * T(b.vol.ro(s)));
 }
 
 // Amut_boundary (sub_turbulence_SA.f90:282-368) on one wall subface
@@ -719,14 +720,14 @@ __device__ __forceinline__ void cell_assemble(const Blk& b, const Par& p, int i,
     }
     if (p.turb == 2) res(5, sa_residual<T>(b, p, i, j, k, s));
     const double g43 = p.gamma > (double)(4.0f / 3.0f) ? p.gamma : (double)(4.0f / 3.0f);
-    double d = b.prim[0][s], u = b.prim[1][s], v = b.prim[2][s], w = b.prim[3][s], c = b.prim[6][s];
-    double D0 = p.visc == 1 ? (g43 / d) * (b.muf[s] / p.PrL + b.mut[s] / p.PrT) : 0.0;
-    double vol = b.vol[s], vol1 = 1.0 / vol;
+    double d = b.prim[0].ro(s), u = b.prim[1].ro(s), v = b.prim[2].ro(s), w = b.prim[3].ro(s), c = b.prim[6].ro(s);
+    double D0 = p.visc == 1 ? (g43 / d) * (b.muf.ro(s) / p.PrL + b.mut.ro(s) / p.PrT) : 0.0;
+    double vol = b.vol.ro(s), vol1 = 1.0 / vol;
 #pragma unroll
     for (int dir = 0; dir < 3; dir++) {
-        double un = 0.5 * ((u * (b.nv[3 * dir][s] + b.nv[3 * dir].at(sp[dir])[s]) + v * (b.nv[3 * dir + 1][s] + b.nv[3 * dir + 1].at(sp[dir])[s]))
-                           + w * (b.nv[3 * dir + 2][s] + b.nv[3 * dir + 2].at(sp[dir])[s]));
-        double S0 = (b.S[dir][s] + b.S[dir].at(sp[dir])[s]) * 0.5;
+        double un = 0.5 * ((u * (b.nv[3 * dir].ro(s) + b.nv[3 * dir].ro(s, sp[dir])) + v * (b.nv[3 * dir + 1].ro(s) + b.nv[3 * dir + 1].ro(s, sp[dir])))
+                           + w * (b.nv[3 * dir + 2].ro(s) + b.nv[3 * dir + 2].ro(s, sp[dir])));
+        double S0 = (b.S[dir].ro(s) + b.S[dir].ro(s, sp[dir])) * 0.5;
         Lc[dir] = (fabs(un) + c) * S0;
         Lv[dir] = ((D0 * S0) * S0) * vol1;
         lam(dir, Lc[dir], Lv[dir]);
@@ -734,7 +735,7 @@ __device__ __forceinline__ void cell_assemble(const Blk& b, const Par& p, int i,
     if (p.local_dt == 1) {
         double dt_fac = b.flags[0] == 0 ? 1.0 : 0.1;
         dt = ((dt_fac * p.CFL) * vol) / (((Lc[0] + Lc[1]) + Lc[2]) + 1.0 * ((Lv[0] + Lv[1]) + Lv[2]));
-        if (p.dtime_mesh == 1) dt = dt * b.dtm[s];
+        if (p.dtime_mesh == 1) dt = dt * b.dtm.ro(s);
         if (dt > p.dtmax) dt = p.dtmax;
         if (dt < p.dtmin) dt = p.dtmin;
     } else {
@@ -764,12 +765,14 @@ __global__ void __launch_bounds__(64) k_cell(BSet S) {
 // the sentinel.  Bound by memory: against a cell pass in box order and a pack of its own, Lc, Lv
 // and the diagonal are not written and read back, nor Res read back (200 B per cell less), cell
 // pass and pack of the 24-block wing with 6.3 M cells 2020 -> 1750 us, of the 257x97x33 C-grid
-// 218 -> 203, of six serving solves 839 -> 759.  The register cap for six waves per SIMD makes it:
+// 218 -> 203, of six serving solves 839 -> 759.  With the array pointers in scalar loads (ctab) and
+// the inputs' loads free to pass the stores (gptr::ro): the wing 1785 -> 1760, the C-grid 215 -> 200,
+// a 65x25x9 grid, where a workgroup's chain of loads is the whole time, 37 -> 29.  The register cap for six waves per SIMD makes it:
 // uncapped (130 VGPRs) one workgroup of eight waves fills a CU and the wing takes 2150 us, with four
 // waves 1780, with seven 1770.
 template <int NV, int TJ, typename T>
-__global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, const LuTask* __restrict__ tiles, double* __restrict__ pk,
-                                                  const int2* __restrict__ wins) {
+__global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, ctab<LuTask> tiles, double* __restrict__ pk,
+                                                  ctab<int2> wins) {
     using F = Pk<NV>;
     __shared__ double buf[NV + 2][LU_COLS][PK_W + 2];
     const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];     // (tile, i-window), windows fastest
@@ -788,9 +791,9 @@ __global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, const LuTask* __res
         double dt;
         cell_assemble<T>(
             b, p, i, j, k, s, [&](int m, double r) { b.Res[m][s] = r; buf[m][c][x] = r; }, [](int, double, double) {}, Lc, Lv, dt);
-        if constexpr (NV == 7) { buf[5][c][x] = b.Res[5][s]; buf[6][c][x] = b.Res[6][s]; }
+        if constexpr (NV == 7) { buf[5][c][x] = b.Res[5].ro(s); buf[6][c][x] = b.Res[6].ro(s); }
         b.dt[s] = dt;
-        const double vol = b.vol[s];
+        const double vol = b.vol.ro(s);
         const double sumLc = (Lc[0] + Lc[1]) + Lc[2], sumLv = (Lv[0] + Lv[1]) + Lv[2];
         double alfa = vol / dt + p.w_LU * sumLc;
         if (p.visc == 1) alfa = alfa + 2.0 * sumLv;
@@ -821,7 +824,7 @@ __global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, const LuTask* __res
     if (live) {
         double u[NV];
 #pragma unroll
-        for (int m = 0; m < NV; m++) u[m] = b.U[m][s];
+        for (int m = 0; m < NV; m++) u[m] = b.U[m].ro(s);
         // comput_DFn's pressure of the undisturbed state, limit_vt's clamp
         const double r = recip_nr(u[0]);
         buf[NV][c][x] = (p.gamma - 1.0) * (u[4] - div_nr(0.5 * ((u[1] * u[1] + u[2] * u[2]) + u[3] * u[3]), u[0], r));
@@ -973,8 +976,8 @@ __global__ void __launch_bounds__(64) k_update_detect(BSet S) {
 constexpr int UP_T = LU_COLS * PK_W;
 
 template <int NV, int TJ>
-__global__ void __launch_bounds__(UP_T) k_update_pk(BSet S, const LuTask* __restrict__ tiles, const double* __restrict__ pk,
-                                                    const int2* __restrict__ wins) {
+__global__ void __launch_bounds__(UP_T) k_update_pk(BSet S, ctab<LuTask> tiles, const double* __restrict__ pk,
+                                                    ctab<int2> wins) {
     using F = Pk<NV>;
     constexpr int M = NV * LU_COLS;
     __shared__ double buf[NV][LU_COLS][PK_W + 2];
@@ -1541,7 +1544,9 @@ static void launch_subs(void (*kern)(SubSet), const SetPlan& P, const SubList& L
 }
 
 static void launch_faces(void (*kern)(FaceSet), const SetPlan& P, hipStream_t st) {
-    FaceSet S{P.blk, P.par, {}, {}, {}};
+    FaceSet S{};
+    S.blk = P.blk;
+    S.par = P.par;
     for (int d = 0; d < 3; d++) {
         S.tile_blk[d] = P.tile_blk[SP_FI + d];
         S.tile0[d] = P.tile0[SP_FI + d];

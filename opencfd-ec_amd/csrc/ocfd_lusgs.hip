@@ -254,8 +254,8 @@ __device__ __forceinline__ double ld_coherent(const double* p) {
 
 // the geometry the sweeps read (S, n), into sweep order once per plan
 template <int NV, int TJ>
-__global__ void __launch_bounds__(PK_T) k_lu_pack_geometry(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
-                                                           double* __restrict__ pk, const int2* __restrict__ wins) {
+__global__ void __launch_bounds__(PK_T) k_lu_pack_geometry(ctab<Blk> blks, ctab<LuTask> tiles,
+                                                           double* __restrict__ pk, ctab<int2> wins) {
     using F = Pk<NV>;
     __shared__ double buf[3][LU_COLS][PK_W + 2];
     const int2 wn = wins[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
@@ -284,8 +284,8 @@ __global__ void __launch_bounds__(PK_T) k_lu_pack_geometry(const Blk* __restrict
 // sweep order -> block arrays for the backward sweep's DU, for a host that reads DU: the storage
 // holds it from the end of the backward sweep until the next pack
 template <int NV, int TJ>
-__global__ void __launch_bounds__(PK_T) k_lu_du_to_box(const Blk* __restrict__ blks, const LuTask* __restrict__ tiles,
-                                                       const double* __restrict__ pk, const int2* __restrict__ wins) {
+__global__ void __launch_bounds__(PK_T) k_lu_du_to_box(ctab<Blk> blks, ctab<LuTask> tiles,
+                                                       const double* __restrict__ pk, ctab<int2> wins) {
     using F = Pk<NV>;
     constexpr int M = NV * LU_COLS;
     __shared__ double buf[NV][LU_COLS][PK_W + 2];
