@@ -686,8 +686,12 @@ __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, i
 // 22 us instead of 37 in three launches; 257x97x33 SA: 271 against 306); on large ones the
 // directions share the primitives in L2 (face_tile; a batch of 6 with 1.9 M cells: 835 against
 // 930 us, 24 blocks with 6.3 M cells: 2090 against 2200, before the metrics were read once).
+// Five waves per SIMD instead of four where that needs no spills (the primitive reconstruction: 90 to
+// 96 instead of 114 VGPRs) and is faster: 257x97x33 Roe 245 -> 238 us, 48 blocks AUSMPW 492 -> 474, 24
+// blocks Roe 1880 -> 1832; Van Leer's flux, with the least arithmetic, 736 -> 743.
+constexpr int face_waves(int recon, int flux) { return recon == 0 && flux != F_VL ? 5 : 1; }
 template <typename T, int RECON, int FLUX>
-__global__ void __launch_bounds__(64) k_face(FaceSet S) {
+__global__ void __launch_bounds__(64, face_waves(RECON, FLUX)) k_face(FaceSet S) {
     int bi, i, j, k;
     switch (locate_face(S, bi, i, j, k)) {
     case 0: face<0, T, RECON, FLUX>(S.blk[bi], S.par[bi], i, j, k); break;
