@@ -30,7 +30,6 @@ struct SetPlan {
     int ntiles[SP_COUNT] = {};
     SubList bc, force;               // force: the wall (bc 2) subfaces, one thread per face
     SubList amut, kbc;               // wall and k subfaces that do not lie on their block's face (usually none)
-    SubList sghost;                  // SST: the six faces of every block with their ghost rows (k_sst_ghost)
     HaloList halo;
     int* limited = nullptr;          // set by the update when a cell of the set needs the limiter
     int* halt_host = nullptr;        // pinned: the word's value at the end of an iteration

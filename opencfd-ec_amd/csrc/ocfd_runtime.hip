@@ -780,20 +780,8 @@ int build_set_plan(Engine& e, const std::vector<BlockRef>& refs, const Par& p0) 
             }
         }
     }
-    std::vector<SubTask> sghost;
-    for (int bi = 0; bi < P.nb && p0.turb == 3; bi++) {
-        const Blk& b = blks[bi];
-        for (int f = 0; f < 6; f++) {
-            SubTask t{};
-            t.blk = bi; t.arg = f;
-            t.n0 = f < 2 ? b.ny + 1 : b.nx + 1;
-            t.n1 = f < 4 ? b.nz + 1 : b.ny + 1;
-            sghost.push_back(t);
-        }
-    }
     if ((r = build_sub_list(e.set_allocs, bc, P.bc)) || (r = build_sub_list(e.set_allocs, amut, P.amut)) ||
         (r = build_sub_list(e.set_allocs, kbc, P.kbc)) || (r = build_sub_list(e.set_allocs, force, P.force)) ||
-        (r = build_sub_list(e.set_allocs, sghost, P.sghost)) ||
         (r = upload_table(e.set_allocs, std::vector<int>(1, 0), &P.limited)))
         return r;
     P.halo.ntiles = (int)halo_tile.size();
