@@ -54,6 +54,17 @@ struct gptr {
     __host__ __device__ __forceinline__ gptr at(long o) const { return gptr{p + o}; }
 };
 
+// s, worked out anew in the basic block that calls it (ID: no two calls are the same): the compiler
+// keeps an array's base in scalar registers only if it sees in the same block that s has 32 bits
+template <int ID>
+__device__ __forceinline__ size_t in_block(size_t s) {
+    uint32_t v = (uint32_t)s;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(v) : "i"(ID));
+#endif
+    return v;
+}
+
 // A table that no kernel writes (blocks, their parameters, tile maps), in the constant address space
 // in device code.  Through a plain pointer the compiler has to assume that a kernel's stores may
 // change the table: it then reads each array pointer with a vector load of its own, just before the

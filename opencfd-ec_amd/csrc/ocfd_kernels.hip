@@ -485,9 +485,10 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, const FaceG
     if constexpr (RECON == 0) {
         for (int m = 0; m < 5; m++) {
             const gptr<T> a = prim_of<T>(b, m);
+            const size_t v = in_block<1>(s);
             T u[8];
 #pragma unroll
-            for (int q = 0; q < 8; q++) u[q] = a.at((q - 4) * st)[s];     // u[q] = cell (face - 4 + q): u(q-3)
+            for (int q = 0; q < 8; q++) u[q] = a.at((q - 4) * st)[v];     // u[q] = cell (face - 4 + q): u(q-3)
             UL[m] = scheme_fP(u + 3, scheme);
             UR[m] = scheme_fm(u + 3, scheme);
         }
@@ -549,6 +550,7 @@ __device__ __forceinline__ void inv_face(const Blk& b, const Par& p, const FaceG
     QR[3] = (UR[1] * s3x + UR[2] * s3y) + UR[3] * s3z; QR[4] = UR[4];
     riemann_t<FLUX, T>(QL, QR, F0, T(p.gamma), p.flux);
     T Sf = g.S;
+    s = in_block<2>(s);
     put_F(b, DIR, 0, s, -F0[0] * Sf);
     put_F(b, DIR, 1, s, -((F0[1] * s1x + F0[2] * s2x) + F0[3] * s3x) * Sf);
     put_F(b, DIR, 2, s, -((F0[1] * s1y + F0[2] * s2y) + F0[3] * s3y) * Sf);
@@ -599,6 +601,7 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, const Face
         return;
     }
     const long m = -OFF(b, di, dj, dk);
+    s = in_block<3>(s);
     const gptr<T> Q[4] = {prim_of<T>(b, 1), prim_of<T>(b, 2), prim_of<T>(b, 3), prim_of<T>(b, 5)};
     // tangential directions: i-faces (j,k), j-faces (i,k), k-faces (i,j)
     constexpr int ai = DIR == 0 ? 0 : 1, aj = DIR == 0 ? 1 : 0;          // first tangential unit step
@@ -615,16 +618,12 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, const Face
     for (int q = 0; q < 4; q++) {
         const gptr<T> a = Q[q];
         T dn = a[s] - a.at(m)[s];
-        T ta1 = T(0), ta2 = T(0), tb1 = T(0), tb2 = T(0);
-        if (!zeroA) {
-            ta1 = T(0.5) * (a.at(-oa)[s] + a.at(m - oa)[s]);
-            ta2 = T(0.5) * (a.at(oa)[s] + a.at(m + oa)[s]);
-        }
-        if (!zeroB) {
-            tb1 = T(0.5) * (a.at(-ob)[s] + a.at(m - ob)[s]);
-            tb2 = T(0.5) * (a.at(ob)[s] + a.at(m + ob)[s]);
-        }
-        T ga = T(0.5) * (ta2 - ta1), gb = T(0.5) * (tb2 - tb1);
+        // no branch around the loads, so that all of them are in flight at once (257x97x33 238 -> 229 us,
+        // 48 blocks SST 625 -> 605, 24 blocks 1838 -> 1775); where zeroA or zeroB they are read for
+        // nothing, inside the box
+        const T ta1 = T(0.5) * (a.at(-oa)[s] + a.at(m - oa)[s]), ta2 = T(0.5) * (a.at(oa)[s] + a.at(m + oa)[s]);
+        const T tb1 = T(0.5) * (a.at(-ob)[s] + a.at(m - ob)[s]), tb2 = T(0.5) * (a.at(ob)[s] + a.at(m + ob)[s]);
+        const T ga = zeroA ? T(0) : T(0.5) * (ta2 - ta1), gb = zeroB ? T(0) : T(0.5) * (tb2 - tb1);
         if (DIR == 0) { gi[q] = dn; gj[q] = ga; gk[q] = gb; }
         else if (DIR == 1) { gi[q] = ga; gj[q] = dn; gk[q] = gb; }
         else { gi[q] = ga; gj[q] = gb; gk[q] = dn; }
@@ -669,14 +668,13 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, const Face
 }
 
 // Every flux through face (i,j,k) of direction DIR, one thread per face, each stored for the cell
-// pass: the SA face terms (sub_turbulence_SA.f90:60-174) or the SST fluxes, the viscous and the inviscid flux.
-// The terms that share the metrics come first and the face's geometry is read once: a wave lives 25
-// us, in which an XCD's L2 is filled three times over, so a second read of a metric or a normal
-// later in the kernel came from memory again (24 blocks with 6.3 M cells: 7.0 -> 4.1 GB read, 2070 ->
-// 1880 us; a batch of 6 with 1.9 M cells 842 -> 737 us; 257x97x33: 264 -> 246).  What bounds it now
-// is FP64 arithmetic: the vector units are busy 64 % of the time at 4 waves per SIMD (118 VGPRs).
-// Slower: the viscous part in workgroups of its own (100 VGPRs, 1980 us; capped for 5 waves 1885),
-// one kernel capped for 5 waves (spills, 2225), non-temporal flux stores and metric loads (1910).
+// pass: the SA face terms (sub_turbulence_SA.f90:60-174) or the SST fluxes, the viscous and the
+// inviscid flux.  The terms that share the metrics come first and the face's geometry is read once:
+// a wave lives 25 us, in which an XCD's L2 is filled three times over, so a second read of a metric
+// or a normal later in the kernel came from memory again (24 blocks with 6.3 M cells: 7.0 -> 4.1 GB
+// read, 2070 -> 1880 us; a batch of 6 with 1.9 M cells 842 -> 737 us; 257x97x33: 264 -> 246).  What
+// bounds it now is FP64 arithmetic: the vector units are busy 64 % of the time.  Slower: the viscous
+// part in workgroups of its own (1980 us), non-temporal flux stores and metric loads (1910).
 template <int DIR, typename T, int RECON, int FLUX, bool SST>
 __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, int k) {
     const size_t s = IX(b, i, j, k);
@@ -707,9 +705,9 @@ __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, i
 // 22 us instead of 37 in three launches; 257x97x33 SA: 271 against 306); on large ones the
 // directions share the primitives in L2 (face_tile; a batch of 6 with 1.9 M cells: 835 against
 // 930 us, 24 blocks with 6.3 M cells: 2090 against 2200, before the metrics were read once).
-// Five waves per SIMD instead of four where that needs no spills (the primitive reconstruction: 90 to
-// 96 instead of 114 VGPRs) and is faster: 257x97x33 Roe 245 -> 238 us, 24 blocks Roe 1880 -> 1832;
-// Van Leer's flux, with the least arithmetic, 736 -> 743, and with SST's fluxes 624 -> 635.
+// Five waves per SIMD instead of four where that needs no spills (the primitive reconstruction: 96
+// instead of 122 VGPRs) and is faster: 24 blocks Roe 1880 -> 1832 us; Van Leer's flux, with the least
+// arithmetic, 719 -> 737, and SST, with the most registers (142), 605 -> 900.
 constexpr int face_waves(int recon, int flux, bool sst) { return recon == 0 && flux != F_VL && !sst ? 5 : 1; }
 template <typename T, int RECON, int FLUX, bool SST>
 __global__ void __launch_bounds__(64, face_waves(RECON, FLUX, SST)) k_face(FaceSet S) {
