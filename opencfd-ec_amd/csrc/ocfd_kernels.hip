@@ -1097,21 +1097,26 @@ __device__ __forceinline__ void flagged_tiles(const BSet& S, int nb, int ntiles,
 // di + 2dj - 4 < 0; dk = 0, dj = -1: di - 2 < 0; dk = dj = 0: di = -1) and two cells with the same
 // w are never neighbours, so the cells of one w are done in parallel after all smaller w, and
 // each reads exactly what the sequential loop gives it.
+// All 27 values are loaded before the first is judged: one trip to memory instead of one per neighbour.
 __device__ __forceinline__ void sa_replace(const Blk& b, const Par& p, int i, int j, int k) {
     const double SAmin = 1.0e-8;
-    double* U6 = b.U[5];
-    const double* orig = b.prim[5];
-    double s0 = 0.0; int kn = 0;
-    for (int ka = -1; ka <= 1; ka++) for (int ja = -1; ja <= 1; ja++) for (int ia = -1; ia <= 1; ia++) {
-        int i1 = i + ia, j1 = j + ja, k1 = k + ka;
-        if (i1 > 0 && i1 < b.nx && j1 > 0 && j1 < b.ny && k1 > 0 && k1 < b.nz) {
-            size_t t = IX(b, i1, j1, k1);
-            bool later = (k1 > k) || (k1 == k && (j1 > j || (j1 == j && i1 > i)));
-            double v = later ? orig[t] : U6[t];
-            if (v >= SAmin && v <= p.LSAmax) { s0 = s0 + v; kn++; }
-        }
+    const size_t s = IX(b, i, j, k);
+    double v[27];
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        const int ia = q % 3 - 1, ja = q / 3 % 3 - 1, ka = q / 9 - 1;
+        const bool later = ka > 0 || (ka == 0 && (ja > 0 || (ja == 0 && ia > 0)));
+        v[q] = later ? b.prim[5].ro(s, OFF(b, ia, ja, ka)) : b.U[5].at(OFF(b, ia, ja, ka))[s];
     }
-    U6[IX(b, i, j, k)] = kn == 0 ? p.LSAmax : s0 / (double)kn;
+    double s0 = 0.0;
+    int kn = 0;
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        const int i1 = i + q % 3 - 1, j1 = j + q / 3 % 3 - 1, k1 = k + q / 9 - 1;
+        const bool in = i1 > 0 && i1 < b.nx && j1 > 0 && j1 < b.ny && k1 > 0 && k1 < b.nz;
+        if (in && v[q] >= SAmin && v[q] <= p.LSAmax) { s0 = s0 + v[q]; kn++; }
+    }
+    b.U[5][s] = kn == 0 ? p.LSAmax : s0 / (double)kn;
 }
 
 __device__ __forceinline__ void limit_sa_isolated_cell(const Blk& b, const Par& p, int i, int j, int k) {
@@ -1141,47 +1146,100 @@ __global__ void __launch_bounds__(64) k_limit(BSet S, int nb, int ntiles) {
                   [](const Blk& b, const Par& p, int i, int j, int k) { limit_sa_isolated_cell(b, p, i, j, k); });
 }
 
-// the flagged cells of block b left by the isolated pass, by increasing w over the box that bounds
-// them, by one workgroup of SA_ORD_T threads; clears the mask
-constexpr int SA_ORD_T = 256;
+// The flagged cells of block b left by the isolated pass, by increasing w, by one workgroup of
+// SA_ORD_T threads; clears the mask.  With up to SA_WMAX values of w in the block they are sorted by w
+// first (a counting sort into aux, which SA does not use), so a step touches its cells only; beyond
+// that every step looks through the box that bounds the cells.  Bound by the steps' latency, one trip
+// to memory and a barrier each.  A 257x97x33 C-grid after 4000 iterations, update stage: 3340 us with
+// every step looked up and the neighbours judged one by one, 1190 sorted (256 threads 1325, 1024: 1150).
+constexpr int SA_ORD_T = 512, SA_WMAX = 4096;
 __device__ __forceinline__ void limit_sa_ordered(const Blk& b, const Par& p) {
     if (b.flags[2] == 0) return;
-    const int nxm = b.nx - 1, nym = b.ny - 1;
-    const long ncell = (long)nxm * nym * (b.nz - 1);
+    const int nxm = b.nx - 1, nym = b.ny - 1, nzm = b.nz - 1, tid = (int)threadIdx.x;
+    const long ncell = (long)nxm * nym * nzm;
     const long nword = (ncell + 63) / 64;
-    __shared__ int lo[3], hi[3];
-    if (threadIdx.x < 3) { lo[threadIdx.x] = 1 << 30; hi[threadIdx.x] = -1; }
-    __syncthreads();
-    int l0 = 1 << 30, l1 = 1 << 30, l2 = 1 << 30, h0 = -1, h1 = -1, h2 = -1;
-    for (long wi = threadIdx.x; wi < nword; wi += SA_ORD_T) {
-        unsigned long long m = b.samask[wi];
-        while (m) {
-            const int bit = __builtin_ctzll(m);
-            m &= m - 1;
-            const long cc = wi * 64 + bit;
-            const int i = (int)(cc % nxm) + 1, j = (int)((cc / nxm) % nym) + 1, k = (int)(cc / ((long)nxm * nym)) + 1;
-            l0 = min(l0, i); l1 = min(l1, j); l2 = min(l2, k);
-            h0 = max(h0, i); h1 = max(h1, j); h2 = max(h2, k);
+    const int nw = nxm + 2 * nym + 4 * nzm - 6;          // values of w, from 7 = 1 + 2 + 4 on
+    __shared__ int lo[3], hi[3], total;
+    __shared__ int ofs[SA_WMAX], part[SA_ORD_T];
+    typedef unsigned long long u64;
+    u64* list = reinterpret_cast<u64*>((double*)b.aux);          // i, j, k in 21 bits each
+    // f(i, j, k) of every cell still in the mask
+    auto each = [&](auto&& f) {
+        for (long wi = tid; wi < nword; wi += SA_ORD_T) {
+            unsigned long long m = b.samask[wi];
+            while (m) {
+                const int bit = __builtin_ctzll(m);
+                m &= m - 1;
+                const unsigned cc = (unsigned)(wi * 64 + bit), row = cc / (unsigned)nxm, k = row / (unsigned)nym;
+                f((int)(cc - row * nxm) + 1, (int)(row - k * nym) + 1, (int)k + 1);
+            }
         }
-    }
+    };
+    if (tid < 3) { lo[tid] = 1 << 30; hi[tid] = -1; }
+    if (tid == 0) total = 0;
+    for (int w = tid; w < min(nw, SA_WMAX); w += SA_ORD_T) ofs[w] = 0;
+    __syncthreads();
+    int l0 = 1 << 30, l1 = 1 << 30, l2 = 1 << 30, h0 = -1, h1 = -1, h2 = -1, n = 0;
+    each([&](int i, int j, int k) {
+        l0 = min(l0, i); l1 = min(l1, j); l2 = min(l2, k);
+        h0 = max(h0, i); h1 = max(h1, j); h2 = max(h2, k);
+        n++;
+        if (nw <= SA_WMAX) atomicAdd(&ofs[i + 2 * j + 4 * k - 7], 1);
+    });
     if (h0 >= 0) {
         atomicMin(&lo[0], l0); atomicMin(&lo[1], l1); atomicMin(&lo[2], l2);
         atomicMax(&hi[0], h0); atomicMax(&hi[1], h1); atomicMax(&hi[2], h2);
+        atomicAdd(&total, n);
     }
     __syncthreads();
     if (hi[0] < 0) return;                      // every flagged cell was isolated
-    const int nj = hi[1] - lo[1] + 1, njk = nj * (hi[2] - lo[2] + 1);
-    const int w0 = lo[0] + 2 * lo[1] + 4 * lo[2], w1 = hi[0] + 2 * hi[1] + 4 * hi[2];
-    for (int w = w0; w <= w1; w++) {
-        for (int a = (int)threadIdx.x; a < njk; a += SA_ORD_T) {
-            const int j = lo[1] + a % nj, k = lo[2] + a / nj, i = w - 2 * j - 4 * k;
-            if (i >= lo[0] && i <= hi[0] && sa_flagged(b, sa_cell_index(b, i, j, k))) sa_replace(b, p, i, j, k);
+    if (nw <= SA_WMAX) {
+        // ofs[w]: the first place of w's cells; after the placing, the first of the next w's
+        constexpr int R = SA_WMAX / SA_ORD_T;
+        int sum = 0;
+        for (int w = tid * R; w < min(nw, tid * R + R); w++) sum += ofs[w];
+        part[tid] = sum;
+        __syncthreads();
+        if (tid == 0) {
+            int a = 0;
+            for (int q = 0; q < SA_ORD_T; q++) { const int c = part[q]; part[q] = a; a += c; }
         }
-        // the replaced values of this w before the next reads them
+        __syncthreads();
+        int a = part[tid];
+        for (int w = tid * R; w < min(nw, tid * R + R); w++) { const int c = ofs[w]; ofs[w] = a; a += c; }
+        __syncthreads();
+        each([&](int i, int j, int k) { list[atomicAdd(&ofs[i + 2 * j + 4 * k - 7], 1)] = (u64)i | (u64)j << 21 | (u64)k << 42; });
         __threadfence_block();
         __syncthreads();
+        int first = 0;
+        u64 next = tid < total ? list[tid] : 0;
+        for (int w = 0; w < nw; w++) {
+            const int end = ofs[w];
+            if (end == first) continue;
+            const u64 mine = next;
+            next = end + tid < total ? list[end + tid] : 0;      // of the next step, ahead of its barrier
+            for (int q = first + tid; q < end; q += SA_ORD_T) {
+                const u64 c = q == first + tid ? mine : list[q];
+                sa_replace(b, p, (int)(c & 0x1fffff), (int)(c >> 21 & 0x1fffff), (int)(c >> 42));
+            }
+            first = end;
+            // the replaced values of this w before the next reads them
+            __threadfence_block();
+            __syncthreads();
+        }
+    } else {
+        const int nj = hi[1] - lo[1] + 1, njk = nj * (hi[2] - lo[2] + 1);
+        const int w0 = lo[0] + 2 * lo[1] + 4 * lo[2], w1 = hi[0] + 2 * hi[1] + 4 * hi[2];
+        for (int w = w0; w <= w1; w++) {
+            for (int a = tid; a < njk; a += SA_ORD_T) {
+                const int j = lo[1] + a % nj, k = lo[2] + a / nj, i = w - 2 * j - 4 * k;
+                if (i >= lo[0] && i <= hi[0] && sa_flagged(b, sa_cell_index(b, i, j, k))) sa_replace(b, p, i, j, k);
+            }
+            __threadfence_block();
+            __syncthreads();
+        }
     }
-    for (long wi = threadIdx.x; wi < nword; wi += SA_ORD_T)
+    for (long wi = tid; wi < nword; wi += SA_ORD_T)
         if (b.samask[wi]) b.samask[wi] = 0ull;
 }
 
@@ -1670,7 +1728,7 @@ static void limit_after_update(const SetPlan& P, hipStream_t st) {
     const int n = P.ntiles[SP_CELL];
     if (n <= 0) return;
     hipLaunchKernelGGL(k_limit, dim3((unsigned)std::min(n, 4096)), dim3(64), 0, st, bset(P, SP_CELL), P.nb, n);
-    hipLaunchKernelGGL(k_limit_finish, dim3((unsigned)(P.nb + std::min((n + 3) / 4, 1024))), dim3(SA_ORD_T), 0, st, bset(P, SP_CELL), P.nb, n);
+    hipLaunchKernelGGL(k_limit_finish, dim3((unsigned)(P.nb + std::min((n + SA_ORD_T / 64 - 1) / (SA_ORD_T / 64), 512))), dim3(SA_ORD_T), 0, st, bset(P, SP_CELL), P.nb, n);
 }
 
 void set_update_limit(const SetPlan& P, hipStream_t st) {
