@@ -814,7 +814,11 @@ __global__ void __launch_bounds__(PK_T, 6) k_cell_pk(BSet S, ctab<LuTask> tiles,
         double dt;
         cell_assemble<T>(
             b, p, i, j, k, s, [&](int m, double r) { b.Res[m][s] = r; buf[m][c][x] = r; }, [](int, double, double) {}, Lc, Lv, dt);
-        if constexpr (NV == 7) { buf[5][c][x] = b.Res[5].ro(s); buf[6][c][x] = b.Res[6].ro(s); }
+        // Res beyond 5: what cell_assemble has just formed (SA's first), else what the array holds (SST's,
+        // or zero where NVAR exceeds what the model needs)
+#pragma unroll
+        for (int m = 5; m < NV; m++)
+            if (m > 5 || p.turb != 2) buf[m][c][x] = b.Res[m].ro(s);
         b.dt[s] = dt;
         const double vol = b.vol.ro(s);
         const double sumLc = (Lc[0] + Lc[1]) + Lc[2], sumLv = (Lv[0] + Lv[1]) + Lv[2];
