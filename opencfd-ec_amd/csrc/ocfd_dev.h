@@ -367,6 +367,23 @@ template <int NV> struct Pk {
     }
 };
 constexpr int LU_PAD_STEPS = 24;
+
+// The LDS ring of a tile's team holds the inputs of LU_RING steps; its waves run their steps in rounds
+// of as many.
+constexpr int LU_RING = 4;
+
+// Whether a wave of a team gave up waiting.  The waves ask after the barrier that ends a round, and
+// have to get the same answer to leave together, so each round has a word of its own: a wave that is
+// ahead may raise the next round's word while another has still to ask about this one, but the round
+// after that, which shares the word, begins behind a barrier that comes after the question.
+struct GaveUp {
+    int word[2];
+    __host__ __device__ __forceinline__ void start(int v) { word[0] = word[1] = v; }
+    __host__ __device__ __forceinline__ void raise(int q) { word[q / LU_RING & 1] = 1; }      // at step q
+    // after the barrier that ends step q, the last of its round, and a fence (no volatile read: it would
+    // be a flat one, which waits for the wave's global loads as well)
+    __host__ __device__ __forceinline__ bool raised(int q) const { return word[q / LU_RING & 1] != 0; }
+};
 constexpr int PK_W = 32;      // i-window of one workgroup of the sweep-order transposes and cell pass
 
 // Before a sweep every DU element it writes holds this NaN (a payload no arithmetic produces); a

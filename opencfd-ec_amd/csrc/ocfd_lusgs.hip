@@ -387,7 +387,7 @@ __device__ __forceinline__ void team_barrier() {
 // step q's piece of the tile's run (R to N forward, NBR to DUF backward) and, for the lanes at the
 // tile's upstream edges, the NBR (and backward SG) chunks that step q + 1 reads of the upstream
 // tiles.  du: the three direction waves' neighbour terms, double-buffered by step parity.
-constexpr int LU_RING = 4, LU_FAR = LU_RING - 1;      // slots, and how many steps ahead the loader writes
+constexpr int LU_FAR = LU_RING - 1;      // how many steps ahead the loader writes
 template <int NV, bool FWD, int TJ> struct TeamLds {
     using F = Pk<NV>;
     static constexpr int BASE = FWD ? F::R : F::NBR;                 // first double of a run's piece
@@ -399,7 +399,7 @@ template <int NV, bool FWD, int TJ> struct TeamLds {
     static_assert(PIECE % 16 == 0 && EDGE * 2 <= LU_NT && LOADS * (LU_FAR - 2) < 64, "loads of a step");
     alignas(16) char ring[LU_RING * SLOT];
     double du[2][3][2][LU_NT];        // [step parity][direction][component a, b][lane]
-    int bail;
+    GaveUp bail;
 };
 
 // inputs of one step of wave D for this lane's components (a: momentum or energy, b: density or a
@@ -490,6 +490,7 @@ __device__ void team_load(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask& 
     wait_loads<L::LOADS * (LU_FAR - 2)>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_barrier();      // the direction waves have read slot -1, which step 0 overwrites
+    asm volatile("" ::: "memory");     // and no load of step 0 moves ahead of that
 #pragma unroll 1
     for (int q = 0; q < nsteps; q++) {
         issue(q + LU_FAR, slot);
@@ -497,7 +498,7 @@ __device__ void team_load(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask& 
         wait_loads<L::LOADS * (LU_FAR - 2)>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (q % LU_RING == LU_RING - 1 && *(volatile int*)&sh.bail != 0) break;
+        if (q % LU_RING == LU_RING - 1 && sh.bail.raised(q)) break;
     }
     wait_loads<0>();      // no load may reach the LDS after the workgroup has given it back
 }
@@ -620,7 +621,7 @@ __device__ void team_sweep(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask&
         if constexpr (D > 0) {
             if ((__builtin_amdgcn_ballot_w64(maybe_sentinel(Da) || maybe_sentinel(Db)) & rmask) != 0) {
                 const bool waiting = remote && i >= 1 && i <= nxm;
-                if (team_wait_remote((const double*)(ea + (long)q * dstep), (const double*)(eb + (long)q * dstep), waiting, Da, Db, err)) sh.bail = 1;
+                if (team_wait_remote((const double*)(ea + (long)q * dstep), (const double*)(eb + (long)q * dstep), waiting, Da, Db, err)) sh.bail.raise(q);
             }
             DUa = pick(rmask, Da, DUa);
             DUb = pick(rmask, Db, DUb);
@@ -642,9 +643,9 @@ __device__ void team_sweep(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask&
     // The loop is unrolled over the ring's slots.  The inputs of step q + 1 are read during step q,
     // an upstream tile's DU is loaded LU_AHEAD steps before its use: every step more adds a step to
     // the lag of each tile hop (257x97x33 C-grid, forward: 232, 263 and 292 us for 1, 2 and 3).  The last step of a round
-    // checks whether a wave gave up (an LDS read after the barrier that the others skip): that wave
-    // has set the error flag, so the waits of the steps in between give up within 256 polls and
-    // their values are discarded, and all waves leave at the same barrier.
+    // checks whether a wave gave up in it (an LDS read after the barrier that the others skip): that
+    // wave has set the error flag, so the waits of the steps in between give up within 256 polls and
+    // their values are discarded, and all waves leave at the same barrier (GaveUp).
     constexpr int LU_AHEAD = 1;
     static_assert(LU_RING % 2 == 0, "the step parity is fixed per unrolled step");
     TeamIn in[2];
@@ -666,7 +667,7 @@ __device__ void team_sweep(TeamLds<NV, FWD, TJ>& sh, const Blk& b, const LuTask&
             read((u + 1) % W, u, in[(u + 1) & 1]);
             step(q, u & 1, in[u & 1], Da[u], Db[u]);
             team_barrier();
-            if (u == W - 1 && sh.bail != 0) return;
+            if (u == W - 1 && sh.bail.raised(q)) return;
         }
     }
     // the DU of the last step
@@ -686,11 +687,11 @@ __global__ void __launch_bounds__(LT_NT) k_lusgs_team(const Blk* __restrict__ bl
     const int wave = threadIdx.x / LU_NT, lane = threadIdx.x % LU_NT;
     // a sweep earlier in the launch sequence gave up waiting: this one does nothing either (its
     // DU stays unused, the update kernels leave U as it is)
-    if (threadIdx.x == 0) sh.bail = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) sh.bail.start(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     // the terms of the steps before a lane's first cell, and of a direction without a neighbour
     for (int e = (int)threadIdx.x; e < 2 * 3 * 2 * LU_NT; e += LT_NT) (&sh.du[0][0][0][0])[e] = 0.0;
     __syncthreads();
-    if (sh.bail != 0) return;
+    if (sh.bail.raised(0)) return;
     const LuTask T = tasks[blockIdx.x];
     const Blk& b = blks[T.blk];
     if (wave == 0) team_sweep<NV, FWD, 0, TJ>(sh, b, T, pk, err, p, lane);
