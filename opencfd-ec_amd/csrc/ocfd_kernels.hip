@@ -1151,11 +1151,15 @@ __global__ void __launch_bounds__(64) k_limit(BSet S, int nb, int ntiles) {
 }
 
 // The flagged cells of block b left by the isolated pass, by increasing w, by one workgroup of
-// SA_ORD_T threads; clears the mask.  With up to SA_WMAX values of w in the block they are sorted by w
-// first (a counting sort into aux, which SA does not use), so a step touches its cells only; beyond
-// that every step looks through the box that bounds the cells.  Bound by the steps' latency, one trip
-// to memory and a barrier each.  A 257x97x33 C-grid after 4000 iterations, update stage: 3340 us with
-// every step looked up and the neighbours judged one by one, 1190 sorted (256 threads 1325, 1024: 1150).
+// SA_ORD_T threads; clears the mask.  With up to SA_WMAX values of w in the block the cells are listed
+// in one pass over the mask (into prim[6], free until the next iteration) and sorted by w (a counting
+// sort into aux, which SA does not use), so a step touches its cells only; beyond that every step looks
+// through the box that bounds the cells.  Bound by the steps' latency, one trip to memory and a barrier
+// each, and for few cells by the pass over the mask.  On a 257x97x33 C-grid one pair of flagged cells
+// costs 18 us (unsorted 34; with a second pass over the mask and a walk over all w of the block 66), the
+// update stage of an iteration after 4000 1125 us (unsorted, the neighbours judged one by one, 3340;
+// 512 threads against 256 and 1024: 1187, 1325 and 1150 when measured).  One block with 6.3 M cells: a
+// pair costs 65 us (unsorted 150, with the second pass 245).
 constexpr int SA_ORD_T = 512, SA_WMAX = 4096;
 __device__ __forceinline__ void limit_sa_ordered(const Blk& b, const Par& p) {
     if (b.flags[2] == 0) return;
@@ -1163,61 +1167,70 @@ __device__ __forceinline__ void limit_sa_ordered(const Blk& b, const Par& p) {
     const long ncell = (long)nxm * nym * nzm;
     const long nword = (ncell + 63) / 64;
     const int nw = nxm + 2 * nym + 4 * nzm - 6;          // values of w, from 7 = 1 + 2 + 4 on
-    __shared__ int lo[3], hi[3], total;
-    __shared__ int ofs[SA_WMAX], part[SA_ORD_T];
+    const bool sorted = nw <= SA_WMAX;
+    __shared__ int lo[4], hi[4], total;                  // of i, j, k and w - 7
+    __shared__ int ofs[SA_WMAX], part[SA_ORD_T / 64];
     typedef unsigned long long u64;
-    u64* list = reinterpret_cast<u64*>((double*)b.aux);          // i, j, k in 21 bits each
-    // f(i, j, k) of every cell still in the mask
-    auto each = [&](auto&& f) {
-        for (long wi = tid; wi < nword; wi += SA_ORD_T) {
-            unsigned long long m = b.samask[wi];
-            while (m) {
-                const int bit = __builtin_ctzll(m);
-                m &= m - 1;
-                const unsigned cc = (unsigned)(wi * 64 + bit), row = cc / (unsigned)nxm, k = row / (unsigned)nym;
-                f((int)(cc - row * nxm) + 1, (int)(row - k * nym) + 1, (int)k + 1);
+    u64 *found = reinterpret_cast<u64*>((double*)b.prim[6]), *list = reinterpret_cast<u64*>((double*)b.aux);      // i, j, k in 21 bits each
+    auto w_of = [](u64 c) { return (int)(c & 0x1fffff) + 2 * (int)(c >> 21 & 0x1fffff) + 4 * (int)(c >> 42) - 7; };
+    if (tid < 4) { lo[tid] = 1 << 30; hi[tid] = -1; }
+    if (tid == 0) total = 0;
+    if (sorted)
+        for (int w = tid; w < nw; w += SA_ORD_T) ofs[w] = 0;
+    __syncthreads();
+    int l[4] = {1 << 30, 1 << 30, 1 << 30, 1 << 30}, h[4] = {-1, -1, -1, -1};
+    auto take = [&](long wi, u64 m) {
+        int at = atomicAdd(&total, __popcll(m));
+        if (sorted) b.samask[wi] = 0ull;
+        while (m) {
+            const int bit = __builtin_ctzll(m);
+            m &= m - 1;
+            const unsigned cc = (unsigned)(wi * 64 + bit), row = cc / (unsigned)nxm, kk = row / (unsigned)nym;
+            const int x[4] = {(int)(cc - row * nxm) + 1, (int)(row - kk * nym) + 1, (int)kk + 1, 0};
+            const int w = x[0] + 2 * x[1] + 4 * x[2] - 7;
+#pragma unroll
+            for (int q = 0; q < 4; q++) { l[q] = min(l[q], q < 3 ? x[q] : w); h[q] = max(h[q], q < 3 ? x[q] : w); }
+            if (sorted) {
+                atomicAdd(&ofs[w], 1);
+                found[at++] = (u64)x[0] | (u64)x[1] << 21 | (u64)x[2] << 42;
             }
         }
     };
-    if (tid < 3) { lo[tid] = 1 << 30; hi[tid] = -1; }
-    if (tid == 0) total = 0;
-    for (int w = tid; w < min(nw, SA_WMAX); w += SA_ORD_T) ofs[w] = 0;
-    __syncthreads();
-    int l0 = 1 << 30, l1 = 1 << 30, l2 = 1 << 30, h0 = -1, h1 = -1, h2 = -1, n = 0;
-    each([&](int i, int j, int k) {
-        l0 = min(l0, i); l1 = min(l1, j); l2 = min(l2, k);
-        h0 = max(h0, i); h1 = max(h1, j); h2 = max(h2, k);
-        n++;
-        if (nw <= SA_WMAX) atomicAdd(&ofs[i + 2 * j + 4 * k - 7], 1);
-    });
-    if (h0 >= 0) {
-        atomicMin(&lo[0], l0); atomicMin(&lo[1], l1); atomicMin(&lo[2], l2);
-        atomicMax(&hi[0], h0); atomicMax(&hi[1], h1); atomicMax(&hi[2], h2);
-        atomicAdd(&total, n);
+    // four words in flight: a block of 6.3 M cells has 192 per thread
+    for (long wi = tid; wi < nword; wi += 4 * SA_ORD_T) {
+        u64 m[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) m[u] = wi + u * SA_ORD_T < nword ? b.samask[wi + u * SA_ORD_T] : 0ull;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (m[u]) take(wi + u * SA_ORD_T, m[u]);
     }
+    if (h[0] >= 0) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) { atomicMin(&lo[q], l[q]); atomicMax(&hi[q], h[q]); }
+    }
+    __threadfence_block();
     __syncthreads();
     if (hi[0] < 0) return;                      // every flagged cell was isolated
-    if (nw <= SA_WMAX) {
-        // ofs[w]: the first place of w's cells; after the placing, the first of the next w's
-        constexpr int R = SA_WMAX / SA_ORD_T;
+    if (sorted) {
+        // ofs[w]: the first place of w's cells, from the counts; after the placing, the first of the next w's
+        const int w0 = lo[3], w1 = hi[3], R = (w1 - w0) / SA_ORD_T + 1, wt = w0 + tid * R;
         int sum = 0;
-        for (int w = tid * R; w < min(nw, tid * R + R); w++) sum += ofs[w];
-        part[tid] = sum;
+        for (int w = wt; w < min(wt + R, w1 + 1); w++) sum += ofs[w];
+        int upto = sum;                         // with the wave's threads before this one
+        for (int d = 1; d < 64; d *= 2) { const int v = __shfl_up(upto, d, 64); if (tid % 64 >= d) upto += v; }
+        if (tid % 64 == 63) part[tid / 64] = upto;
         __syncthreads();
-        if (tid == 0) {
-            int a = 0;
-            for (int q = 0; q < SA_ORD_T; q++) { const int c = part[q]; part[q] = a; a += c; }
-        }
+        int a = upto - sum;
+        for (int q = 0; q < tid / 64; q++) a += part[q];
+        for (int w = wt; w < min(wt + R, w1 + 1); w++) { const int c = ofs[w]; ofs[w] = a; a += c; }
         __syncthreads();
-        int a = part[tid];
-        for (int w = tid * R; w < min(nw, tid * R + R); w++) { const int c = ofs[w]; ofs[w] = a; a += c; }
-        __syncthreads();
-        each([&](int i, int j, int k) { list[atomicAdd(&ofs[i + 2 * j + 4 * k - 7], 1)] = (u64)i | (u64)j << 21 | (u64)k << 42; });
+        for (int q = tid; q < total; q += SA_ORD_T) { const u64 c = found[q]; list[atomicAdd(&ofs[w_of(c)], 1)] = c; }
         __threadfence_block();
         __syncthreads();
         int first = 0;
         u64 next = tid < total ? list[tid] : 0;
-        for (int w = 0; w < nw; w++) {
+        for (int w = w0; w <= w1; w++) {
             const int end = ofs[w];
             if (end == first) continue;
             const u64 mine = next;
@@ -1231,17 +1244,17 @@ __device__ __forceinline__ void limit_sa_ordered(const Blk& b, const Par& p) {
             __threadfence_block();
             __syncthreads();
         }
-    } else {
-        const int nj = hi[1] - lo[1] + 1, njk = nj * (hi[2] - lo[2] + 1);
-        const int w0 = lo[0] + 2 * lo[1] + 4 * lo[2], w1 = hi[0] + 2 * hi[1] + 4 * hi[2];
-        for (int w = w0; w <= w1; w++) {
-            for (int a = tid; a < njk; a += SA_ORD_T) {
-                const int j = lo[1] + a % nj, k = lo[2] + a / nj, i = w - 2 * j - 4 * k;
-                if (i >= lo[0] && i <= hi[0] && sa_flagged(b, sa_cell_index(b, i, j, k))) sa_replace(b, p, i, j, k);
-            }
-            __threadfence_block();
-            __syncthreads();
+        return;
+    }
+    const int nj = hi[1] - lo[1] + 1, njk = nj * (hi[2] - lo[2] + 1);
+    const int w0 = lo[0] + 2 * lo[1] + 4 * lo[2], w1 = hi[0] + 2 * hi[1] + 4 * hi[2];
+    for (int w = w0; w <= w1; w++) {
+        for (int a = tid; a < njk; a += SA_ORD_T) {
+            const int j = lo[1] + a % nj, k = lo[2] + a / nj, i = w - 2 * j - 4 * k;
+            if (i >= lo[0] && i <= hi[0] && sa_flagged(b, sa_cell_index(b, i, j, k))) sa_replace(b, p, i, j, k);
         }
+        __threadfence_block();
+        __syncthreads();
     }
     for (long wi = tid; wi < nword; wi += SA_ORD_T)
         if (b.samask[wi]) b.samask[wi] = 0ull;
