@@ -7,6 +7,13 @@ namespace ocfd {
 
 constexpr int PK_T = LU_COLS * PK_W;      // a thread per cell
 
+// The steps [i0 - 1, i0 - 1 + n) of a tile whose DU elements the window of W cells from i0 on resets:
+// as many as it has cells, the last window's to the tile's end, so a tile's windows take every step
+// once.
+__device__ __host__ __forceinline__ int sentinel_steps(int nx, int tj, int tk, int i0, int W) {
+    return i0 + W == nx ? nx - 1 + tj + tk - 2 - (i0 - 1) : W;
+}
+
 // One tile and i-window of PK_W cells on its way from the block arrays to the sweep order, through
 // LDS so both sides move in contiguous runs: get() reads, a thread per cell (i fastest) with all its
 // fields in flight at once, put() writes, a wave per step with the lanes along the step's elements.
@@ -50,11 +57,10 @@ struct PackTile {
                 if (q >= d && q < d + W) dst[(size_t)q * F::RUN] = src[q];
         }
     }
-    // the sentinel into both DU arrays of the window's own steps [i0 - 1, i0 - 1 + W) (the last
-    // window's: to the tile's end)
+    // the sentinel into both DU arrays, which end a run, of the window's own steps
     __device__ __forceinline__ void sentinel() const {
-        const int steps = i0 + W - 1 == b.nx - 1 ? b.nx - 1 + T.tj + T.tk - 2 - (i0 - 1) : W;
-        constexpr int PAIRS = NV * LU_COLS;
+        const int steps = sentinel_steps(b.nx, T.tj, T.tk, i0, W);
+        constexpr int PAIRS = (F::RUN - F::DUF) / 2;
         double2 s;
         s.x = s.y = sentinel_value();
         for (int e = (int)threadIdx.x; e < steps * PAIRS; e += PK_T)

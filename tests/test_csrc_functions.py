@@ -23,7 +23,7 @@ def program(tmp_path_factory):
     return str(out)
 
 
-@pytest.mark.parametrize("check", ["give_up"])
+@pytest.mark.parametrize("check", ["give_up", "vector_groups", "face_tiles", "sweep_tables"])
 def test_check(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
