@@ -393,8 +393,10 @@ def main() -> int:
         tj, tms = s.autotune_lu(args.autotune)          # ordinary iterations, untimed
         tune = dict(kept=f"{tj}x{16 // tj}", ms_per_sweep_pair={f"{t}x{16 // t}": round(v, 4) for t, v in tms.items()})
         print(f"# LU tile autotune: {tune}", file=sys.stderr, flush=True)
+    # the warm-up goes the timed way, whose graphs (one per stage) it captures; plain steps would leave
+    # that to the timed region
     for _ in range(args.warmup):
-        s.step(1)
+        s.step_timed(1)
     s.sync()
 
     t0 = time.perf_counter()
