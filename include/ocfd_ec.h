@@ -148,7 +148,7 @@ int ocfd_block_status(ocfd_ctx *ctx, int32_t block_no, int32_t *overlimit, int32
 int ocfd_get_counters(ocfd_ctx *ctx, int32_t *kstep, double *tt);
 
 /* Stages of one iteration, in order.  ocfd_step_lusgs runs them one after the other; with graphs
- * on, each stage is captured in its own hipGraph on first use and replayed afterwards.
+ * on, it captures the whole iteration in one hipGraph on first use and replays that afterwards.
  *   PRE         comput_duvtpc, get_viscous, Turbulence_model_SA/SST, Amut_boundary
  *               (sub_Residual.f90:62-80)
  *   INVISCID    flux_inviscous_i/j/k incl. the k-face boundary flux (sub_Residual.f90:86-88)
@@ -168,11 +168,13 @@ int ocfd_get_counters(ocfd_ctx *ctx, int32_t *kstep, double *tt);
 
 /* ocfd_step_lusgs with a HIP event at every stage boundary on the context's stream:
  * stage_ms[s] = device time of stage s summed over the niter iterations.  Instrumentation; the
- * reference has no counterpart (show_Wall_time, opencfd_ec3d_v1.16a.f90:235, times whole steps). */
+ * reference has no counterpart (show_Wall_time, opencfd_ec3d_v1.16a.f90:235, times whole steps).
+ * With graphs on, each stage is a hipGraph of its own here. */
 int ocfd_step_timed(ocfd_ctx *ctx, int32_t niter, double *stage_ms);
 
-/* Capture each stage of the iteration in a hipGraph on first use and replay it (1) or launch
- * eagerly (0). */
+/* Capture the iteration in a hipGraph on first use and replay it (1; ocfd_step_timed and
+ * ocfd_autotune_lu: a graph per stage) or launch eagerly (0).  ocfd_residual and the other routines of
+ * its granularity launch eagerly either way. */
 int ocfd_set_graph(ocfd_ctx *ctx, int32_t enable);
 
 /* Schedule of the LU-SGS sweeps; all give the reference's DU bit for bit.

@@ -153,7 +153,6 @@ struct SAc {
     static constexpr double Cw2 = 0.3, Cw3 = 2.0, Ct3 = 1.2, Ct4 = 0.5;
 };
 
-// nu-tilde face flux of the SA equation on face (fi,fj,fk) of direction DIR (I-1/2 convention):
 // a face's normal, area and metrics
 template <typename T> struct FaceGeo { T n[3], S, m[9]; };
 template <int DIR, typename T>
@@ -167,6 +166,7 @@ __device__ __forceinline__ void face_geo(const Blk& b, size_t s, FaceGeo<T>& g, 
     }
 }
 
+// nu-tilde face flux of the SA equation on face (fi,fj,fk) of direction DIR (I-1/2 convention):
 // fv = (-upwind convection + (1+cb2)/sigma (vt+mu/rho)/Re grad(vt).n) S and f2 = grad(vt).n S
 // (sub_turbulence_SA.f90:60-174)
 template <int DIR, typename T>
@@ -672,8 +672,8 @@ __device__ __forceinline__ void visc_face(const Blk& b, const Par& p, const Face
 // inviscid flux.  The terms that share the metrics come first and the face's geometry is read once:
 // a wave lives 25 us, in which an XCD's L2 is filled three times over, so a second read of a metric
 // or a normal later in the kernel came from memory again (24 blocks with 6.3 M cells: 7.0 -> 4.1 GB
-// read, 2070 -> 1880 us; a batch of 6 with 1.9 M cells 842 -> 737 us; 257x97x33: 264 -> 246).  What
-// bounds it now is FP64 arithmetic: the vector units are busy 64 % of the time.  Slower: the viscous
+// read, 2070 -> 1880 us; a batch of 6 with 2.4 M cells 842 -> 737 us; 257x97x33: 264 -> 246).  What
+// bounds it now is FP64 arithmetic: the vector units are busy 69 % of the time.  Slower: the viscous
 // part in workgroups of its own (1980 us), non-temporal flux stores and metric loads (1910).
 template <int DIR, typename T, int RECON, int FLUX, bool SST>
 __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, int k) {
@@ -703,7 +703,7 @@ __device__ __forceinline__ void face(const Blk& b, const Par& p, int i, int j, i
 // The three directions' faces in one launch.  On small grids, where a direction's tiles do not fill
 // the GPU and a launch costs more than its work, they run side by side (97x33x9 without viscosity:
 // 22 us instead of 37 in three launches; 257x97x33 SA: 271 against 306); on large ones the
-// directions share the primitives in L2 (face_tile; a batch of 6 with 1.9 M cells: 835 against
+// directions share the primitives in L2 (face_tile; a batch of 6 with 2.4 M cells: 835 against
 // 930 us, 24 blocks with 6.3 M cells: 2090 against 2200, before the metrics were read once).
 // Five waves per SIMD instead of four where that needs no spills (the primitive reconstruction: 96
 // instead of 122 VGPRs) and is faster: 24 blocks Roe 1880 -> 1832 us; Van Leer's flux, with the least
@@ -781,7 +781,8 @@ __global__ void __launch_bounds__(64) k_cell(BSet S) {
 // The cell pass of an iteration with the pipelined sweeps: one sweep tile's cells of an i-window
 // per workgroup, a thread per cell.  Res and dt go to the block arrays (for the host), and the
 // sweeps' inputs straight into sweep order, a group of fields at a time through one LDS buffer (35
-// KB for SA, so four workgroups share a CU): Res; du_LU_SGS's diagonal (sub_LU_SGS.f90:27-37
+// KB for SA: the registers, not the LDS, allow three of these eight-wave workgroups per CU, four with
+// FP32 faces): Res; du_LU_SGS's diagonal (sub_LU_SGS.f90:27-37
 // forward, :81-90 backward: of components 1..5, and 6, 7 of SST, and for SA of the SA component in
 // the forward and in the backward sweep, which sum the viscous radii in different orders) with its
 // reciprocals; the spectral radii; U with its pressure and reciprocal density.  The DU arrays get
